@@ -16,16 +16,19 @@
 //     int32 (sum order does not matter for integers);
 //   * the 16 partial sums of a feature are combined with four DPP row
 //     rotations (no LDS round trip), then lane m of the row stores output m.
-// Requires K % 16 == 0 and 16-byte aligned A/BT; other shapes use the generic
-// kernel at the end of this file.
+// Requires K % 16 == 0 and 16-byte aligned A/BT; of the kernels here the
+// any-K one also takes K % 4 == 0 and 4-byte alignment.
 //
-// Kernels by shape: gemv_i8_fixed_kernel (dot4, M <= 4, K <= 3072 and the
-// fused GPT-2 prologues), gemv_i8_mfma16_kernel (MFMA, 5 <= M <= 16,
-// K <= 4096), gemv_i8_burst_kernel (K = 768 / 3072 with N >= 16384 and
-// M <= 8: the LM head), and at K = 8192 gemv_i8_parted_kernel (4-feature
-// items, M <= 4 or N >= 16384) and gemv_i8_slice_kernel (16-feature groups
-// split over K, the rest); gemv_i8_kernel covers any other K.
+// Kernels by shape: gemv_i8_fixed_kernel (dot4, K = 768 with M <= 4, 3072
+// with M = 1, and the fused GPT-2 prologues), gemv_i8_mfma16_kernel (MFMA,
+// 5 <= M <= 16, K = 768 and the fused prologues), gemv_i8_burst_kernel (K =
+// 768 / 3072 with N >= 16384: the LM head), and at K = 8192 with wide N
+// gemv_i8_parted_kernel (4-feature items) and gemv_i8_slice_kernel
+// (16-feature groups split over K); gemv_i8_any_kernel takes every other K
+// and alignment (MFMA, 4-feature items, K sliced at run time) except short
+// rows and activation blocks past LDS, which gemv_i8_kernel keeps.
 #include <algorithm>
+#include <type_traits>
 
 #include "device_util.h"
 #include "epilogue.h"
@@ -715,6 +718,178 @@ __global__ __launch_bounds__(256) void gemv_i8_burst_kernel(int M, int N, const 
     }
 }
 
+// Any K from 16 up (K % 4 == 0, 4-byte aligned A and BT) whose activation
+// block fits LDS: the 4-feature-item MFMA layout above with K, the slicing
+// and the item walk at run time.
+//   * A workgroup of 8 waves takes 8 / KS items at a time, KS = 2^ks_log
+//     waves on each, every one over its own run of spk 256-byte steps; the
+//     launcher picks KS so that the rounds a workgroup makes times the steps
+//     of one are fewest.  The slices of an item add one int32 per lane
+//     through LDS (exact), one barrier per item, double buffered.
+//   * A wave's (item, step) sequence is one stream through a ring of R sets of
+//     U loads, refilled across item ends, so 8 loads (8 KiB) stay in flight
+//     per wave; batches past the end re-read the last item's.
+//   * LDS holds the M activation rows, zero past K, so a step that runs over
+//     the row's end needs no mask: its weight loads are clamped to the row's
+//     last 16 bytes and meet zeros.  Where K % 16 != 0 the chunk that
+//     straddles K is loaded from K - 16 on both sides, the words already
+//     counted zeroed on the activation side.
+// Bound by what a CU takes in (weights / CUs + M K activation bytes) behind
+// ~2.5 us of launch, staging and reduction: 4096 x 4096 at M = 16 (128 KB per
+// CU) 21.7 us on the dot4 kernel below, 6.4 here; 1000 x 4001 at M = 1 (K %
+// 16 != 0) 60 us with one thread per output, 3.2 here (weights rotated
+// through 600 MB).  A ring of 8 sets measured level with 4; two sets where
+// a wave has no more batches than that.
+template <int EPI, bool NT, int MB, int R>
+__global__ __launch_bounds__(512) void gemv_i8_any_kernel(int M, int N, int K, int ks_log, int spk, uint32_t inv_cpr,
+                                                          const int8_t* __restrict__ A,
+                                                          const int8_t* __restrict__ BT,
+                                                          const float* __restrict__ sA,
+                                                          const float* __restrict__ sB, const float* bias,
+                                                          const float* residual, void* C) {
+    constexpr int U = 2, SB = 2 * MB;
+    typedef i32x4 i32x4_a4 __attribute__((aligned(4)));
+    extern __shared__ __attribute__((aligned(16))) int8_t any_lds[];
+    int32_t* red = reinterpret_cast<int32_t*>(any_lds);  // [2][8][64]
+    int8_t* a_lds = any_lds + 2 * 8 * 64 * 4;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15, q = lane >> 4;
+    const int part = col & 3, f = col >> 2;
+    const int ks = 1 << ks_log, slots = 8 >> ks_log;
+    const int slice = wave & (ks - 1), gslot = wave >> ks_log;
+    const int cpr = (spk << ks_log) * 16;  // 16-byte chunks per LDS row
+    const int lda = cpr * 16 + 64;         // padded: conflict-free fragment reads
+    const int nitems_all = (N + 3) / 4;
+    const int stride = slots * (int)gridDim.x;
+    const int rounds = (nitems_all - 1 - (int)blockIdx.x) / stride + 1;  // grid <= items
+    const int total = rounds * (spk / U);
+    auto item = [&](int t) { return t * stride + gslot * (int)gridDim.x + (int)blockIdx.x; };
+
+    // Activation chunks first (the LDS writes below wait only for them),
+    // unconditional clamped loads: n chunks over 512 threads, SB at a time.
+    // (inv_cpr = ceil(2^32 / cpr): i / cpr for the i here, all below 2^16)
+    const int nch = M * cpr;
+    auto chunk_load = [&](int i) {
+        const int ic = min(i, nch - 1), m = (int)__umulhi(ic, inv_cpr), c = ic - m * cpr;
+        return *reinterpret_cast<const i32x4_a4*>(A + (size_t)m * K + min(16 * c, K - 16));
+    };
+    auto chunk_store = [&](int i, i32x4 v) {
+        if (i >= nch) return;
+        const int m = (int)__umulhi(i, inv_cpr), c = i - m * cpr, over = 16 * c + 16 - K;  // bytes past K
+#pragma unroll
+        for (int w = 0; w < 4; ++w) v[w] = 4 * w < over ? 0 : v[w];
+        *reinterpret_cast<i32x4*>(a_lds + m * lda + 16 * c) = v;
+    };
+    i32x4 stage[SB];
+#pragma unroll
+    for (int j = 0; j < SB; ++j) stage[j] = chunk_load(threadIdx.x + 512 * j);
+
+    const int kofs = (4 * q + part) * 16;
+    const int kb0 = slice * spk * 256 + kofs;
+    const int8_t* bt = opaque_global(BT);
+    auto row_ptr = [&](int t) { return bt + (size_t)min(4 * item(min(t, rounds - 1)) + f, N - 1) * K; };
+    int rt = 0, rs = 0;  // the ring's next batch: round, step
+    const int8_t* rp = row_ptr(0);
+    i32x4 w[R][U];
+    auto refill = [&](i32x4 (&d)[U]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const i32x4_a4* p = reinterpret_cast<const i32x4_a4*>(rp + min(kb0 + (rs + u) * 256, K - 16));
+            if constexpr (NT)
+                d[u] = __builtin_nontemporal_load(p);
+            else
+                d[u] = *p;
+        }
+        rs += U;
+        if (rs == spk) {
+            rs = 0;
+            rp = row_ptr(++rt);
+        }
+    };
+    const int out_m = 4 * part + q;  // as gemv_i8_parted_kernel
+    const bool out_ok = part < MB && out_m < M;
+    const int m_c = min(out_m, M - 1);
+    auto epi_of = [&](int t) { return epi_load<EPI>(m_c, min(4 * item(min(t, rounds - 1)) + f, N - 1), N, sB, bias, residual); };
+    const float sa = EPI != IE_EPI_I32 ? sA[m_c] : 0.0f;
+    EpiIn e = epi_of(0);
+#pragma unroll
+    for (int r = 0; r < R; ++r) refill(w[r]);
+#pragma unroll
+    for (int j = 0; j < SB; ++j) chunk_store(threadIdx.x + 512 * j, stage[j]);
+    for (int b = 512 * SB; b < nch; b += 512 * SB) {
+#pragma unroll
+        for (int j = 0; j < SB; ++j) stage[j] = chunk_load(b + threadIdx.x + 512 * j);
+#pragma unroll
+        for (int j = 0; j < SB; ++j) chunk_store(b + threadIdx.x + 512 * j, stage[j]);
+    }
+    auto wg_barrier = [] {
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    wg_barrier();
+
+    const int8_t* arow[MB];
+#pragma unroll
+    for (int j = 0; j < MB; ++j) arow[j] = a_lds + min(4 * j + f, M - 1) * lda + kb0;
+    i32x4 acc[MB][2];
+    auto clear = [&] {
+#pragma unroll
+        for (int j = 0; j < MB; ++j) acc[j][0] = acc[j][1] = i32x4{0, 0, 0, 0};
+    };
+    clear();
+    int ct = 0, cs = 0, par = 0;  // being consumed: round, step; reduction buffer
+    auto finish = [&] {
+        int32_t mine = 0;
+#pragma unroll
+        for (int j = 0; j < MB; ++j) {
+            const i32x4 x4 = acc[j][0] + acc[j][1];
+            int32_t x = part == 0 ? x4[0] : part == 1 ? x4[1] : part == 2 ? x4[2] : x4[3];
+            x += __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xf, 0xf, false);  // quad_perm [1, 0, 3, 2]
+            x += __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xf, 0xf, false);  // quad_perm [2, 3, 0, 1]
+            mine = part == j ? x : mine;
+        }
+        const int n = 4 * item(ct) + f;
+        if (ks > 1) {
+            red[(par * 8 + wave) * 64 + lane] = mine;
+            wg_barrier();
+            if (slice == 0)
+                for (int s = 1; s < ks; ++s) mine += red[(par * 8 + wave + s) * 64 + lane];
+            par ^= 1;
+        }
+        if (slice == 0 && out_ok && n < N) gemv_store<EPI>(C, out_m, n, N, mine, sa, e, 0, GemvFusion{});
+        clear();
+        ++ct;
+        e = epi_of(ct);
+    };
+    auto body = [&](int b, auto more) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            if (decltype(more)::value || b + r < total) {
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int j = 0; j < MB; ++j)
+                        acc[j][u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                            *reinterpret_cast<const i32x4*>(arow[j] + (cs + u) * 256), w[r][u], acc[j][u], 0, 0, 0);
+                if constexpr (decltype(more)::value) refill(w[r]);
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+                cs += U;
+                if (cs == spk) {
+                    cs = 0;
+                    finish();
+                }
+            }
+        }
+    };
+    int b = 0;
+#pragma unroll 1
+    for (; b + R < total; b += R) body(b, std::true_type{});
+    body(b, std::false_type{});
+}
+
 // Any K % 4 == 0 and any alignment: one thread per output element.
 template <int EPI>
 __global__ __launch_bounds__(256) void gemm_i8_generic_kernel(
@@ -746,6 +921,7 @@ constexpr size_t kStreamWeightBytes = 64ull << 20;
 // weights up to this size: each row block re-reads the weights, which for
 // these stay in the caches.
 constexpr size_t kRowSplitWeightBytes = 8ull << 20;
+constexpr size_t kLdsBytes = 160ull << 10;  // per workgroup on gfx950
 
 template <int MT, int EPI, int K16, int SRC = kSrcInt8, int GF = 0, int NW = 4>
 void launch_fixed(const GemmArgs& a, hipStream_t s, const GemvFusion& f = GemvFusion{}) {
@@ -859,6 +1035,55 @@ void launch_burst(const GemmArgs& a, hipStream_t s) {
     else go(std::integral_constant<int, 4>{});
 }
 
+// Slicing of the any-K kernel: the KS (1, 2, 4 or 8 waves per item) whose
+// rounds x (steps per slice + 1) is least, the 1 for an item's reduction and
+// store; one workgroup per CU.
+struct AnyPlan {
+    int ks_log, spk;
+    long long batches;  // of a wave's stream
+    unsigned blocks;
+    size_t lds;
+};
+constexpr int kAnyRing = 4;
+AnyPlan any_plan(const GemmArgs& a) {
+    const long long items = (a.N + 3) / 4, cus = num_cus();
+    const int steps = (a.K + 255) / 256;
+    AnyPlan best{};
+    long long cost = -1;
+    for (int l = 0; l <= 3; ++l) {
+        const int slots = 8 >> l, spk = ((steps + (1 << l) - 1) / (1 << l) + 1) / 2 * 2;
+        const long long blocks = std::min((items + slots - 1) / slots, cus);
+        const long long rounds = (items + blocks * slots - 1) / (blocks * slots), c = rounds * (spk + 1);
+        if (cost < 0 || c < cost) {
+            cost = c;
+            best = {l, spk, rounds * (spk / 2), (unsigned)blocks, 2 * 8 * 64 * 4 + (size_t)a.M * ((spk << l) * 256 + 64)};
+        }
+    }
+    return best;
+}
+bool any_applies(const GemmArgs& a) { return a.K >= 16 && any_plan(a).lds <= kLdsBytes; }
+
+template <int EPI>
+struct AnyLaunch {
+    static void run(const GemmArgs& a, hipStream_t s) {
+        const AnyPlan p = any_plan(a);
+        const bool nt = (size_t)a.N * a.K >= kStreamWeightBytes;
+        const unsigned cpr = (unsigned)(p.spk << p.ks_log) * 16;
+        auto go = [&](auto mb) {
+            constexpr int MB = decltype(mb)::value;
+            auto* k = nt              ? gemv_i8_any_kernel<EPI, true, MB, kAnyRing>
+                      : p.batches > 2 ? gemv_i8_any_kernel<EPI, false, MB, kAnyRing>
+                                      : gemv_i8_any_kernel<EPI, false, MB, 2>;
+            k<<<p.blocks, 512, p.lds, s>>>(a.M, a.N, a.K, p.ks_log, p.spk, (unsigned)(((1ull << 32) + cpr - 1) / cpr),
+                                           reinterpret_cast<const int8_t*>(a.A),
+                                           reinterpret_cast<const int8_t*>(a.BT), a.sA, a.sB, a.bias, a.residual, a.C);
+        };
+        if (a.M <= 4) go(std::integral_constant<int, 1>{});
+        else if (a.M <= 8) go(std::integral_constant<int, 2>{});
+        else go(std::integral_constant<int, 4>{});
+    }
+};
+
 // One decode row (M = 1): 16 rows per workgroup (one group of 4 rows per
 // wave) and, at K = 3072 or N <= 1024, one-wave workgroups, so more CUs
 // share the few hundred KB of weights and each wave's dot and epilogue chain
@@ -893,34 +1118,54 @@ void launch_mt(const GemmArgs& a, hipStream_t s) {
         if (a.K == 3072) return launch_burst<EPI, 12>(a, s);
     }
     if constexpr (MT > 4) {
-        if (a.K == 768) return launch_mfma16<EPI, 12>(a, s);
-        if (a.K == 3072) return launch_mfma16<EPI, 48>(a, s);
+        // 768: the MFMA GEMV for narrow N and for weights past its row split
+        // (N = 1024 / 12000, M = 16: 3.15 / 5.03 against 3.71 / 6.33 us); in
+        // between, where it re-reads the weights once per 4 rows, the any-K
+        // kernel (M = 16, N = 4096 / 8000: 5.10 / 7.56 -> 4.03 / 4.29 us).
+        if (a.K == 768 && (a.N < 2048 || (size_t)a.N * a.K > kRowSplitWeightBytes))
+            return launch_mfma16<EPI, 12>(a, s);
     }
-    // K = 8192 (measured at N = 8192 and 28672, M = 1..16, fraction of HBM
-    // peak on one box): the 4-feature-item kernel for M <= 8 (N = 28672:
-    // M = 1 0.76 -> 0.79 against dot4, M = 4 0.62 -> 0.79 against the 16-row
-    // MFMA kernels; N = 8192, rotated weights: M = 5 / 8 13.94 / 14.31 ->
-    // 13.15 / 13.59 us against the K-sliced kernel) and for any M once each
-    // wave has two items or more (N >= 16384; N = 28672, M = 16: 0.64 ->
-    // 0.69); below that, at 9 <= M <= 16, the K-sliced 16-feature kernel,
-    // whose activation staging costs a quarter as much per wave (N = 8192,
-    // M = 16: 14.9 against 16.9 us).
-    if (a.K == 8192) {
+    // K = 8192 (measured at N = 500 to 28672, M = 1..16): the 4-feature-item
+    // kernel for M <= 8 (N = 28672: M = 1 0.76 -> 0.79 of HBM peak against
+    // dot4, M = 4 0.62 -> 0.79 against the 16-row MFMA kernels; N = 8192,
+    // rotated weights: M = 5 / 8 13.94 / 14.31 -> 13.15 / 13.59 us against
+    // the K-sliced kernel) and for any M once each wave has two items or more
+    // (N >= 16384; N = 28672, M = 16: 0.64 -> 0.69); below that, at 9 <= M <=
+    // 16, the K-sliced 16-feature kernel, whose activation staging costs a
+    // quarter as much per wave (N = 8192, M = 16: 14.9 against 16.9 us).
+    // Both walk all of K per wave, so where N leaves waves without an item
+    // the any-K kernel, which slices K, is ahead: N = 500 / 2048 at M = 1
+    // 4.37 / 5.93 -> 3.33 / 4.97 us, M = 16 10.4 / 10.8 -> 5.9 / 7.9, N =
+    // 4096 at M = 16 11.8 -> 11.2 (M <= 8 level from 3000 on; N = 5120, M =
+    // 16: 12.05 against 13.2).
+    if (a.K == 8192 && a.N >= (a.M <= 8 ? 3000 : 4100)) {
         if (a.M <= 8 || a.N >= 16384) return launch_parted<EPI>(a, s);
         return launch_slice<EPI>(a, s);
     }
     // Specialised K: the GPT-2 widths, with the decode step's grouping (one
-    // 4-row group per wave; one-wave workgroups at N <= 1024 and at K = 3072
-    // for M <= 2): M = 1 / 2 / 4 at 768 x 2304 3.83 / 3.92 / 4.17 -> 2.82 /
-    // 2.87 / 2.97 us, 3072 x 768 3.48 / 3.80 -> 3.01 / 3.63 us (M = 4 keeps
-    // four waves, level at 4.42 us), same bits; the step built from the C ABI
-    // 466 -> 451 us at batch 1, 546 -> 497 us at batch 4.
+    // 4-row group per wave; one-wave workgroups at N <= 1024 and at K =
+    // 3072): M = 1 / 2 / 4 at 768 x 2304 3.83 / 3.92 / 4.17 -> 2.82 / 2.87 /
+    // 2.97 us, 3072 x 768 at M = 1 3.48 -> 3.01 us, same bits; the step built
+    // from the C ABI 466 -> 451 us at batch 1, 546 -> 497 us at batch 4.  At
+    // K = 3072 the any-K kernel is ahead from two rows or 2048 features on
+    // (N = 768, M = 2 / 4 / 8 / 16: 3.34 / 4.06 / 4.94 / 5.00 -> 3.16 / 3.25 /
+    // 3.66 / 4.57 us; N = 12288, M = 4: 13.7 -> 8.8).
     if constexpr (MT <= 4) {
         if (a.K == 768 && a.N <= 1024) return launch_fixed<MT, EPI, 48, kSrcInt8, 1, 1>(a, s);
         if (a.K == 768) return launch_fixed<MT, EPI, 48, kSrcInt8, 1, 4>(a, s);
-        if (a.K == 3072 && MT <= 2) return launch_fixed<MT, EPI, 192, kSrcInt8, 1, 1>(a, s);
-        if (a.K == 3072) return launch_fixed<MT, EPI, 192, kSrcInt8, 1, 4>(a, s);
     }
+    if constexpr (MT == 1)
+        if (a.K == 3072 && a.N < 2048) return launch_fixed<MT, EPI, 192, kSrcInt8, 1, 1>(a, s);
+    // Any other K.  The dot4 kernel below starts 0.3-0.4 us sooner (no plan,
+    // no reduction) and keeps short rows: K <= 512 (256 x 4096, M = 1 / 8:
+    // 2.17 / 2.42 against 2.59 / 3.04 us) and, for a few workgroups or very
+    // many, K <= 640 (M <= 2: K <= 1280; 1024 x 1024, M = 1: 2.40 against
+    // 2.65).  Otherwise the any-K kernel: 1024 x 3000, M = 1 / 16 3.40 / 6.42 ->
+    // 3.11 / 4.03 us, 4096 x 4096 9.45 / 21.7 -> 5.0 / 6.4, 6144 x 8192 17.3 /
+    // 35.9 -> 10.3 / 13.0.
+    const bool edge = a.N <= (a.K <= 640 ? 2048 : 1024) || a.N >= 8192;
+    const bool short_k = MT <= 8 && (a.K <= 512 || (edge && a.K <= (a.M <= 2 ? 1280 : 640)));
+    if (!short_k && any_applies(a)) return AnyLaunch<EPI>::run(a, s);
     const dim3 grid((a.N + kRowsPerWG - 1) / kRowsPerWG);
     gemv_i8_kernel<MT, EPI><<<grid, 256, 0, s>>>(a.M, a.N, a.K, a.A, a.BT, a.sA, a.sB, a.bias,
                                                   a.residual, a.C);
@@ -969,6 +1214,8 @@ void launch_gemv_i8(const GemmArgs& a, hipStream_t s) {
     if (a.M == 0 || a.N == 0) return;
     if (vec_ok(a))
         dispatch_epilogue<GemvLaunch>(a.epi, a, s);
+    else if (any_applies(a))
+        dispatch_epilogue<AnyLaunch>(a.epi, a, s);
     else
         dispatch_epilogue<GenericLaunch>(a.epi, a, s);
 }

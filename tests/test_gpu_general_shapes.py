@@ -1,0 +1,66 @@
+"""Widths and alignments that no kernel is specialised for, through the public
+entry points: the kernels that take K, N and the operands' alignment at run
+time, at the sizes where their tiles, slices and last chunks end."""
+import numpy as np
+import pytest
+
+from conftest import pack_i8, rng
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev(a):
+    import torch
+
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def _padded(a, words):
+    """The int8 matrix as device words that start `words` words past a 256-byte boundary, 0x7f bytes on both sides (a
+    read past a row's end would show in the sums)."""
+    import torch
+
+    flat = pack_i8(a).reshape(-1)
+    buf = torch.full((words + flat.size + 64,), 0x7F7F7F7F, dtype=torch.int32, device="cuda")
+    buf[words:words + flat.size] = torch.from_numpy(flat)
+    return buf[words:words + flat.size].view(a.shape[0], -1)
+
+
+def _gemm_case(ie, orc, M, N, K, epi, words, seed):
+    r = rng(seed)
+    A = r.integers(-128, 128, (M, K), dtype=np.int64).astype(np.int8)
+    B = r.integers(-128, 128, (N, K), dtype=np.int64).astype(np.int8)
+    Ap, Bp = _padded(A, words), _padded(B, words)
+    if epi == ie.EPI_I32:
+        got = ie.int8_gemm(Ap, Bp, epilogue=epi).cpu().numpy()
+        assert np.array_equal(got, orc.gemm_i32(pack_i8(A), pack_i8(B)))
+        return
+    sA, sB = (r.uniform(1e-3, 1e-2, n).astype(np.float32) for n in (M, N))
+    bias = r.standard_normal(N).astype(np.float32)
+    res = r.standard_normal((M, N)).astype(np.float32)
+    out = _dev(res)  # the residual in place
+    got = ie.int8_gemm(Ap, Bp, _dev(sA), _dev(sB), epi, _dev(bias) if epi else None, out if epi == 3 else None,
+                       out if epi == 3 else None).cpu().numpy()
+    want = orc.gemm(pack_i8(A), pack_i8(B), sA, sB, epi, bias if epi else None, res if epi == 3 else None)
+    if epi == ie.EPI_BIAS_GELU:  # the device and host tanhf differ in their last bits; 1 + tanh cancels near -1
+        v = orc.gemm(pack_i8(A), pack_i8(B), sA, sB, ie.EPI_BIAS, bias, None)
+        assert (np.abs(got - want) <= 2e-6 * np.abs(want) + 1.2e-7 * np.abs(v)).all()
+    else:
+        assert np.array_equal(got, want)
+
+
+# Decode rows.  K: one 16-byte chunk, a straddling chunk (K % 16 != 0) in a first, middle and last step, just past a
+# 256-byte step, and slices of uneven length; N: one feature, a partial 4-feature item, fewer items than workgroups,
+# several items per wave; M: one, two and four blocks of activation rows, each full and partial.
+@pytest.mark.parametrize("K,N,words", [(16, 5, 0), (20, 1, 1), (252, 33, 0), (260, 1030, 1), (1000, 515, 3),
+                                       (1040, 4099, 0), (2176, 500, 0), (4096, 9, 0), (4100, 4097, 1), (8188, 301, 0),
+                                       (1536, 9001, 0), (3072, 4100, 0), (8192, 700, 0), (768, 4099, 2)])
+@pytest.mark.parametrize("M", [1, 2, 4, 5, 8, 9, 16])
+def test_gemv_any_width(ie, orc, M, K, N, words):
+    _gemm_case(ie, orc, M, N, K, ie.EPI_I32, words, 3 * M + K + N)
+
+
+@pytest.mark.parametrize("M,K,N,words", [(1, 1000, 1030, 1), (6, 2176, 501, 0), (16, 4096, 1027, 0), (16, 10176, 37, 0)])
+@pytest.mark.parametrize("epi", [0, 1, 2, 3])
+def test_gemv_any_width_epilogues(ie, orc, epi, M, K, N, words):
+    _gemm_case(ie, orc, M, N, K, epi, words, M + K + N + epi)
