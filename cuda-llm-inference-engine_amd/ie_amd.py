@@ -102,6 +102,7 @@ class IeError(RuntimeError):
 
 
 _lib = None
+_fns: dict = {}  # entry points by name, filled by load()
 
 
 def load() -> ctypes.CDLL:
@@ -126,6 +127,7 @@ def load() -> ctypes.CDLL:
             fn = getattr(lib, name)
             fn.restype = res
             fn.argtypes = args
+            _fns[name] = fn
         _lib = lib
     return _lib
 
@@ -136,48 +138,71 @@ def last_error() -> str:
 
 def call(name: str, *args) -> int:
     """Calls an ie_* entry point and returns its status without raising."""
-    return getattr(load(), name)(*args)
+    fn = _fns.get(name)
+    if fn is None:
+        fn = getattr(load(), name)
+    return fn(*args)
 
 
 def check(name: str, *args) -> None:
-    st = call(name, *args)
+    fn = _fns.get(name)
+    st = fn(*args) if fn is not None else call(name, *args)
     if st != IE_OK:
         raise IeError(name, st, last_error())
 
 
 # ---------------------------------------------------------------- torch glue
+# A call's own cost matters here: a decode step's small operations take 2-5 us
+# on the GPU.  Pointers and the stream cross as plain integers (the argument
+# types convert them), the current stream is read without building a stream
+# object, and torch is imported only where a wrapper allocates: 7.2 -> 3.9 us
+# for a quantizer call, of which the launch itself is about 3.
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_raw_stream = None  # () -> handle of the current device's current stream
+
+
+def _bind_raw_stream():
+    global _raw_stream
+    import torch
+
+    torch.cuda.current_stream()  # initialises the device as a first use does
+    get_device, get_stream = torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream
+    _raw_stream = lambda: get_stream(get_device())  # noqa: E731
+    return _raw_stream
 
 
 def _stream(stream=None):
-    import torch
-
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    if stream is not None:
+        return stream.cuda_stream
+    return (_raw_stream or _bind_raw_stream())()
 
 
 def quantize(x, out_packed=None, out_scales=None, stream=None):
     """x: [rows, cols] fp32 cuda -> (packed int32 [rows, cols/4], scales [rows])."""
-    import torch
-
     rows, cols = x.shape
-    packed = out_packed if out_packed is not None else torch.empty(
-        (rows, cols // 4), dtype=torch.int32, device=x.device)
-    scales = out_scales if out_scales is not None else torch.empty(
-        rows, dtype=torch.float32, device=x.device)
-    check("ie_quantize_fp32_to_int8", rows, cols, _ptr(x), _ptr(packed), _ptr(scales), _stream(stream))
-    return packed, scales
+    if out_packed is None or out_scales is None:
+        import torch
+
+        if out_packed is None:
+            out_packed = torch.empty((rows, cols // 4), dtype=torch.int32, device=x.device)
+        if out_scales is None:
+            out_scales = torch.empty(rows, dtype=torch.float32, device=x.device)
+    check("ie_quantize_fp32_to_int8", rows, cols, x.data_ptr(), out_packed.data_ptr(), out_scales.data_ptr(),
+          _stream(stream))
+    return out_packed, out_scales
 
 
 def int8_gemm(A_packed, BT_packed, sA=None, sB=None, epilogue=EPI_PLAIN, bias=None,
               residual=None, out=None, path=PATH_AUTO, stream=None):
     """Returns C [M, N] (fp32, or int32 for EPI_I32)."""
-    import torch
-
     M, K4 = A_packed.shape
     N = BT_packed.shape[0]
     if out is None:
+        import torch
+
         dt = torch.int32 if epilogue == EPI_I32 else torch.float32
         out = torch.empty((M, N), dtype=dt, device=A_packed.device)
     check("ie_int8_gemm_ex", M, N, 4 * K4, _ptr(A_packed), _ptr(BT_packed), _ptr(sA), _ptr(sB),
@@ -196,15 +221,16 @@ def workspace_bytes(B: int, H_q: int, d: int, splits: int) -> int:
 def decode_attn(Q, k_cache, v_cache, block_table, context_lens, max_ctx, block_size, H_kv,
                 kv_dtype=KV_F32, splits=0, out=None, workspace=None, stream=None):
     """Q [B, H_q, d] fp32; caches [P, bs, H_kv, d]; returns O [B, H_q, d]."""
-    import torch
-
     B, H_q, d = Q.shape
     nbps = block_table.shape[1]
-    S = num_splits(max_ctx, block_size, splits)
-    need = workspace_bytes(B, H_q, d, S)
     if workspace is None:
+        import torch
+
+        need = workspace_bytes(B, H_q, d, num_splits(max_ctx, block_size, splits))
         workspace = torch.empty(max(need // 4, 1), dtype=torch.float32, device=Q.device)
     if out is None:
+        import torch
+
         out = torch.empty_like(Q)
     check("ie_decode_attn", B, H_q, H_kv, d, _ptr(Q), _ptr(k_cache), _ptr(v_cache), kv_dtype,
           _ptr(block_table), _ptr(context_lens), max_ctx, block_size, nbps, _ptr(out),
@@ -216,10 +242,10 @@ def decode_attn_noalloc(Q, k_cache, v_cache, block_table, context_lens, max_ctx,
                         kv_dtype=KV_F32, splits=0, out=None, stream=None):
     """ie_decode_attn_noalloc: as decode_attn, split partials in the library's
     per-device scratch (no workspace)."""
-    import torch
-
     B, H_q, d = Q.shape
     if out is None:
+        import torch
+
         out = torch.empty_like(Q)
     check("ie_decode_attn_noalloc", B, H_q, H_kv, d, _ptr(Q), _ptr(k_cache), _ptr(v_cache), kv_dtype,
           _ptr(block_table), _ptr(context_lens), max_ctx, block_size, block_table.shape[1], _ptr(out),
@@ -231,10 +257,10 @@ def prefill_attn(Q, k_cache, v_cache, block_table, start_pos, block_size, H_kv, 
                  out=None, stream=None):
     """Q [B, P, H_q, d] fp32 (token t at position start_pos + t, its K/V already
     cached); returns causal O [B, P, H_q, d]."""
-    import torch
-
     B, P, H_q, d = Q.shape
     if out is None:
+        import torch
+
         out = torch.empty_like(Q)
     check("ie_prefill_attn", B, P, H_q, H_kv, d, _ptr(Q), _ptr(k_cache), _ptr(v_cache), kv_dtype,
           _ptr(block_table), block_table.shape[1], block_size, start_pos, _ptr(out), _stream(stream))
@@ -243,10 +269,10 @@ def prefill_attn(Q, k_cache, v_cache, block_table, start_pos, block_size, H_kv, 
 
 def flash_attn(Q, K, V, causal=True, out=None, stream=None):
     """Q, K, V [B, H, N, d] fp32 -> O [B, H, N, d] (run_flash_attn_v2)."""
-    import torch
-
     B, H, N, d = Q.shape
     if out is None:
+        import torch
+
         out = torch.empty_like(Q)
     check("ie_flash_attn", B, H, N, d, _ptr(Q), _ptr(K), _ptr(V), _ptr(out), int(causal), _stream(stream))
     return out
@@ -268,10 +294,11 @@ def kv_cache_append_batch(K, V, k_cache, v_cache, block_table, positions, block_
 
 
 def layernorm(x, gamma, beta, out=None, eps=1e-5, stream=None):
-    import torch
-
     rows, cols = x.shape
-    out = out if out is not None else torch.empty_like(x)
+    if out is None:
+        import torch
+
+        out = torch.empty_like(x)
     check("ie_layernorm", rows, cols, _ptr(x), _ptr(gamma), _ptr(beta), _ptr(out), eps, _stream(stream))
     return out
 
@@ -279,11 +306,12 @@ def layernorm(x, gamma, beta, out=None, eps=1e-5, stream=None):
 def layernorm_residual(x, residual, gamma, beta, out=None, residual_out=None, eps=1e-5, stream=None):
     """(LayerNorm(x + residual), x + residual); out / residual_out may alias
     the inputs."""
-    import torch
-
     rows, cols = x.shape
-    out = out if out is not None else torch.empty_like(x)
-    residual_out = residual_out if residual_out is not None else torch.empty_like(x)
+    if out is None or residual_out is None:
+        import torch
+
+        out = torch.empty_like(x) if out is None else out
+        residual_out = torch.empty_like(x) if residual_out is None else residual_out
     check("ie_layernorm_residual", rows, cols, _ptr(x), _ptr(residual), _ptr(gamma), _ptr(beta), _ptr(out),
           _ptr(residual_out), eps, _stream(stream))
     return out, residual_out
@@ -300,11 +328,12 @@ def embedding(ids, start_pos, wte, wpe, out=None, stream=None):
 
 
 def vocab_proj(h, wte, out=None, stream=None):
-    import torch
-
     rows, d = h.shape
     V = wte.shape[0]
-    out = out if out is not None else torch.empty((rows, V), dtype=torch.float32, device=h.device)
+    if out is None:
+        import torch
+
+        out = torch.empty((rows, V), dtype=torch.float32, device=h.device)
     check("ie_vocab_proj", rows, _ptr(h), _ptr(wte), _ptr(out), d, V, _stream(stream))
     return out
 
