@@ -1,4 +1,6 @@
-// gemm_i8_mfma.hip — INT8 GEMM on the gfx950 i8 matrix cores.
+// gemm_i8_mfma.hip — INT8 GEMM on the gfx950 i8 matrix cores: the dispatch,
+// and the kernel for widths and alignments that the copying kernels cannot
+// take.
 //
 // Same result as the reference's K14 kernel (kernels/quantization/
 // 14_int8_gemm.cu:65-170): exact int32 sum over K of int8 products, then the
@@ -6,13 +8,19 @@
 // register tile; here the sum runs on v_mfma_i32_32x32x32_i8 (32x32 outputs,
 // 32 K-bytes per instruction) with LDS-staged int8 tiles.
 //
-// Tiling: a 256-thread workgroup (4 waves, 2x2) computes a 128x128 tile of C;
-// each wave a 64x64 sub-tile as 2x2 MFMA blocks (64 int32 accumulators/lane).
-// K advances 64 bytes per step; the next step's A/B tiles are fetched from
-// global memory into registers while the current step runs on the matrix
-// cores, then written to the other half of a double-buffered LDS (one barrier
-// per step).  LDS rows are padded from 64 to 80 bytes, which makes both the
-// 16-byte writes and the 16-byte MFMA-operand reads bank-conflict free.
+// The kernel here: rows at any 4-byte address (K % 4 == 0, K >= 16).  Direct
+// copies into LDS want 16-byte aligned sources, so the operands pass through
+// registers: a 256-thread workgroup (4 waves, 2x2, one 32x32 block each) owns
+// a 64x64 tile of C; K advances 128 bytes per stage through two LDS buffers,
+// and a stage's loads are issued two stages before they are written, so two
+// stages are in flight per workgroup, with several workgroups per CU.  LDS
+// rows are 128 bytes with chunk c of row r at slot c ^ ((r >> 1) & 7).  A
+// chunk past the row's end is read as the row's last 16 bytes on both sides,
+// and the A words already counted (all of them past K) are zeroed.
+// Bound by its stages' memory latency; one thread per output, which took
+// these before, read every row uncoalesced: M = 512, K = 1000, N = 3000 1513 ->
+// 9.9 us, M = 100, K = N = 1000 104 -> 5.6.  It also takes K < 128, too short
+// for a whole stage (M = N = 2048, K = 80: 13.6 us on 128x128 tiles, 6.9).
 //
 // MFMA operand convention: lane l supplies row (l % 32) of A and column
 // (l % 32) of B, each with 16 K-bytes; A and B take the same K-bytes from the
@@ -28,129 +36,128 @@
 namespace ie {
 namespace {
 
-constexpr int BM = 128, BN = 128, BK = 64;
-constexpr int LDS_STRIDE = BK + 16;           // bytes per LDS row
-constexpr int TILE_BYTES = BM * LDS_STRIDE;   // one operand, one stage
+constexpr int BM = 64, BN = 64, BK = 128;
+constexpr int CHUNKS = BK / 16;       // 16-byte chunks per LDS row
+constexpr int OPER = BM * BK;         // bytes of one operand, one stage
+constexpr int PER = OPER / 16 / 256;  // chunks of an operand per thread
 
-struct TileRegs {
-    i32x4 a[2];
-    i32x4 b[2];
-};
-
-__device__ __forceinline__ void load_tile(TileRegs& r, const int8_t* __restrict__ A,
-                                          const int8_t* __restrict__ BT, int M, int N,
-                                          int K, int m0, int n0, int k0) {
-    const int t = threadIdx.x;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int row = (t >> 2) + h * 64;
-        const int kc = k0 + (t & 3) * 16;
-        const i32x4 zero = {0, 0, 0, 0};
-        const int gm = m0 + row, gn = n0 + row;
-        r.a[h] = (gm < M && kc < K)
-                     ? *reinterpret_cast<const i32x4*>(A + (size_t)gm * K + kc)
-                     : zero;
-        r.b[h] = (gn < N && kc < K)
-                     ? *reinterpret_cast<const i32x4*>(BT + (size_t)gn * K + kc)
-                     : zero;
-    }
-}
-
-__device__ __forceinline__ void store_tile(const TileRegs& r, int8_t* As, int8_t* Bs) {
-    const int t = threadIdx.x;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        const int row = (t >> 2) + h * 64;
-        const int off = row * LDS_STRIDE + (t & 3) * 16;
-        *reinterpret_cast<i32x4*>(As + off) = r.a[h];
-        *reinterpret_cast<i32x4*>(Bs + off) = r.b[h];
-    }
+__device__ __forceinline__ int slot_of(int row, int chunk) {
+    return row * BK + ((chunk ^ ((row >> 1) & 7)) << 4);
 }
 
 template <int EPI>
-__global__ __launch_bounds__(256) void gemm_i8_mfma_kernel(
+__global__ __launch_bounds__(256) void gemm_i8_ragged_kernel(
     int M, int N, int K, const int8_t* __restrict__ A, const int8_t* __restrict__ BT,
     const float* __restrict__ sA, const float* __restrict__ sB, const float* bias,
     const float* residual, void* C) {
-    __shared__ __attribute__((aligned(16))) int8_t lds[2 * 2 * TILE_BYTES];
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    typedef i32x4 i32x4_a4 __attribute__((aligned(4)));
+    __shared__ __attribute__((aligned(16))) int8_t lds[2][2][OPER];  // [buffer][A, B]
+    const int t = threadIdx.x, lane = t & 63;
+    const int wave = t >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-
-    i32x16 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0;
-
     const int nk = (K + BK - 1) / BK;
-    TileRegs r;
-    load_tile(r, A, BT, M, N, K, m0, n0, 0);
-    store_tile(r, lds, lds + TILE_BYTES);
-    __syncthreads();
 
-    const int lrow = lane & 31;
-    const int lk = (lane >> 5) * 16;
-    for (int kt = 0; kt < nk; ++kt) {
-        const int cur = kt & 1;
-        const int8_t* As = lds + cur * 2 * TILE_BYTES;
-        const int8_t* Bs = As + TILE_BYTES;
-        if (kt + 1 < nk) load_tile(r, A, BT, M, N, K, m0, n0, (kt + 1) * BK);
+    // This thread's chunks: rows t / 8 + 32 j, chunk t % 8.
+    const int crow = t / CHUNKS, cc = t % CHUNKS;
+    const int8_t* pa[PER];
+    const int8_t* pb[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        pa[j] = A + (size_t)min(m0 + crow + 32 * j, M - 1) * K;
+        pb[j] = BT + (size_t)min(n0 + crow + 32 * j, N - 1) * K;
+    }
+    struct Regs {
+        i32x4 a[PER], b[PER];
+    };
+    auto load = [&](Regs& r, int kt) {
+        const int k = min(kt * BK + cc * 16, K - 16);
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            r.a[j] = *reinterpret_cast<const i32x4_a4*>(pa[j] + k);
+            r.b[j] = *reinterpret_cast<const i32x4_a4*>(pb[j] + k);
+        }
+    };
+    auto store = [&](const Regs& r, int kt) {
+        const int over = kt * BK + cc * 16 + 16 - K;  // bytes of the chunk past K
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            i32x4 a = r.a[j];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) a[w] = 4 * w < over ? 0 : a[w];
+            *reinterpret_cast<i32x4*>(lds[kt & 1][0] + slot_of(crow + 32 * j, cc)) = a;
+            *reinterpret_cast<i32x4*>(lds[kt & 1][1] + slot_of(crow + 32 * j, cc)) = r.b[j];
+        }
+    };
+
+    i32x16 acc;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] = 0;
+    const int frow = lane & 31, fchunk = lane >> 5;
+    // Stage kt from LDS while stages kt + 1 (in r) and kt + 2 are in flight;
+    // kt + 1 goes into the other buffer, free since the last barrier.
+    auto step = [&](Regs& r, int kt) {
+        const int8_t* sa = lds[kt & 1][0];
+        const int8_t* sb = lds[kt & 1][1];
 #pragma unroll
         for (int ks = 0; ks < BK / 32; ++ks) {
-            i32x4 af[2], bf[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-                af[i] = *reinterpret_cast<const i32x4*>(
-                    As + (wm * 64 + i * 32 + lrow) * LDS_STRIDE + ks * 32 + lk);
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-                bf[j] = *reinterpret_cast<const i32x4*>(
-                    Bs + (wn * 64 + j * 32 + lrow) * LDS_STRIDE + ks * 32 + lk);
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[i], bf[j], acc[i][j],
-                                                                     0, 0, 0);
+            const i32x4 af = *reinterpret_cast<const i32x4*>(sa + slot_of(wm * 32 + frow, ks * 2 + fchunk));
+            const i32x4 bf = *reinterpret_cast<const i32x4*>(sb + slot_of(wn * 32 + frow, ks * 2 + fchunk));
+            acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bf, acc, 0, 0, 0);
         }
-        if (kt + 1 < nk) {
-            int8_t* Ns = lds + (cur ^ 1) * 2 * TILE_BYTES;
-            store_tile(r, Ns, Ns + TILE_BYTES);
-        }
+        if (kt + 1 < nk) store(r, kt + 1);
+        load(r, kt + 3);  // past the last stage: its last chunks again, never stored
         __syncthreads();
+    };
+    Regs r0, r1;
+    load(r0, 0);
+    load(r1, 1);
+    store(r0, 0);
+    load(r0, 2);
+    __syncthreads();
+    for (int kt = 0; kt < nk; kt += 2) {
+        step(r1, kt);
+        if (kt + 1 >= nk) break;
+        step(r0, kt + 1);
     }
 
+    // Every operand the stores need first (clamped indices), as in
+    // gemm_i8_tile.hip.
+    const int rbase = m0 + wm * 32 + 4 * (lane >> 5);
+    const int n = n0 + wn * 32 + (lane & 31), nc = min(n, N - 1);
+    constexpr bool HAS_BIAS = EPI == IE_EPI_BIAS || EPI == IE_EPI_BIAS_GELU || EPI == IE_EPI_BIAS_RESIDUAL;
+    constexpr bool HAS_RES = EPI == IE_EPI_BIAS_RESIDUAL;
+    float sa[16] = {}, rv[16] = {}, sb = 0.0f, bv = 0.0f;
+    auto row = [&](int v) { return rbase + 8 * (v >> 2) + (v & 3); };
+    if constexpr (EPI != IE_EPI_I32) {
+        sb = sB[nc];
+        if constexpr (HAS_BIAS) bv = bias[nc];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int n = n0 + wn * 64 + j * 32 + (lane & 31);
-            if (n >= N) continue;
-            float sb = 0.0f;
-            if constexpr (EPI != IE_EPI_I32) sb = sB[n];
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int m = m0 + wm * 64 + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
-                if (m < M) {
-                    float sa = 0.0f;
-                    if constexpr (EPI != IE_EPI_I32) sa = sA[m];
-                    store_epilogue<EPI>(C, (size_t)m * N + n, acc[i][j][v], sa, sb, bias,
-                                        residual, n);
-                }
-            }
+        for (int v = 0; v < 16; ++v) {
+            const int m = min(row(v), M - 1);
+            sa[v] = sA[m];
+            if constexpr (HAS_RES) rv[v] = residual[(size_t)m * N + nc];
         }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            asm volatile("" ::"v"(sa[v]));
+            if constexpr (HAS_RES) asm volatile("" ::"v"(rv[v]));
+        }
+        asm volatile("" ::"v"(sb));
+        if constexpr (HAS_BIAS) asm volatile("" ::"v"(bv));
+    }
+    if (n < N) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+            if (row(v) < M) store_epilogue_v<EPI>(C, (size_t)row(v) * N + n, acc[v], sa[v], sb, bv, rv[v]);
     }
 }
 
 template <int EPI>
-struct MfmaLaunch {
+struct RaggedLaunch {
     static void run(const GemmArgs& a, hipStream_t s) {
         const dim3 grid((a.N + BN - 1) / BN, (a.M + BM - 1) / BM);
-        gemm_i8_mfma_kernel<EPI><<<grid, 256, 0, s>>>(
+        gemm_i8_ragged_kernel<EPI><<<grid, 256, 0, s>>>(
             a.M, a.N, a.K, reinterpret_cast<const int8_t*>(a.A),
             reinterpret_cast<const int8_t*>(a.BT), a.sA, a.sB, a.bias, a.residual, a.C);
     }
@@ -171,8 +178,12 @@ void launch_gemm_i8_qkv_route(const GemmArgs& a, hipStream_t s) {
 void launch_gemm_i8_mfma(const GemmArgs& a, hipStream_t s) {
     if (a.M == 0 || a.N == 0) return;
     const bool vec = (a.K % 16) == 0 && ((uintptr_t)a.A % 16) == 0 && ((uintptr_t)a.BT % 16) == 0;
-    if (!vec) {
-        launch_gemm_i8_generic(a, s);
+    if (!vec || a.K < 128) {
+        // K < 16, or more 64-row tiles than a grid has in y: one thread per output
+        if (a.K >= 16 && (a.M + BM - 1) / BM <= 65535)
+            dispatch_epilogue<RaggedLaunch>(a.epi, a, s);
+        else
+            launch_gemm_i8_generic(a, s);
         return;
     }
     if (gemm_i8_wide_applies(a)) {
@@ -192,11 +203,10 @@ void launch_gemm_i8_mfma(const GemmArgs& a, hipStream_t s) {
     // Prefill-sized problems: the multi-stage LDS tile kernel (M = 2048:
     // 22.1 -> 12.1 us at N = 2304, 37.7 -> 13.0 us at K = 3072, N = 768;
     // at par with or ahead of hipBLASLt on the same shapes).
-    if (gemm_i8_tile_applies(a)) {
+    if (gemm_i8_tile_applies(a))
         launch_gemm_i8_tile(a, s);
-        return;
-    }
-    dispatch_epilogue<MfmaLaunch>(a.epi, a, s);
+    else
+        dispatch_epilogue<RaggedLaunch>(a.epi, a, s);
 }
 
 }  // namespace ie

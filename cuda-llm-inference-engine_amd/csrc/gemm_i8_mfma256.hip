@@ -36,8 +36,11 @@
 //     stores: vmcnt counts stores too, so a wait for copies issued after the
 //     stores would drain them (8192^3: 437.8 -> 431.8 us, medians of 6
 //     alternated same-box runs, same bits).
-// Requirements (checked by the launcher): K % 128 == 0, 16-byte aligned A/BT.
-// Rows past M or N read the last valid row (no fault, results discarded).
+// Requirements (checked by the launcher): K % 16 == 0, K >= 128, 16-byte
+// aligned A/BT.  Rows past M or N read the last valid row (no fault, results
+// discarded).  K % 128 != 0 (TAIL): the last stage covers the row's last 128
+// bytes, and the A fragments of chunks that the stage before already counted
+// are zeroed (that stage's body is peeled, so the loop is the same).
 #include <algorithm>
 #include <type_traits>
 
@@ -121,7 +124,7 @@ __device__ __forceinline__ void quad_transpose(int32_t (&x)[4], int j) {
 // of 128 x 64 (two per SIMD, so one wave's MFMAs can run while the other
 // waits at the stage barrier or for its copies).
 // BUF: M*K and N*K below 2^31, so operands take the buffer-form copies.
-template <int EPI, int NW, bool BUF>
+template <int EPI, int NW, bool BUF, bool TAIL>
 __global__ __launch_bounds__(64 * NW, 1) void gemm_i8_256_kernel(
     int M, int N, int K, const int8_t* __restrict__ A, const int8_t* __restrict__ BT,
     const float* __restrict__ sA, const float* __restrict__ sB, const float* bias,
@@ -159,7 +162,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_i8_256_kernel(
 
     i32x16 acc[4][NJ];
 
-    const int nk = K / BK;
+    const int nk = TAIL ? (K + BK - 1) / BK : K / BK;
     constexpr bool HAS_BIAS = EPI == IE_EPI_BIAS || EPI == IE_EPI_BIAS_GELU || EPI == IE_EPI_BIAS_RESIDUAL;
     constexpr bool HAS_RES = EPI == IE_EPI_BIAS_RESIDUAL;
     // Full tiles of a C with 16-byte rows (N % 4 == 0) leave through the
@@ -187,7 +190,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_i8_256_kernel(
                      const uint32_t (&ob)[LOADS_PER_WAVE]) {
         int8_t* sa = lds + slot * STAGE;
         int8_t* sb = sa + OPER;
-        const int k0 = kt_src * BK;
+        const int k0 = TAIL ? min(kt_src * BK, K - BK) : kt_src * BK;
 #pragma unroll
         for (int j = 0; j < LOADS_PER_WAVE; ++j) {
             const int r0 = (wave * LOADS_PER_WAVE + j) * ROWS_PER_LOAD;
@@ -221,6 +224,15 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_i8_256_kernel(
         for (int i = 0; i < 4; ++i) af[slot][i] = read_frag(sa, wm * 128 + i * 32 + frow, ks * 2 + fchunk);
 #pragma unroll
         for (int j = 0; j < NJ; ++j) bf[slot][j] = read_frag(sb, wn * 32 * NJ + j * 32 + frow, ks * 2 + fchunk);
+    };
+    // TAIL, last stage: zero the A fragments of k-substep ks that lie in the
+    // first `skip` bytes of the stage
+    const int skip = nk * BK - K;
+    auto drop_counted = [&](int ks, int slot) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) af[slot][i][v] = (ks * 2 + fchunk) * 16 < skip ? 0 : af[slot][i][v];
     };
     auto mfma_rows = [&](int slot, int i0, int i1) {
 #pragma unroll
@@ -265,6 +277,7 @@ __global__ __launch_bounds__(64 * NW, 1) void gemm_i8_256_kernel(
 #pragma unroll
         for (int ks = 0; ks < SUB; ++ks) {
             const int slot = ks & 1;
+            if constexpr (TAIL && NEXT) drop_counted(ks, slot);
             __builtin_amdgcn_sched_barrier(0);
             if (ks + 1 < SUB) {
                 // MFMAs on this substep's slot; in their shadow the next
@@ -462,21 +475,18 @@ struct BigLaunch {
         const bool buf = (long long)a.M * a.K < (1LL << 31) && (long long)a.N * a.K < (1LL << 31);
         // one persistent workgroup per CU (128 KiB of LDS each)
         const unsigned grid = (unsigned)std::min<long long>((long long)tm * tn, num_cus());
-        if (buf)
-            gemm_i8_256_kernel<EPI, NW, true><<<grid, 64 * NW, 0, s>>>(
-                a.M, a.N, a.K, reinterpret_cast<const int8_t*>(a.A), reinterpret_cast<const int8_t*>(a.BT),
-                a.sA, a.sB, a.bias, a.residual, a.C, tm, tn);
-        else
-            gemm_i8_256_kernel<EPI, NW, false><<<grid, 64 * NW, 0, s>>>(
-                a.M, a.N, a.K, reinterpret_cast<const int8_t*>(a.A), reinterpret_cast<const int8_t*>(a.BT),
-                a.sA, a.sB, a.bias, a.residual, a.C, tm, tn);
+        const bool tail = a.K % BK != 0;
+        auto* k = buf ? (tail ? gemm_i8_256_kernel<EPI, NW, true, true> : gemm_i8_256_kernel<EPI, NW, true, false>)
+                      : (tail ? gemm_i8_256_kernel<EPI, NW, false, true> : gemm_i8_256_kernel<EPI, NW, false, false>);
+        k<<<grid, 64 * NW, 0, s>>>(a.M, a.N, a.K, reinterpret_cast<const int8_t*>(a.A),
+                                   reinterpret_cast<const int8_t*>(a.BT), a.sA, a.sB, a.bias, a.residual, a.C, tm, tn);
     }
 };
 
 }  // namespace
 
 bool gemm_i8_big_applies(const GemmArgs& a) {
-    if (a.K % BK != 0 || a.K == 0) return false;
+    if (a.K % 16 != 0 || a.K < BK) return false;
     if (((uintptr_t)a.A % 16) || ((uintptr_t)a.BT % 16)) return false;
     const long long tiles = (long long)((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
     return tiles >= 128 && tiles < (1LL << 31);

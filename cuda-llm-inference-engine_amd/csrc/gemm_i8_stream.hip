@@ -30,9 +30,10 @@
 //   * KS = 2 (K split over two waves, their int32 tiles added in LDS, exact)
 //     measured best at K = 640-3072; one, three or four waves were slower
 //     (M = 128, K = 3072: 8.8 / 6.9 / 6.9 / 7.3 us for KS = 1 / 2 / 3 / 4).
-// Requirements (checked by gemm_i8_stream_applies): K % 128 == 0, 16-byte
-// aligned A and BT.  Rows past M or N read the last valid row (results
-// discarded).
+// Requirements (checked by gemm_i8_stream_applies): K % 16 == 0, K >= 128,
+// 16-byte aligned A and BT.  Rows past M or N read the last valid row (results
+// discarded).  K % 128 != 0 (TAIL): the last group covers the row's last 128
+// bytes, the A chunks already counted copied from a block of zeros.
 #include "device_util.h"
 #include "epilogue.h"
 #include "ie_internal.h"
@@ -50,25 +51,30 @@ typedef const __attribute__((address_space(1))) void* gbl_ptr_t;
 
 __device__ __forceinline__ int swz(int r) { return (r >> 1) & 7; }
 
+__device__ __attribute__((aligned(16))) int8_t g_zero_chunk[16];
+
 // Rows [r0, r0 + 8) x 128 bytes at K offset k0 of a K-contiguous operand
 // into LDS with one wave-wide 16-byte-per-lane direct load: lane l fetches
 // chunk (l % 8) ^ swz(r) of row r = r0 + l / 8 into slot l % 8, so chunk c of
 // row r lands at slot c ^ swz(r).
+// SKIP: the first `skip` bytes of each row (a multiple of 16) as zeros.
+template <bool SKIP = false>
 __device__ __forceinline__ void copy_rows(const int8_t* __restrict__ src, int ld, int rows_valid, int row0, int k0,
-                                          int r0, int8_t* dst) {
+                                          int r0, int8_t* dst, int skip = 0) {
     const int lane = threadIdx.x & 63;
     const int r = r0 + (lane >> 3);
     const int c = (lane & 7) ^ swz(r);
     const int gr = min(row0 + r, rows_valid - 1);
-    __builtin_amdgcn_global_load_lds((gbl_ptr_t)(src + (size_t)gr * ld + k0 + c * 16),
-                                     (lds_ptr_t)(dst + r0 * KG), 16, 0, 0);
+    const int8_t* g = src + (size_t)gr * ld + k0 + c * 16;
+    if constexpr (SKIP) g = c * 16 < skip ? g_zero_chunk : g;
+    __builtin_amdgcn_global_load_lds((gbl_ptr_t)g, (lds_ptr_t)(dst + r0 * KG), 16, 0, 0);
 }
 
 __device__ __forceinline__ i32x4 read_frag(const int8_t* oper, int row, int chunk) {
     return *reinterpret_cast<const i32x4*>(oper + row * KG + ((chunk ^ swz(row)) << 4));
 }
 
-template <int EPI, int KS>
+template <int EPI, int KS, bool TAIL>
 __global__ __launch_bounds__(64 * KS) void gemm_i8_stream_kernel(
     int M, int N, int K, const int8_t* __restrict__ A, const int8_t* __restrict__ BT,
     const float* __restrict__ sA, const float* __restrict__ sB, const float* bias,
@@ -79,7 +85,7 @@ __global__ __launch_bounds__(64 * KS) void gemm_i8_stream_kernel(
     const int wave = KS == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
     int8_t* ring = lds + wave * (LR * LSLOT);
-    const int ngt = K / KG;
+    const int ngt = TAIL ? (K + KG - 1) / KG : K / KG;
     const int g0 = (int)((long long)ngt * wave / KS), g1 = (int)((long long)ngt * (wave + 1) / KS);
     const int nk = g1 - g0;
 
@@ -89,9 +95,9 @@ __global__ __launch_bounds__(64 * KS) void gemm_i8_stream_kernel(
     // Copies group g of the block's A and B rows into ring slot `slot`.
     auto issue = [&](int g, int slot) {
         int8_t* dst = ring + slot * LSLOT;
-        const int k0 = g * KG;
+        const int k0 = TAIL ? min(g * KG, K - KG) : g * KG;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) copy_rows(A, K, M, m0, k0, 8 * j, dst);
+        for (int j = 0; j < 4; ++j) copy_rows<TAIL>(A, K, M, m0, k0, 8 * j, dst, g * KG - k0);
 #pragma unroll
         for (int j = 0; j < 4; ++j) copy_rows(BT, K, N, n0, k0, 8 * j, dst + 32 * KG);
     };
@@ -183,7 +189,10 @@ struct StreamLaunch {
     template <int KS>
     static void go(const GemmArgs& a, hipStream_t s) {
         const dim3 grid((a.N + 31) / 32, (a.M + 31) / 32);
-        gemm_i8_stream_kernel<EPI, KS><<<grid, 64 * KS, 0, s>>>(
+        auto* k = gemm_i8_stream_kernel<EPI, KS, false>;
+        if constexpr (EPI != kEpiQKVRoute)
+            if (a.K % KG) k = gemm_i8_stream_kernel<EPI, KS, true>;
+        k<<<grid, 64 * KS, 0, s>>>(
             a.M, a.N, a.K, reinterpret_cast<const int8_t*>(a.A), reinterpret_cast<const int8_t*>(a.BT),
             a.sA, a.sB, a.bias, a.residual, a.C, a.route);
     }
@@ -204,7 +213,7 @@ struct StreamLaunch {
 // 512 blocks: 5.26-8.8 against 5.47-10.5), behind from the second round on
 // (576 blocks, M = 256, N = 2304: 7.97 against 5.63 us).
 bool gemm_i8_stream_applies(const GemmArgs& a) {
-    if (a.K % KG != 0 || a.K == 0) return false;
+    if (a.K % (a.epi == kEpiQKVRoute ? KG : 16) != 0 || a.K < KG) return false;
     if (((uintptr_t)a.A % 16) || ((uintptr_t)a.BT % 16)) return false;
     const long long blocks = (long long)((a.M + 31) / 32) * ((a.N + 31) / 32);
     return (a.M + 31) / 32 <= 65535 && blocks <= 2LL * num_cus();

@@ -21,8 +21,13 @@
 //   * workgroup ids are remapped so each XCD (ids = xcd mod 8) receives a
 //     contiguous run of tiles, walked in groups of GROUP_M tile rows, so the
 //     workgroups resident on one XCD share A and B panels in its L2.
-// Requirements (checked by the launcher): K % 128 == 0, 16-byte aligned A/BT.
-// Rows past M or N read the last valid row (no fault, results discarded).
+// Requirements (checked by the launcher): K % 16 == 0, K >= 128, 16-byte
+// aligned A/BT.  Rows past M or N read the last valid row (no fault, results
+// discarded).  K % 128 != 0 (TAIL): the last stage covers the row's last 128
+// bytes, and the A chunks of it that the stage before already counted are
+// copied from a block of zeros instead, so every copy stays inside its row
+// and the loop is the same (M = 300, K = 1600, N = 4801 30.2 us on a
+// 128 x 128 register-staged kernel with one step in flight, 12.0 here).
 
 #include "device_util.h"
 #include "epilogue.h"
@@ -40,15 +45,20 @@ typedef const __attribute__((address_space(1))) void* gbl_ptr_t;
 
 __device__ __forceinline__ int swz(int r) { return (r >> 1) & 7; }
 
+__device__ __attribute__((aligned(16))) int8_t g_zero_chunk[16];
+
 // Rows [r0, r0 + 8) x BK bytes of a K-contiguous operand into LDS with one
-// wave-wide 16-byte-per-lane direct load.
+// wave-wide 16-byte-per-lane direct load, the first `skip` bytes of each row
+// (a multiple of 16) as zeros.
+template <bool SKIP = false>
 __device__ __forceinline__ void load_rows(const int8_t* __restrict__ src, int ld, int rows_valid, int row0, int k0,
-                                          int r0, int8_t* lds_oper) {
+                                          int r0, int8_t* lds_oper, int skip = 0) {
     const int lane = threadIdx.x & 63;
     const int r = r0 + lane / CHUNKS;
     const int c = (lane % CHUNKS) ^ swz(r);
     const int gr = min(row0 + r, rows_valid - 1);
     const int8_t* g = src + (size_t)gr * ld + k0 + c * 16;
+    if constexpr (SKIP) g = c * 16 < skip ? g_zero_chunk : g;
     __builtin_amdgcn_global_load_lds((gbl_ptr_t)g, (lds_ptr_t)(lds_oper + r0 * BK), 16, 0, 0);
 }
 
@@ -56,7 +66,7 @@ __device__ __forceinline__ i32x4 read_frag(const int8_t* lds_oper, int row, int 
     return *reinterpret_cast<const i32x4*>(lds_oper + row * BK + ((chunk ^ swz(row)) << 4));
 }
 
-template <int EPI, int BM, int BN, int NSTAGE, bool NT>
+template <int EPI, int BM, int BN, int NSTAGE, bool NT, bool TAIL>
 __global__ __launch_bounds__(256) void gemm_i8_tile_kernel(int M, int N, int K, const int8_t* __restrict__ A,
                                                            const int8_t* __restrict__ BT,
                                                            const float* __restrict__ sA,
@@ -97,16 +107,16 @@ __global__ __launch_bounds__(256) void gemm_i8_tile_kernel(int M, int N, int K, 
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0;
 
-    const int nk = K / BK;
+    const int nk = TAIL ? (K + BK - 1) / BK : K / BK;
     // Copies stage kt_src into LDS slot `slot`.  Every iteration issues one
     // stage, so the loop body is branch-free: past the last stage the copy
     // re-reads stage nk-1 into the slot just freed, which is never read again.
     auto issue = [&](int kt_src, int slot) {
         int8_t* sa = lds + slot * STAGE;
         int8_t* sb = sa + OA;
-        const int k0 = kt_src * BK;
+        const int k0 = TAIL ? min(kt_src * BK, K - BK) : kt_src * BK;
 #pragma unroll
-        for (int j = 0; j < LA; ++j) load_rows(A, K, M, m0, k0, (wave * LA + j) * 8, sa);
+        for (int j = 0; j < LA; ++j) load_rows<TAIL>(A, K, M, m0, k0, (wave * LA + j) * 8, sa, kt_src * BK - k0);
 #pragma unroll
         for (int j = 0; j < LB; ++j) load_rows(BT, K, N, n0, k0, (wave * LB + j) * 8, sb);
     };
@@ -250,9 +260,15 @@ struct TileLaunch {
         // N = 2304 12.5 -> 10.9 us, N = 3072 13.5 -> 11.0 us; at N = 768,
         // 6.3 MB of C, they measured slower: 6.15 -> 6.7 us)
         // (routed stores are plain: Q and the caches are read next)
-        auto* k = gemm_i8_tile_kernel<EPI, BM, BN, NSTAGE, false>;
-        if constexpr (EPI != kEpiQKVRoute)
-            if ((size_t)a.M * a.N * 4 >= ((size_t)16 << 20)) k = gemm_i8_tile_kernel<EPI, BM, BN, NSTAGE, true>;
+        auto* k = gemm_i8_tile_kernel<EPI, BM, BN, NSTAGE, false, false>;
+        if constexpr (EPI != kEpiQKVRoute) {
+            const bool nt = (size_t)a.M * a.N * 4 >= ((size_t)16 << 20);
+            if (a.K % BK)
+                k = nt ? gemm_i8_tile_kernel<EPI, BM, BN, NSTAGE, true, true>
+                       : gemm_i8_tile_kernel<EPI, BM, BN, NSTAGE, false, true>;
+            else if (nt)
+                k = gemm_i8_tile_kernel<EPI, BM, BN, NSTAGE, true, false>;
+        }
         k<<<tm * tn, 256, 0, s>>>(a.M, a.N, a.K, reinterpret_cast<const int8_t*>(a.A),
                                  reinterpret_cast<const int8_t*>(a.BT), a.sA, a.sB, a.bias, a.residual, a.C, tm, tn,
                                  a.route);
@@ -297,7 +313,7 @@ int gemm_i8_tile_shape(const GemmArgs& a) {
 // Grids small enough for one round of 32 x 32 blocks take the K-split
 // stream kernel first (gemm_i8_stream_applies).
 bool gemm_i8_tile_applies(const GemmArgs& a) {
-    if (a.K % BK != 0 || a.K == 0) return false;
+    if (a.K % (a.epi == kEpiQKVRoute ? BK : 16) != 0 || a.K < BK) return false;
     if (((uintptr_t)a.A % 16) || ((uintptr_t)a.BT % 16)) return false;
     const long long t = (long long)((a.M + 63) / 64) * ((a.N + 63) / 64);
     return t < (1LL << 31);

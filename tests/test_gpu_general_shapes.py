@@ -64,3 +64,23 @@ def test_gemv_any_width(ie, orc, M, K, N, words):
 @pytest.mark.parametrize("epi", [0, 1, 2, 3])
 def test_gemv_any_width_epilogues(ie, orc, epi, M, K, N, words):
     _gemm_case(ie, orc, M, N, K, epi, words, M + K + N + epi)
+
+
+# Prompt rows.  K % 16 == 0: the small-grid kernel (one and two 128-byte groups), the 64x64 and 128x64 LDS tiles (two to
+# four stages) and the 256x256 tiles (two and an odd number of stages, a second tile per workgroup), each with a last
+# stage that repeats 16 to 112 bytes.  K % 16 != 0, K < 128 or 4-byte aligned rows: the register-staged kernel, whose
+# last chunk straddles K (K = 20: the only one), with one to eight stages.
+@pytest.mark.parametrize("M,K,N,words", [(40, 144, 700, 0), (17, 240, 33, 0), (40, 8176, 200, 0), (1200, 272, 1100, 0),
+                                         (700, 1616, 1000, 0), (2100, 400, 2200, 0), (2100, 2064, 2200, 0),
+                                         (2900, 272, 3000, 0), (4352, 400, 4352, 0), (17, 16, 5, 0), (17, 20, 9, 1),
+                                         (64, 124, 64, 0), (65, 132, 65, 0), (130, 1000, 700, 3), (300, 768, 301, 1),
+                                         (257, 80, 129, 0)])
+def test_gemm_any_width(ie, orc, M, K, N, words):
+    _gemm_case(ie, orc, M, N, K, ie.EPI_I32, words, M + K + N)
+
+
+@pytest.mark.parametrize("M,K,N,words", [(33, 208, 701, 0), (1200, 272, 1099, 0), (2100, 144, 2200, 0), (2900, 144, 3001, 0),
+                                         (130, 140, 131, 1)])
+@pytest.mark.parametrize("epi", [0, 1, 2, 3])
+def test_gemm_any_width_epilogues(ie, orc, epi, M, K, N, words):
+    _gemm_case(ie, orc, M, N, K, epi, words, M + K + N + epi)
