@@ -12,8 +12,14 @@
 //     wave reduction (no LDS, no barrier);
 //   * cols <= 4096: one 256-thread workgroup per row, up to four float4s per
 //     lane, the four wave maxima combined through LDS;
-//   * wider rows: the same workgroup walks the row twice (max, then
+//   * cols <= 16384: 512 threads per row, four or eight float4s per lane
+//     (two passes by 256 threads before: 1 / 16 x 8192 4.39 / 4.70 -> 2.63 /
+//     2.91 us, 8192 x 8192 91.0 -> 52.9 us, 335 MB at 6.3 TB/s; 256 threads
+//     with eight 2.80 / 3.08 / 61.3, 1024 with two 2.70 / 2.95 / 57.9);
+//   * wider rows: a 256-thread workgroup walks the row twice (max, then
 //     quantize; the second pass hits L2).
+// Inputs past half of the 256 MiB MALL are read non-temporally (8192 x 8192:
+// 61.1 -> 52.9 us; level or slower below: 2048 x 3072 6.95 against 7.26).
 // Every form issues its loads unconditionally with the index clamped into the
 // row, so they all go out before the first wait; a clamped duplicate cannot
 // change the max, and only in-row words are stored.  The max is exact in any
@@ -54,18 +60,33 @@ __global__ __launch_bounds__(256) void quantize_rows_wave_kernel(int rows, int c
         if (lane + 64 * j < n4) o[lane + 64 * j] = quant_word(v[j], inv);
 }
 
-// Maximum of the four waves' m through LDS (every thread gets it).
-__device__ __forceinline__ float block4_max(float m) {
-    __shared__ float wmax[4];
+// Maximum of the T / 64 waves' m through LDS (every thread gets it).
+template <int T>
+__device__ __forceinline__ float block_max(float m) {
+    __shared__ float wmax[T / 64];
     m = wave_max(m);
     if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
     __syncthreads();
-    return fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+    m = wmax[0];
+#pragma unroll
+    for (int w = 1; w < T / 64; ++w) m = fmaxf(m, wmax[w]);
+    return m;
 }
 
-// cols <= 256 NV * 4: one workgroup per row, NV float4s per thread.
-template <int NV>
-__global__ __launch_bounds__(256) void quantize_rows_reg_kernel(int cols, const float* __restrict__ in,
+template <bool NT>
+__device__ __forceinline__ float4 load4(const float4* p) {
+    if constexpr (NT) {
+        typedef float f32x4 __attribute__((ext_vector_type(4)));
+        const f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
+        return make_float4(v.x, v.y, v.z, v.w);
+    } else {
+        return *p;
+    }
+}
+
+// cols <= T NV * 4: one T-thread workgroup per row, NV float4s per thread.
+template <int T, int NV, bool NT = false>
+__global__ __launch_bounds__(T) void quantize_rows_reg_kernel(int cols, const float* __restrict__ in,
                                                                 int32_t* __restrict__ out,
                                                                 float* __restrict__ scales) {
     const int row = blockIdx.x;
@@ -73,18 +94,18 @@ __global__ __launch_bounds__(256) void quantize_rows_reg_kernel(int cols, const 
     const float4* x = reinterpret_cast<const float4*>(in + (size_t)row * cols);
     float4 v[NV];
 #pragma unroll
-    for (int j = 0; j < NV; ++j) v[j] = x[min((int)threadIdx.x + 256 * j, n4 - 1)];
+    for (int j = 0; j < NV; ++j) v[j] = load4<NT>(x + min((int)threadIdx.x + T * j, n4 - 1));
     float m = 0.0f;
 #pragma unroll
     for (int j = 0; j < NV; ++j) m = fmaxf(m, abs_max4(v[j]));
-    m = block4_max(m);
+    m = block_max<T>(m);
     const float scale = quant_scale(m);
     const float inv = 1.0f / scale;
     if (threadIdx.x == 0) scales[row] = scale;
     int32_t* o = out + (size_t)row * n4;
 #pragma unroll
     for (int j = 0; j < NV; ++j)
-        if ((int)threadIdx.x + 256 * j < n4) o[threadIdx.x + 256 * j] = quant_word(v[j], inv);
+        if ((int)threadIdx.x + T * j < n4) o[threadIdx.x + T * j] = quant_word(v[j], inv);
 }
 
 // Any cols: one workgroup per row, two passes.
@@ -97,7 +118,7 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(
 
     float m = 0.0f;
     for (int i = threadIdx.x; i < n4; i += 256) m = fmaxf(m, abs_max4(x[i]));
-    m = block4_max(m);
+    m = block_max<256>(m);
 
     const float scale = quant_scale(m);
     const float inv = 1.0f / scale;
@@ -108,6 +129,8 @@ __global__ __launch_bounds__(256) void quantize_rows_kernel(
         o[i] = quant_word(x[i], inv);
     }
 }
+
+constexpr size_t kStreamInputBytes = 128ull << 20;
 
 }  // namespace
 
@@ -130,12 +153,17 @@ void launch_quantize(int rows, int cols, const float* in, int32_t* packed,
     else if (n4 <= 256)
         quantize_rows_wave_kernel<4><<<wblocks, 256, 0, s>>>(rows, cols, in, packed, scales);
     else if (n4 <= 512)
-        quantize_rows_reg_kernel<2><<<rows, 256, 0, s>>>(cols, in, packed, scales);
+        quantize_rows_reg_kernel<256, 2><<<rows, 256, 0, s>>>(cols, in, packed, scales);
     else if (n4 <= 768)
-        quantize_rows_reg_kernel<3><<<rows, 256, 0, s>>>(cols, in, packed, scales);
+        quantize_rows_reg_kernel<256, 3><<<rows, 256, 0, s>>>(cols, in, packed, scales);
     else if (n4 <= 1024)
-        quantize_rows_reg_kernel<4><<<rows, 256, 0, s>>>(cols, in, packed, scales);
-    else
+        quantize_rows_reg_kernel<256, 4><<<rows, 256, 0, s>>>(cols, in, packed, scales);
+    else if (n4 <= 4096) {
+        const bool nt = (size_t)rows * cols * sizeof(float) >= kStreamInputBytes;
+        auto* k = n4 <= 2048 ? (nt ? quantize_rows_reg_kernel<512, 4, true> : quantize_rows_reg_kernel<512, 4>)
+                             : (nt ? quantize_rows_reg_kernel<512, 8, true> : quantize_rows_reg_kernel<512, 8>);
+        k<<<rows, 512, 0, s>>>(cols, in, packed, scales);
+    } else
         quantize_rows_kernel<<<rows, 256, 0, s>>>(cols, in, packed, scales);
 }
 

@@ -84,3 +84,17 @@ def test_gemm_any_width(ie, orc, M, K, N, words):
 @pytest.mark.parametrize("epi", [0, 1, 2, 3])
 def test_gemm_any_width_epilogues(ie, orc, epi, M, K, N, words):
     _gemm_case(ie, orc, M, N, K, epi, words, M + K + N + epi)
+
+
+# Rows of more than 4096 columns: 512 threads with the row in registers up to 8192 and 16384 columns (a partial and a
+# full last chunk on both sides of each limit), two passes beyond, and an input past the size that is read
+# non-temporally.
+@pytest.mark.parametrize("rows,cols", [(3, 4100), (2, 8188), (5, 8192), (2, 8196), (3, 16384), (2, 16388), (4100, 8192)])
+def test_quantize_wide_rows(ie, orc, rows, cols):
+    r = rng(rows + cols)
+    x = r.standard_normal((rows, cols)).astype(np.float32)
+    x[0, -4:] = [127.0, -126.5, 0.5, -1.5]  # the row's maximum in its last chunk; ties
+    x[1] = 0.0
+    p, s = (t.cpu().numpy() for t in ie.quantize(_dev(x)))
+    want_p, want_s = orc.quantize(x)
+    assert np.array_equal(s, want_s) and np.array_equal(p, want_p)
