@@ -14,34 +14,64 @@
 //   * contiguous [B, H, N, d] fp32 for Q, K, V, O (the reference's K10
 //     signature, run_flash_attn_v2).
 //
-// MI355X layout (one workgroup of four waves per (query tile, h, b)):
-//   * a workgroup owns 16 consecutive queries of one (b, h); its four waves
-//     take the 16-token KV chunks up to the tile's causal limit round-robin,
-//     each keeping its own running (m, l, o), and merge them in LDS at the end;
-//   * the grid is one-dimensional, tile rank major: workgroup u takes pair
-//     p = u % (H_q B) and tile rank r = u / (H_q B) (rank 0 = the last,
-//     longest tile), so the longest tiles (causal triangles) are dispatched
-//     first.  Workgroups go to the XCDs round-robin, so with H_q B a multiple
-//     of 8 all tiles of one (b, h) run on one XCD (its K/V fetched into one
-//     L2) and every XCD gets the same mix of tile lengths.  (With the tile
-//     index fastest, XCD x took tile rank x of every pair: at 8 tiles XCD 0
-//     held all the longest tiles, and each pair's K/V went to eight L2s);
-//   * S^T = K Q^T and O^T += V^T P^T run on v_mfma_f32_16x16x4_f32.  Lane l
-//     (i = l % 16, g = l / 16) holds, for query i of the tile:
-//       - q: elements d/4*g .. d/4*g + d/4 - 1 (the B operand: MFMA step s
-//         reads element d/4*g + s, and the K operand (A) of key i uses the
-//         same element map, so the K-sum is exact in a permuted order);
-//       - scores of keys 4g .. 4g+3 of the chunk (the MFMA result layout),
-//         which are directly the B operand P^T of the P.V product (step s
-//         takes key 4g + s);
-//       - output elements d/16*(4g + v) + t (t = output tile, v = result row);
-//   * the per-query max and sum run over the four lanes i, i+16, i+32, i+48
-//     (two cross-row swaps), so a wave rescales once per 16 keys;
-//   * scores are pre-multiplied by log2(e)/sqrt(d) (folded into q), so the
-//     softmax uses the hardware exp2 (the decode kernel does the same);
-//   * K/V of the next chunk are loaded while the current one is computed;
-//     with block size 16 a chunk is one block and its physical id comes from a
-//     wave-uniform scalar load.
+// Two families of kernels.
+//
+// prefill_fp32_kernel (fp32 operands): S^T = K Q^T and O^T += V^T P^T on
+// v_mfma_f32_16x16x4_f32, one workgroup per 16 queries, its four waves taking
+// the 16-token chunks round-robin, merged in LDS.  Lane l (i = l % 16, g =
+// l / 16) holds, for query i of the tile, q elements d/4 g .. + d/4 - 1 (MFMA
+// step s takes element d/4 g + s of K and q alike), the scores of keys 4g .. 4g+3
+// of a chunk (the MFMA result layout, which is the B operand P^T of the second
+// product), and output elements d/16 (4g + v) + t.
+//
+// prefill_split_kernel and prefill_tile_kernel: the fp32 matrix rate is a
+// sixteenth of the bf16 one, so here the two products run on
+// v_mfma_f32_16x16x32_bf16 with every fp32 operand written as the sum of three
+// bf16 (each rounded to nearest even, 8 bits apiece, so the sum is the fp32
+// value): six of the nine partial products (those down to 2^-16 of the
+// largest; the rest are below 2^-24 of it) accumulate in fp32.  A bf16 cache is
+// exact in one part and takes three.  Error against 64 bits: about half the
+// fp32 kernel's over d, keys and caches (flash 2048 x 128 1.9e-7 against
+// 3.7e-7, paged bf16 300 x 64 1.1e-7 against 2.2e-7).  Every query sees the same
+// operations in the same order whatever the tile or kernel of the two:
+//   * keys in blocks of 32 from position 0 on, block c in group c % 4; each
+//     group keeps its own running maximum m, sum l and output o (an online
+//     softmax step per block), and the four groups are merged in order at the
+//     end (merge_weights).  Keys past a query's limit have weight exactly 0, so
+//     a block or group without keys changes nothing;
+//   * scores are pre-multiplied by log2(e)/sqrt(d) (folded into q, as in the
+//     fp32 kernel), so the softmax uses the hardware exp2.
+// An operand that is infinite, NaN or rounds to an infinite bf16 has no
+// three-part form and makes NaN: a tile whose outputs are not all finite is
+// computed again with fp32 MFMAs (exact_tile), which gives what the operands'
+// own arithmetic gives.
+//
+// Which family: a paged launch by the cache type alone (bf16: the three-part
+// kernels), so a query's bits never depend on the batch or on how a prompt is
+// chunked; a contiguous one by its shape (prefill_form).
+//
+// In the three-part kernels a wave owns 16 queries of one (b, h).  Operands
+// (lane l: i = l % 16, g = l / 16): S^T = K Q^T, 16 keys x 16 queries per MFMA, leaves lane l with query i and
+// key 4g + v of the tile in result v, so the eight weights of a 32-key block
+// that a lane ends with (keys 4g + v and 16 + 4g + v: octet g) are already the
+// B operand P^T of O^T += V^T P^T, whose A operand V^T takes the same octet.
+//   * prefill_tile_kernel: 64 queries on GW x 4 waves, waves w, w + 4, ...
+//     sharing 16 queries, each four walking 4 / GW of the groups.  They load
+//     their next step's K and V into registers, split them once for the four
+//     and write them to LDS (K rows as they are, V transposed with a row's
+//     keys in octet order, 16-byte chunks XOR-swizzled); two barriers a step.
+//     GW = 1 leaves LDS for several workgroups per CU, which fill each other's
+//     gaps; GW = 2 halves a tile's chain of dependent steps.
+//   * prefill_split_kernel (few or short queries): one workgroup per 16
+//     queries, its four waves the four groups, each loading its blocks
+//     straight into the operand layout (O^T row (t, i) then is element
+//     d/16 i + t, so V loads are 16 bytes per key); the merge goes through LDS.
+// The grid is one-dimensional, tile rank major: workgroup u takes pair p =
+// u % (H_q B) and tile rank r = u / (H_q B) (rank 0 = the last, longest tile),
+// so the longest tiles (causal triangles) are dispatched first and, as
+// workgroups go to the XCDs round-robin, with H_q B a multiple of 8 all tiles
+// of one (b, h) run on one XCD (its K/V fetched into one L2) and every XCD
+// gets the same mix of tile lengths.
 #include <cmath>
 
 #include "device_util.h"
@@ -52,7 +82,12 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kQTile = 16;  // queries per workgroup
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int kQW = 16;     // queries per wave
+constexpr int kKB = 32;     // keys per block
+constexpr int kGroups = 4;  // block c belongs to group c % 4
 constexpr int kWaves = 4;
 
 template <int W>
@@ -87,6 +122,7 @@ __device__ __forceinline__ float elem(const uint32_t (&w)[W], int j) {
     }
 }
 
+// ---- fp32 MFMA form: 16 queries, 16-token chunks.
 // A lane's share of one 16-token chunk: d/4 elements of key i's K, and
 // d/16 elements (from d/16 * i) of each of the keys 4g .. 4g+3's V.
 template <int D, typename KV>
@@ -169,24 +205,26 @@ __device__ __forceinline__ void consume(const Chunk<D, KV>& c, int c0, int g, co
     }
 }
 
+// ---- fp32 MFMA kernel: 16 queries per workgroup, its four waves taking the
+// 16-token chunks round-robin, merged in LDS.
 // LAYOUT 0: Q/O [B, P, H_q, D], keys = start + P cached tokens.
 // LAYOUT 1: Q/K/V/O [B, H, P, D], keys = P, start = 0.
 template <int D, typename KV, int LAYOUT, bool BS16>
-__global__ __launch_bounds__(256) void prefill_attn_kernel(
+__global__ __launch_bounds__(256) void prefill_fp32_kernel(
     const float* __restrict__ Q, const KV* __restrict__ kcache, const KV* __restrict__ vcache,
     const int* __restrict__ block_table, int nbps, int block_size, int P, int H_q, int H_kv,
     int start, int causal, float qscale, float* __restrict__ O) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i = lane & 15, g = lane >> 4;
-    const int ntiles = (P + kQTile - 1) / kQTile;
+    const int ntiles = (P + kQW - 1) / kQW;
     const int pairs = (int)(gridDim.x / (unsigned)ntiles);  // H_q B
     const int r = (int)blockIdx.x / pairs, pr = (int)blockIdx.x - r * pairs;
     const int qt = ntiles - 1 - r;  // longest (last) tiles first
     const int h = pr % H_q, b = pr / H_q;
     const int kvh = h / (H_q / H_kv);
-    const int q0 = qt * kQTile;
-    const int qlast = min(q0 + kQTile - 1, P - 1);
+    const int q0 = qt * kQW;
+    const int qlast = min(q0 + kQW - 1, P - 1);
     const int nkeys = start + P;
     // Keys this tile needs, and this lane's own limit.
     const int kend = causal ? min(start + qlast + 1, nkeys) : nkeys;
@@ -255,8 +293,8 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(
     }
 
     // Merge the four waves' partial softmax states in LDS.
-    __shared__ float sm_o[kWaves][kQTile][D + 4];
-    __shared__ float sm_m[kWaves][kQTile], sm_l[kWaves][kQTile];
+    __shared__ float sm_o[kWaves][kQW][D + 4];
+    __shared__ float sm_m[kWaves][kQW], sm_l[kWaves][kQW];
 #pragma unroll
     for (int t = 0; t < D / 16; ++t)
 #pragma unroll
@@ -267,7 +305,7 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(
     }
     __syncthreads();
 
-    constexpr int PER = kQTile * D / 256;  // outputs per thread (4 or 8)
+    constexpr int PER = kQW * D / 256;  // outputs per thread (4 or 8)
     const int qq = threadIdx.x / 16, col = (threadIdx.x % 16) * PER;
     if (q0 + qq >= P) return;
     float mx = -INFINITY;
@@ -296,27 +334,657 @@ __global__ __launch_bounds__(256) void prefill_attn_kernel(
         *reinterpret_cast<float4*>(orow + col + e) = make_float4(out[e], out[e + 1], out[e + 2], out[e + 3]);
 }
 
+// ---- three-part bf16 form
+// bf16 parts of a pair: x0 in the low half of each word.
+__device__ __forceinline__ uint32_t round_pair(float x0, float x1) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x0, x1}), bf16x2));
+}
+__device__ __forceinline__ void split_pair(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
+    h = round_pair(x0, x1);
+    const float r0 = x0 - __builtin_bit_cast(float, h << 16), r1 = x1 - __builtin_bit_cast(float, h & 0xffff0000u);
+    m = round_pair(r0, r1);
+    l = round_pair(r0 - __builtin_bit_cast(float, m << 16), r1 - __builtin_bit_cast(float, m & 0xffff0000u));
+}
+
+// Eight elements of an MFMA operand, NP parts: 3 for fp32, 1 for bf16.
+template <int NP>
+struct Parts {
+    uint4 p[NP];
+};
+template <typename KV>
+constexpr int kParts = sizeof(KV) == 4 ? 3 : 1;
+
+__device__ __forceinline__ Parts<3> split8(const float (&x)[8]) {
+    Parts<3> r;
+    split_pair(x[0], x[1], r.p[0].x, r.p[1].x, r.p[2].x);
+    split_pair(x[2], x[3], r.p[0].y, r.p[1].y, r.p[2].y);
+    split_pair(x[4], x[5], r.p[0].z, r.p[1].z, r.p[2].z);
+    split_pair(x[6], x[7], r.p[0].w, r.p[1].w, r.p[2].w);
+    return r;
+}
+
+// Elements `odd` (0 or 1) of two words, as one word (one v_perm; of the mask and
+// shift form the compiler read a register it had overwritten).
+__device__ __forceinline__ uint32_t pair_bf16(uint32_t lo, uint32_t hi, int odd) {
+    return __builtin_amdgcn_perm(hi, lo, odd ? 0x07060302u : 0x05040100u);
+}
+// A lane's eight consecutive raw elements as parts.
+template <typename KV, int W>
+__device__ __forceinline__ Parts<kParts<KV>> parts8(const uint32_t (&w)[W]) {
+    if constexpr (sizeof(KV) == 4) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = __builtin_bit_cast(float, w[e]);
+        return split8(x);
+    } else {
+        return Parts<1>{{make_uint4(w[0], w[1], w[2], w[3])}};
+    }
+}
+
+__device__ __forceinline__ f32x4 mfma(uint4 a, uint4 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+
+template <int D>
+struct Group {
+    float m, l;
+    f32x4 o[D / 16];  // o[t][v]: row 4g + v of tile t
+    __device__ __forceinline__ void clear() {
+        m = -INFINITY;
+        l = 0.0f;
+#pragma unroll
+        for (int t = 0; t < D / 16; ++t) o[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+};
+
+// Scores of one block: key(j, s) = the A operand of keys 16 j .. 16 j + 15 at
+// k-step s; sc[4 j + v] is key 16 j + 4 g + v.  Keys at or past klim are masked
+// when `edge` (uniform) says that the block has some.
+template <int D, int NP, typename GetK>
+__device__ __forceinline__ void scores(GetK&& key, const Parts<3> (&q)[D / 32], int c0, int klim, bool edge, int g,
+                                       float (&sc)[8]) {
+    f32x4 big[2], small[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) big[j] = small[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int s = 0; s < D / 32; ++s) {
+        Parts<NP> k[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) k[j] = key(j, s);
+        // small and large products in chains of their own, the two key tiles side by side
+        auto all = [&](f32x4(&acc)[2], int kp, int qp) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[j] = mfma(k[j].p[kp], q[s].p[qp], acc[j]);
+        };
+        if constexpr (NP == 3) {
+            all(small, 2, 0);
+            all(small, 0, 2);
+            all(small, 1, 1);
+            all(small, 1, 0);
+        } else {
+            all(small, 0, 2);
+        }
+        all(small, 0, 1);
+        all(big, 0, 0);
+    }
+#pragma unroll
+    for (int v = 0; v < 8; ++v) sc[v] = big[v >> 2][v & 3] + small[v >> 2][v & 3];
+    if (edge) {
+#pragma unroll
+        for (int v = 0; v < 8; ++v)
+            if (c0 + 16 * (v >> 2) + 4 * g + (v & 3) >= klim) sc[v] = -INFINITY;
+    }
+}
+
+// Online softmax step and P.V of one block: val(t) = the A operand (16 rows
+// of tile t, octet g).
+template <int D, int NP, typename GetV>
+__device__ __forceinline__ void attend(GetV&& val, const float (&sc)[8], Group<D>& gr) {
+    float cm = sc[0];
+#pragma unroll
+    for (int v = 1; v < 8; ++v) cm = fmaxf(cm, sc[v]);
+    cm = max_xor32(max_xor16(cm));
+    const float mn = fmaxf(gr.m, cm);
+    const float mu = mn == -INFINITY ? 0.0f : mn;  // no key yet: keep o, l at 0
+    const float alpha = exp2_sm(gr.m - mu);
+    float p[8], ls = 0.0f;
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+        p[v] = exp2_sm(sc[v] - mu);
+        ls += p[v];
+    }
+    ls = sum_xor32(sum_xor16(ls));
+    gr.l = fmaf(gr.l, alpha, ls);
+    gr.m = mn;
+    if (__ballot(alpha != 1.0f)) {  // (a factor of 1 changes nothing)
+#pragma unroll
+        for (int t = 0; t < D / 16; ++t) gr.o[t] *= alpha;
+    }
+    const Parts<3> pp = split8(p);
+    // four tiles side by side, so that an accumulator's MFMAs are not back to back
+#pragma unroll
+    for (int t0 = 0; t0 < D / 16; t0 += 4) {
+        Parts<NP> x[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[k] = val(t0 + k);
+        auto all = [&](int vp, int wp) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) gr.o[t0 + k] = mfma(x[k].p[vp], pp.p[wp], gr.o[t0 + k]);
+        };
+        if constexpr (NP == 3) {
+            all(2, 0);
+            all(0, 2);
+            all(1, 1);
+            all(1, 0);
+        } else {
+            all(0, 2);
+        }
+        all(0, 1);
+        all(0, 0);
+    }
+}
+
+// Weights of the running total (M) and of the next group (m); the total is
+// scaled by a and the group added with b.
+__device__ __forceinline__ float merge_weights(float M, float m, float& a, float& b) {
+    const float mn = fmaxf(M, m);
+    a = M == -INFINITY ? 0.0f : exp2_sm(M - mn);
+    b = m == -INFINITY ? 0.0f : exp2_sm(m - mn);
+    return mn;
+}
+__device__ __forceinline__ float merge_value(float X, float x, float a, float b) { return fmaf(X, a, x * b); }
+
+// Where a tile's queries, keys and outputs are.
+template <int D, typename KV, int LAYOUT, bool BS16>
+struct Where {
+    TokenMap<LAYOUT, BS16> map{};
+    const KV *kbase, *vbase;
+    const float* Q;
+    float* O;
+    int P, H_q, h, b, start, causal, nkeys;
+
+    __device__ __forceinline__ size_t qrow(int qi) const {
+        return LAYOUT == 0 ? (((size_t)b * P + qi) * H_q + h) * D : (((size_t)b * H_q + h) * P + qi) * D;
+    }
+    // keys that queries up to qi need
+    __device__ __forceinline__ int limit(int qi) const { return causal ? min(start + qi + 1, nkeys) : nkeys; }
+    __device__ __forceinline__ int phys(int pos, int kend) const {
+        if constexpr (LAYOUT == 0 && BS16) return map.bt[min(pos, kend - 1) >> 4];
+        else return 0;
+    }
+};
+
+template <int D, typename KV, int LAYOUT, bool BS16>
+__device__ __forceinline__ Where<D, KV, LAYOUT, BS16> locate(const float* Q, const KV* kcache, const KV* vcache,
+                                                             const int* block_table, int nbps, int block_size, int P,
+                                                             int H_q, int H_kv, int start, int causal, float* O, int h,
+                                                             int b) {
+    Where<D, KV, LAYOUT, BS16> w;
+    const int kvh = h / (H_q / H_kv);
+    if constexpr (LAYOUT == 0) {
+        w.map.bt = block_table + (size_t)b * nbps;
+        w.map.block_size = block_size;
+        w.map.stride = (size_t)H_kv * D;
+        w.kbase = kcache + (size_t)kvh * D;
+        w.vbase = vcache + (size_t)kvh * D;
+    } else {
+        w.map.stride = D;
+        w.kbase = kcache + ((size_t)b * H_kv + kvh) * P * D;
+        w.vbase = vcache + ((size_t)b * H_kv + kvh) * P * D;
+    }
+    w.Q = Q;
+    w.O = O;
+    w.P = P;
+    w.H_q = H_q;
+    w.h = h;
+    w.b = b;
+    w.start = start;
+    w.causal = causal;
+    w.nkeys = start + P;
+    return w;
+}
+
+// 16 queries from q0 on with fp32 MFMAs, one wave over all their keys: the
+// form for operands that have no three-part one.
+template <int D, typename KV, int LAYOUT, bool BS16>
+__device__ __forceinline__ void exact_tile(const Where<D, KV, LAYOUT, BS16>& w, int q0, float qscale) {
+    if (q0 >= w.P) return;
+    const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+    const int qi = min(q0 + i, w.P - 1);
+    const int kend = w.limit(min(q0 + 15, w.P - 1)), klim = w.limit(qi);
+    float q[D / 4];
+#pragma unroll
+    for (int e = 0; e < D / 4; e += 4) {
+        const float4 v = *reinterpret_cast<const float4*>(w.Q + w.qrow(qi) + (D / 4) * g + e);
+        q[e] = v.x * qscale;
+        q[e + 1] = v.y * qscale;
+        q[e + 2] = v.z * qscale;
+        q[e + 3] = v.w * qscale;
+    }
+    float m = -INFINITY, l = 0.0f;
+    f32x4 o[D / 16];
+#pragma unroll
+    for (int t = 0; t < D / 16; ++t) o[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+    for (int c0 = 0; c0 < kend; c0 += 16) {
+        Chunk<D, KV> c;
+        load_chunk(c, c0, kend, i, g, w.phys(c0, kend), w.map, w.kbase, w.vbase);
+        consume(c, c0, g, q, klim, m, l, o);
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    if (q0 + i < w.P) {
+        float* out = w.O + w.qrow(qi);
+#pragma unroll
+        for (int t = 0; t < D / 16; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) out[(D / 16) * (4 * g + v) + t] = o[t][v] * inv;
+    }
+}
+
+template <int D>
+__device__ __forceinline__ void load_query(const float* row, float qscale, int g, Parts<3> (&q)[D / 32]) {
+#pragma unroll
+    for (int s = 0; s < D / 32; ++s) {
+        const float4 a = *reinterpret_cast<const float4*>(row + 32 * s + 8 * g);
+        const float4 b = *reinterpret_cast<const float4*>(row + 32 * s + 8 * g + 4);
+        const float x[8] = {a.x * qscale, a.y * qscale, a.z * qscale, a.w * qscale,
+                            b.x * qscale, b.y * qscale, b.z * qscale, b.w * qscale};
+        q[s] = split8(x);
+    }
+}
+
+// Rows of a block's keys for a lane.  With 16-token pages and contiguous rows
+// key r of half j of a block at c0 lies at a uniform base (of the page, or of
+// the half) plus r rows, so an address is a scalar base plus a 32-bit lane
+// offset; other block sizes look each key up.  Keys at or past kend read the
+// last one.
+template <typename KV, int LAYOUT, bool BS16>
+struct BlockRows {
+    const TokenMap<LAYOUT, BS16>& map;
+    const KV* base;  // the head's rows
+    const KV *half0, *half1;
+    int c0, kend;
+    __device__ __forceinline__ BlockRows(const TokenMap<LAYOUT, BS16>& m, const KV* b, int c0_, int kend_)
+        : map(m), base(b), c0(c0_), kend(kend_) {
+        half0 = start_of(c0);
+        half1 = start_of(min(c0 + 16, (kend - 1) & ~15));  // (past the end: its keys read the first half's last)
+    }
+    __device__ __forceinline__ const KV* start_of(int pos) const {
+        if constexpr (LAYOUT == 1) return base + (size_t)pos * map.stride;
+        else if constexpr (BS16) return base + (size_t)map.bt[pos >> 4] * 16 * map.stride;
+        else return base;
+    }
+    // elements `elem` on of key 16 j + r (r < 16); j uniform
+    __device__ __forceinline__ const KV* at(int j, int r, int elem) const {
+        if constexpr (LAYOUT == 0 && !BS16) {
+            return base + map.off(min(c0 + 16 * j + r, kend - 1), 0) + elem;
+        } else {
+            const int pos = min(c0 + 16 * j, (kend - 1) & ~15);
+            // (16 rows of at most 65535 heads: below 2^32 bytes)
+            const uint32_t ofs = ((uint32_t)min(r, kend - 1 - pos) * (uint32_t)map.stride + elem) * (uint32_t)sizeof(KV);
+            return reinterpret_cast<const KV*>(reinterpret_cast<const char*>(j ? half1 : half0) + ofs);
+        }
+    }
+};
+
+// LAYOUT 0: Q/O [B, P, H_q, D], keys = start + P cached tokens.
+// LAYOUT 1: Q/K/V/O [B, H, P, D], keys = P, start = 0.
+template <int D, typename KV, int LAYOUT, bool BS16, int GW>
+__global__ __launch_bounds__(256 * GW, D == 64 && GW == 1 ? 3 : 2) void prefill_tile_kernel(
+    const float* __restrict__ Q, const KV* __restrict__ kcache, const KV* __restrict__ vcache,
+    const int* __restrict__ block_table, int nbps, int block_size, int P, int H_q, int H_kv,
+    int start, int causal, float qscale, float* __restrict__ O) {
+    constexpr int NP = kParts<KV>, QT = kWaves * kQW, T = 256;
+    constexpr int CK = D / 8;                   // 16-byte chunks of a K row
+    constexpr int KBYTES = kKB * D * 2;         // one part of a block's K (or V)
+    constexpr int HBYTES = 2 * NP * KBYTES;     // K and V of a block
+    constexpr int KT = kKB * CK / T;            // K chunks per thread
+    constexpr int VE = 8 * D / T;               // V: elements per thread, of four keys
+    constexpr int KW = 4 * (int)sizeof(KV) / 2, VW = VE * (int)sizeof(KV) / 4;  // raw words
+    constexpr int TT = D / 16;
+    // (the merge passes two states per lane of four waves through it)
+    constexpr int MBYTES = GW == 1 ? 0 : 2 * kWaves * 64 * (TT * 16 + 8), PER = kGroups / GW;
+    __shared__ __attribute__((aligned(16))) int8_t lds_all[GW * HBYTES > MBYTES ? GW * HBYTES : MBYTES];
+    const int lane = threadIdx.x & 63, g = lane >> 4, i = lane & 15;
+    const int wave8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int hf = GW == 1 ? 0 : wave8 >> 2, wave = wave8 & 3, tid = threadIdx.x & (T - 1);
+    int8_t* lds = lds_all + hf * HBYTES;
+    const int ntiles = (P + QT - 1) / QT;
+    const int pairs = (int)(gridDim.x / (unsigned)ntiles);  // H_q B
+    const int r = (int)blockIdx.x / pairs, pr = (int)blockIdx.x - r * pairs;
+    const int q0 = (ntiles - 1 - r) * QT;  // longest (last) tiles first
+    const auto w = locate<D, KV, LAYOUT, BS16>(Q, kcache, vcache, block_table, nbps, block_size, P, H_q, H_kv, start,
+                                               causal, O, pr % H_q, pr / H_q);
+    const int kend = w.limit(min(q0 + QT - 1, P - 1));
+    const int nblk = (kend + kKB - 1) / kKB;
+    const int qw = q0 + wave * kQW, qi = min(qw + i, P - 1);
+    const int klim = w.limit(qi);
+    const int wlo = w.limit(min(qw, P - 1)), whi = qw < P ? w.limit(min(qw + kQW - 1, P - 1)) : 0;  // uniform
+
+    // The thread's raw share of a block, and its way into LDS: K chunks of
+    // eight elements; V, VE elements of keys 16 vj + 4 vo .. + 3 (half vj of
+    // octet vo).
+    uint32_t kr[KT][KW], vr[4][VW];
+    const int vj = wave & 1, vo = 2 * (wave >> 1) + (lane >> 5), ve = (lane & 31) * VE;
+    auto load = [&](int blk) {
+        const int c0 = blk * kKB;
+        const BlockRows<KV, LAYOUT, BS16> kb(w.map, w.kbase, c0, kend), vb(w.map, w.vbase, c0, kend);
+#pragma unroll
+        for (int j = 0; j < KT; ++j) {
+            const int id = tid + T * j, key = id / CK, c = id % CK;
+            load_words(kb.at(__builtin_amdgcn_readfirstlane(key >> 4), key & 15, 8 * c), kr[j]);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) load_words(vb.at(vj, 4 * vo + e, ve), vr[e]);
+    };
+    auto k_at = [&](int part, int key, int c) {
+        return reinterpret_cast<uint4*>(lds + part * KBYTES + key * (2 * D) +
+                                        ((c ^ (D == 128 ? key & 15 : (key >> 1) & 7)) << 4));
+    };
+    auto v_at = [&](int part, int e, int c) {
+        return lds + (NP + part) * KBYTES + e * (2 * kKB) + ((c ^ ((e >> 2) & 3)) << 4);
+    };
+    auto store = [&] {
+#pragma unroll
+        for (int j = 0; j < KT; ++j) {
+            const int id = tid + T * j, key = id / CK, c = id % CK;
+            const Parts<NP> s = parts8<KV>(kr[j]);
+#pragma unroll
+            for (int p = 0; p < NP; ++p) *k_at(p, key, c) = s.p[p];
+        }
+#pragma unroll
+        for (int d = 0; d < VE; ++d) {
+            uint2 s[NP];
+            if constexpr (NP == 3) {
+                split_pair(elem<KV>(vr[0], d), elem<KV>(vr[1], d), s[0].x, s[1].x, s[2].x);
+                split_pair(elem<KV>(vr[2], d), elem<KV>(vr[3], d), s[0].y, s[1].y, s[2].y);
+            } else {
+                s[0] = make_uint2(pair_bf16(vr[0][d / 2], vr[1][d / 2], d & 1), pair_bf16(vr[2][d / 2], vr[3][d / 2], d & 1));
+            }
+#pragma unroll
+            for (int p = 0; p < NP; ++p) *reinterpret_cast<uint2*>(v_at(p, ve + d, vo) + 8 * vj) = s[p];
+        }
+    };
+
+    // These four waves' steps: groups PER hf .. PER hf + PER - 1, a block at a time.
+    int grp = PER * hf, blk = grp;
+    bool act = blk < nblk;
+    if (act) load(blk);
+    auto steps = [&](int k) { return k < nblk ? (nblk - k + kGroups - 1) / kGroups : 0; };
+    int iters = 0;  // (the second half has no more than the first)
+#pragma unroll
+    for (int k = 0; k < PER; ++k) iters += steps(k);
+    Parts<3> q[D / 32];
+    load_query<D>(Q + w.qrow(qi), qscale, g, q);
+    Group<D> gr, tot;
+    gr.clear();
+    tot.clear();
+    auto merge = [&](const Group<D>& x) {
+        float a, b;
+        tot.m = merge_weights(tot.m, x.m, a, b);
+        tot.l = merge_value(tot.l, x.l, a, b);
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) tot.o[t][v] = merge_value(tot.o[t][v], x.o[t][v], a, b);
+    };
+#pragma unroll 1
+    for (int it = 0; it < iters; ++it) {
+        const int c0 = blk * kKB, cg = grp;
+        const bool cact = act, gend = blk + kGroups >= nblk;
+        __syncthreads();  // the last block has been read
+        if (cact) store();
+        __syncthreads();
+        blk = gend ? ++grp : blk + kGroups;
+        act = act && grp < PER * hf + PER && blk < nblk;
+        if (act) load(blk);
+        if (!cact) continue;
+        if (c0 < whi) {
+            float sc[8];
+            scores<D, NP>(
+                [&](int j, int s) {
+                    Parts<NP> x;
+#pragma unroll
+                    for (int p = 0; p < NP; ++p) x.p[p] = *k_at(p, 16 * j + i, 4 * s + g);
+                    return x;
+                },
+                q, c0, klim, c0 + kKB > wlo, g, sc);
+            attend<D, NP>(
+                [&](int t) {
+                    Parts<NP> x;
+#pragma unroll
+                    for (int p = 0; p < NP; ++p) x.p[p] = *reinterpret_cast<uint4*>(v_at(p, 16 * t + i, g));
+                    return x;
+                },
+                sc, gr);
+        }
+        // into the total in order; of GW = 2's second half, group 2 into its
+        // own (empty, so it is kept as it is) and 3 stays in gr
+        if (gend && (GW == 1 || cg < 3)) {
+            merge(gr);
+            gr.clear();
+        }
+    }
+    if constexpr (GW == 2) {
+    // Groups 2 and 3 from the second half, in order.
+    __syncthreads();
+    float4* mo = reinterpret_cast<float4*>(lds_all);
+    float2* ml = reinterpret_cast<float2*>(lds_all + 2 * kWaves * 64 * TT * 16);
+    auto slot = [&](int k) { return (k * kWaves + wave) * 64 + lane; };
+    if (hf == 1) {
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+            mo[t * (2 * kWaves * 64) + slot(0)] = make_float4(tot.o[t][0], tot.o[t][1], tot.o[t][2], tot.o[t][3]);
+            mo[t * (2 * kWaves * 64) + slot(1)] = make_float4(gr.o[t][0], gr.o[t][1], gr.o[t][2], gr.o[t][3]);
+        }
+        ml[slot(0)] = make_float2(tot.m, tot.l);
+        ml[slot(1)] = make_float2(gr.m, gr.l);
+    }
+    __syncthreads();
+    if (hf == 1) return;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const float2 x = ml[slot(k)];
+        gr.m = x.x;
+        gr.l = x.y;
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+            const float4 y = mo[t * (2 * kWaves * 64) + slot(k)];
+            gr.o[t] = f32x4{y.x, y.y, y.z, y.w};
+        }
+        merge(gr);
+    }
+    }
+
+    const float inv = tot.l > 0.0f ? 1.0f / tot.l : 0.0f;
+    float bad = 0.0f;
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            tot.o[t][v] *= inv;
+            bad = fmaf(tot.o[t][v], 0.0f, bad);
+        }
+    if (__ballot(!(bad == 0.0f))) {  // uniform: not all finite
+        exact_tile(w, qw, qscale);
+    } else if (qw + i < P) {
+        float* out = O + w.qrow(qi) + 4 * g;
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+            *reinterpret_cast<float4*>(out + 16 * t) = make_float4(tot.o[t][0], tot.o[t][1], tot.o[t][2], tot.o[t][3]);
+    }
+}
+
+template <int D, typename KV, int LAYOUT, bool BS16>
+__global__ __launch_bounds__(256, D == 64 ? 2 : 1) void prefill_split_kernel(
+    const float* __restrict__ Q, const KV* __restrict__ kcache, const KV* __restrict__ vcache,
+    const int* __restrict__ block_table, int nbps, int block_size, int P, int H_q, int H_kv,
+    int start, int causal, float qscale, float* __restrict__ O) {
+    constexpr int NP = kParts<KV>;
+    constexpr int KW = 4 * (int)sizeof(KV) / 2;       // raw words of eight elements
+    constexpr int VW = D / 16 * (int)sizeof(KV) / 4;  // of d / 16
+    __shared__ float sm_o[kGroups][kQW][D + 4];
+    __shared__ float sm_m[kGroups][kQW], sm_l[kGroups][kQW];
+    const int lane = threadIdx.x & 63, g = lane >> 4, i = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // its group
+    const int ntiles = (P + kQW - 1) / kQW;
+    const int pairs = (int)(gridDim.x / (unsigned)ntiles);  // H_q B
+    const int r = (int)blockIdx.x / pairs, pr = (int)blockIdx.x - r * pairs;
+    const int q0 = (ntiles - 1 - r) * kQW;  // longest (last) tiles first
+    const auto w = locate<D, KV, LAYOUT, BS16>(Q, kcache, vcache, block_table, nbps, block_size, P, H_q, H_kv, start,
+                                               causal, O, pr % H_q, pr / H_q);
+    const int kend = w.limit(min(q0 + kQW - 1, P - 1));
+    const int qi = min(q0 + i, P - 1);
+    const int klim = w.limit(qi), wlo = w.limit(q0);
+
+    // K: elements 32 s + 8 g .. of key 16 j + i; V: elements d/16 i .. of the
+    // keys of octet g.
+    uint32_t kr[2][D / 32][KW], vr[8][VW];
+    auto load_k = [&](int c0) {
+        const BlockRows<KV, LAYOUT, BS16> kb(w.map, w.kbase, c0, kend);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int s = 0; s < D / 32; ++s) load_words(kb.at(j, i, 32 * s + 8 * g), kr[j][s]);
+    };
+    auto load_v = [&](int c0) {
+        const BlockRows<KV, LAYOUT, BS16> vb(w.map, w.vbase, c0, kend);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) load_words(vb.at(e >> 2, 4 * g + (e & 3), D / 16 * i), vr[e]);
+    };
+
+    Group<D> gr;
+    gr.clear();
+    int c0 = wave * kKB;
+    if (c0 < kend) {
+        load_k(c0);
+        load_v(c0);
+    }
+    Parts<3> q[D / 32];
+    load_query<D>(Q + w.qrow(qi), qscale, g, q);
+    while (c0 < kend) {
+        const int cn = c0 + kGroups * kKB;
+        float sc[8];
+        scores<D, NP>([&](int j, int s) { return parts8<KV>(kr[j][s]); }, q, c0, klim, c0 + kKB > wlo, g, sc);
+        if (cn < kend) load_k(cn);
+        attend<D, NP>(
+            [&](int t) {
+                if constexpr (NP == 3) {
+                    const float x[8] = {elem<KV>(vr[0], t), elem<KV>(vr[1], t), elem<KV>(vr[2], t), elem<KV>(vr[3], t),
+                                        elem<KV>(vr[4], t), elem<KV>(vr[5], t), elem<KV>(vr[6], t), elem<KV>(vr[7], t)};
+                    return split8(x);
+                } else {
+                    auto pair = [&](int e) { return pair_bf16(vr[e][t / 2], vr[e + 1][t / 2], t & 1); };
+                    return Parts<1>{{make_uint4(pair(0), pair(2), pair(4), pair(6))}};
+                }
+            },
+            sc, gr);
+        if (cn < kend) load_v(cn);
+        c0 = cn;
+    }
+
+#pragma unroll
+    for (int t = 0; t < D / 16; ++t)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) sm_o[wave][i][(D / 16) * (4 * g + v) + t] = gr.o[t][v];
+    if (g == 0) {
+        sm_m[wave][i] = gr.m;
+        sm_l[wave][i] = gr.l;
+    }
+    __syncthreads();
+
+    constexpr int PER = kQW * D / 256;  // outputs per thread (4 or 8)
+    const int qq = threadIdx.x / 16, col = (threadIdx.x % 16) * PER;
+    float M = -INFINITY, L = 0.0f, x[PER];
+#pragma unroll
+    for (int e = 0; e < PER; ++e) x[e] = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kGroups; ++k) {
+        float a, b;
+        M = merge_weights(M, sm_m[k][qq], a, b);
+        L = merge_value(L, sm_l[k][qq], a, b);
+#pragma unroll
+        for (int e = 0; e < PER; ++e) x[e] = merge_value(x[e], sm_o[k][qq][col + e], a, b);
+    }
+    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    float bad = 0.0f;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+        x[e] *= inv;
+        bad = fmaf(x[e], 0.0f, bad);
+    }
+    if (__syncthreads_or(!(bad == 0.0f))) {
+        if (wave == 0) exact_tile(w, q0, qscale);
+        return;
+    }
+    if (q0 + qq < P) {
+        float* out = O + w.qrow(q0 + qq) + col;
+#pragma unroll
+        for (int e = 0; e < PER; e += 4) *reinterpret_cast<float4*>(out + e) = make_float4(x[e], x[e + 1], x[e + 2], x[e + 3]);
+    }
+}
+
+enum PrefillForm { kFp32, kSplit, kTile1, kTile2 };
+
+// Measured on one box (us, graph-timed; W = 64-query tiles of the launch).
+// Paged bf16: few tiles take the split kernel (d 64: 1 x 256 x 8 heads 7.35 on
+// the fp32 MFMAs, 5.75 here; 1 x 1024 x 8 23.5 -> 13.6; d 128: 41.2 -> 20.9), from
+// 320 on the tile kernel, one workgroup of waves over short contexts (d 128, 16 x
+// 128 x 12: split 20.4, GW = 1 13.9, GW = 2 21.5; fp32 MFMAs 24.7) and two over
+// longer ones until there are tiles for several workgroups per CU (d 64, 4 x 512 x
+// 12: 18.7 / 20.5 / 17.5).
+// Contiguous fp32: the tile kernels where they have the tiles (d 128: 4 x 512 x 32
+// heads 146 -> 76 on GW = 1, 1 x 2048 x 16 210 -> 126 on GW = 2, 161 on GW = 1; d
+// 64: 4 x 256 x 32 23.9 -> 19.1, 1 x 2048 x 16 97 -> 78), the split kernel for a
+// few long ones (d 128, 1 x 1024 x 4 33.2 -> 29.7), the fp32 kernel for the rest,
+// whose launches are over before the splitting pays (d 64, 2 x 512 x 12: 17.8
+// against 19.5 split, 22.3 GW = 2).
+PrefillForm prefill_form(const PrefillArgs& a) {
+    const long long tiles = (long long)((a.P + kWaves * kQW - 1) / (kWaves * kQW)) * a.H_q * a.B;
+    const int keys = a.start_pos + a.P;
+    if (a.paged) {
+        if (a.kv_dtype != IE_KV_BF16) return kFp32;
+        if (tiles < 320) return kSplit;
+        return tiles >= 1024 || keys <= 256 ? kTile1 : kTile2;
+    }
+    if (tiles >= (keys <= 768 ? 512 : 1024)) return kTile1;
+    if (keys >= 768) return tiles >= 256 ? kTile2 : tiles <= 128 ? kSplit : kFp32;
+    return a.d == 128 && keys >= 384 && tiles <= 64 ? kSplit : kFp32;
+}
+
 template <int D, typename KV, int LAYOUT, bool BS16>
 void launch_t(const PrefillArgs& a, hipStream_t s) {
-    const dim3 grid((unsigned)((a.P + kQTile - 1) / kQTile * a.H_q * a.B));
     const float qscale = 1.4426950408889634f / sqrtf((float)D);
-    prefill_attn_kernel<D, KV, LAYOUT, BS16><<<grid, 256, 0, s>>>(
-        a.Q, static_cast<const KV*>(a.k), static_cast<const KV*>(a.v), a.block_table,
-        a.num_blocks_per_seq, a.block_size, a.P, a.H_q, a.H_kv, a.start_pos, a.causal ? 1 : 0, qscale,
-        a.O);
+    const PrefillForm form = prefill_form(a);
+    const int per = form == kTile1 || form == kTile2 ? kWaves * kQW : kQW;  // queries per workgroup
+    const unsigned grid = (unsigned)((long long)((a.P + per - 1) / per) * a.H_q * a.B);
+    auto* k = prefill_split_kernel<D, KV, LAYOUT, BS16>;
+    if (form == kTile1) k = prefill_tile_kernel<D, KV, LAYOUT, BS16, 1>;
+    if (form == kTile2) k = prefill_tile_kernel<D, KV, LAYOUT, BS16, 2>;
+    k<<<grid, form == kTile2 ? 512 : 256, 0, s>>>(a.Q, static_cast<const KV*>(a.k), static_cast<const KV*>(a.v),
+                                                 a.block_table, a.num_blocks_per_seq, a.block_size, a.P, a.H_q, a.H_kv,
+                                                 a.start_pos, a.causal ? 1 : 0, qscale, a.O);
+}
+
+template <int D, int LAYOUT, bool BS16>
+void launch_fp32(const PrefillArgs& a, hipStream_t s) {
+    const float qscale = 1.4426950408889634f / sqrtf((float)D);
+    const unsigned grid = (unsigned)((long long)((a.P + kQW - 1) / kQW) * a.H_q * a.B);
+    prefill_fp32_kernel<D, float, LAYOUT, BS16><<<grid, 256, 0, s>>>(
+        a.Q, static_cast<const float*>(a.k), static_cast<const float*>(a.v), a.block_table, a.num_blocks_per_seq,
+        a.block_size, a.P, a.H_q, a.H_kv, a.start_pos, a.causal ? 1 : 0, qscale, a.O);
 }
 
 template <int D>
 void launch_d(const PrefillArgs& a, hipStream_t s) {
-    if (a.paged) {
-        const bool bs16 = a.block_size == 16;
-        if (a.kv_dtype == IE_KV_BF16)
-            bs16 ? launch_t<D, uint16_t, 0, true>(a, s) : launch_t<D, uint16_t, 0, false>(a, s);
-        else
-            bs16 ? launch_t<D, float, 0, true>(a, s) : launch_t<D, float, 0, false>(a, s);
-    } else {
-        launch_t<D, float, 1, false>(a, s);
-    }
+    const bool fp32 = prefill_form(a) == kFp32, bs16 = a.block_size == 16;
+    if (!a.paged)
+        fp32 ? launch_fp32<D, 1, false>(a, s) : launch_t<D, float, 1, false>(a, s);
+    else if (fp32)
+        bs16 ? launch_fp32<D, 0, true>(a, s) : launch_fp32<D, 0, false>(a, s);
+    else
+        bs16 ? launch_t<D, uint16_t, 0, true>(a, s) : launch_t<D, uint16_t, 0, false>(a, s);
 }
 
 }  // namespace

@@ -1,0 +1,114 @@
+"""The prompt attention's kernels for bf16 caches and for long or many contiguous
+problems (three-part bf16 products), through the public entry points: every
+form the launch rule can take, its ends of tiles, blocks and groups, the
+promise that a query's bits do not depend on the form, and operands that have
+no three-part form.  Reference and bar as test_gpu_prefill_attn.py's."""
+import numpy as np
+import pytest
+
+from conftest import rng
+from test_gpu_prefill_attn import REL, case, dev, host, oracle_prefill, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+# Paged bf16.  Fewer than 320 tiles of 64 queries: the split kernel (one key, one to five 32-key blocks, a context that
+# ends in a block's second page, other block sizes); 320 and more: the tile kernel, one set of waves up to 256 keys
+# and from 1024 tiles on, two between (a partial last tile, groups of unequal length).
+@pytest.mark.parametrize("B,P,start,H_kv,G,d,bs", [
+    (1, 1, 0, 1, 1, 64, 16), (2, 33, 0, 2, 1, 64, 16), (1, 17, 126, 2, 4, 128, 16), (2, 50, 300, 2, 2, 64, 16),
+    (1, 40, 57, 2, 1, 128, 8), (1, 70, 13, 2, 2, 64, 48),
+    (4, 100, 11, 20, 2, 64, 16), (2, 130, 0, 27, 2, 128, 16), (4, 65, 100, 20, 2, 128, 48),
+    (2, 129, 190, 27, 2, 64, 16), (2, 150, 200, 27, 2, 128, 16), (2, 150, 140, 27, 2, 64, 8),
+    (8, 65, 330, 64, 1, 64, 16)])
+def test_paged_bf16_forms(ie, orc, B, P, start, H_kv, G, d, bs):
+    Q, kc, vc, table = case(P + start + H_kv + d, B, P, start, H_kv, G, d, bs, 1)
+    want = oracle_prefill(orc, Q, kc, vc, table, start, bs, H_kv, 1)
+    got = host(ie.prefill_attn(dev(Q), dev(kc), dev(vc), dev(table), start, bs, H_kv, kv_dtype=ie.KV_BF16))
+    assert rel_err(got, want) < REL
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("P,B", [(200, 4), (300, 4), (130, 12)])
+def test_paged_bf16_bits_do_not_depend_on_the_form(ie, d, P, B):
+    """B prompts at once (the tile kernel: 20 heads x 4 x 4 tiles of at most
+    256 keys, x 5 of more, or x 3 x 12) against one prompt in chunks of 37 and
+    of 1 (the split kernel)."""
+    Q, kc, vc, table = case(7 * P + d, B, P, 0, 20, 1, d, 16, 1)
+    whole = host(ie.prefill_attn(dev(Q), dev(kc), dev(vc), dev(table), 0, 16, 20, kv_dtype=ie.KV_BF16))
+    kd, vd, td = dev(kc), dev(vc), dev(table[1:2])
+    for t0, t1 in ((0, 37), (37, 74), (P - 40, P - 3), (P - 1, P)):
+        part = host(ie.prefill_attn(dev(Q[1:2, t0:t1]), kd, vd, td, t0, 16, 20, kv_dtype=ie.KV_BF16))
+        assert np.array_equal(part[0], whole[1, t0:t1])
+
+
+# Contiguous fp32: few long problems on the split kernel, the tile kernel with two sets of waves (256 tiles of 768 keys
+# and more) and with one (512 tiles, 1024 of long ones).
+@pytest.mark.parametrize("B,H,N,d,causal", [(1, 2, 769, 64, True), (1, 2, 801, 128, False), (1, 4, 385, 128, True),
+                                            (1, 24, 780, 64, True), (2, 10, 800, 128, False), (2, 64, 250, 64, True),
+                                            (4, 32, 200, 128, False), (8, 32, 97, 64, False), (2, 40, 801, 64, True)])
+def test_flash_forms(ie, orc, B, H, N, d, causal):
+    r = rng(N + H + d)
+    Q, K, V = (r.standard_normal((B, H, N, d)).astype(np.float32) for _ in range(3))
+    kc, vc, Qt = (np.ascontiguousarray(x.transpose(0, 2, 1, 3)) for x in (K, V, Q))
+    table = np.arange(B, dtype=np.int32).reshape(B, 1)
+    got = host(ie.flash_attn(dev(Q), dev(K), dev(V), causal=causal)).transpose(0, 2, 1, 3)
+    # every head of a few query positions (all keys' block and group ends among them)
+    for t in sorted({0, 15, 16, 31, 32, 63, 64, 95, N // 2, N - 2, N - 1}):
+        n = t + 1 if causal else N
+        want = orc.decode_attn(np.ascontiguousarray(Qt[:, t]), kc, vc, table, np.full(B, n, np.int32), n, N, H)
+        assert rel_err(got[:, t], want) < REL
+
+
+# A K entry of -inf gives its key a weight of 0 for the queries whose element there is positive; a V entry of inf makes
+# that output element inf for the queries that see its key and leaves the others' finite; values that round to an
+# infinite bf16 stay what they are.
+@pytest.mark.parametrize("shape", ["split", "tile1", "tile2"])
+@pytest.mark.parametrize("d", [64, 128])
+def test_flash_operands_without_three_parts(ie, d, shape):
+    import torch
+
+    B, H, N = {"split": (1, 1, 800), "tile1": (2, 64, 250), "tile2": (1, 24, 780)}[shape]
+    g = torch.Generator().manual_seed(d + N)
+    Q, K, V = (torch.randn(B, H, N, d, generator=g) for _ in range(3))
+    Q[..., 3] = Q[..., 3].abs() + 0.1
+    K[0, 0, 70, 3] = -float("inf")       # never attended to by head 0
+    V[0, 0, 150, 5] = float("inf")
+    V[0, 0, 40, 7] = 3.4e38              # bf16 rounds it to inf; its weight keeps the output finite
+    K[0, 0, 90, 9] = -3.4e38
+    Q[0, 0, :, 9] = 1e-37                # a score of -3.4 / sqrt(d) from that element
+    got = ie.flash_attn(Q.cuda(), K.cuda(), V.cuda(), causal=True).cpu().double()
+    q, k, v = (x[0, 0].double() for x in (Q, K, V))
+    s = (q @ k.t()) / d**0.5
+    w = torch.softmax(s.masked_fill(~torch.ones(N, N, dtype=torch.bool).tril(), -float("inf")), dim=1)
+    # weight 0 times an infinity is no part of the sum
+    want = torch.where(w[:, :, None] == 0, torch.zeros(()), w[:, :, None] * v[None]).sum(1)
+    # fp32 MFMAs take 16 queries and their keys together: the queries of the infinite value's own tile that
+    # do not see its key get 0 x inf
+    rows = torch.ones(N, dtype=torch.bool)
+    rows[144:150] = False
+    o = got[0, 0]
+    assert torch.equal(o[rows].isinf(), want[rows].isinf()) and not o[rows].isnan().any()
+    finite = rows & ~want.isinf().any(1)
+    scale = want[finite].abs().amax(0)
+    assert ((o[finite] - want[finite]).abs().amax(0) <= REL * scale).all()
+    # untouched heads are as they are
+    assert got[0, 1 % H][200:].isfinite().all() or H == 1
+
+
+def test_paged_bf16_infinite_value(ie):
+    """An infinity in a bf16 cache (exact in one part, but the weights' parts
+    have signs of their own): inf where its key is seen, finite elsewhere."""
+    B, P, H, d = 1, 100, 2, 64
+    Q, kc, vc, table = case(5, B, P, 0, H, 1, d, 16, 1)
+    page, slot = int(table[0, 3]), 5  # position 53
+    vc = vc.copy()
+    vc[page, slot, 0, 8] = 0x7F80
+    kc = kc.copy()
+    kc[page, slot + 2, 1, 4] = 0xFF80  # position 55, head 1: -inf
+    Q[:, :, 1, 4] = np.abs(Q[:, :, 1, 4]) + 0.1
+    got = host(ie.prefill_attn(dev(Q), dev(kc), dev(vc), dev(table), 0, 16, H, kv_dtype=ie.KV_BF16))[0]
+    assert np.isposinf(got[53:, 0, 8]).all()
+    assert np.isfinite(got[:48]).all() and np.isfinite(got[64:, 1]).all()
+    kept = np.delete(got[53:, 0], 8, axis=1)
+    assert np.isfinite(kept).all()
