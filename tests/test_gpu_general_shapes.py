@@ -4,7 +4,7 @@ time, at the sizes where their tiles, slices and last chunks end."""
 import numpy as np
 import pytest
 
-from conftest import pack_i8, rng
+from conftest import bf16_bits, pack_i8, rng
 
 pytestmark = pytest.mark.gpu
 
@@ -98,3 +98,38 @@ def test_quantize_wide_rows(ie, orc, rows, cols):
     p, s = (t.cpu().numpy() for t in ie.quantize(_dev(x)))
     want_p, want_s = orc.quantize(x)
     assert np.array_equal(s, want_s) and np.array_equal(p, want_p)
+
+
+# Paged cache writes.  Rows of whole float4s (one, a partial workgroup, exactly one, several), rows that are not
+# (H dh % 4 != 0), and buffers that start one element into a 16-byte chunk; the first position inside a page.
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("seq,start,H,dh,bs,skew", [(1, 0, 1, 4, 16, 0), (7, 5, 3, 20, 4, 0), (33, 15, 16, 64, 16, 0),
+                                                    (3, 2, 20, 128, 5, 0), (9, 30, 3, 5, 16, 0), (20, 3, 12, 64, 8, 1),
+                                                    (2, 1, 24, 96, 16, 2)])
+def test_kv_write_rows(ie, seq, start, H, dh, bs, skew, bf16):
+    import torch
+
+    r = rng(seq + H + dh)
+    P = (start + seq + bs - 1) // bs + 2
+    table = r.permutation(P).astype(np.int32)
+    K, V = (r.standard_normal((seq, H, dh)).astype(np.float32) for _ in range(2))
+    K.reshape(-1)[:4] = [np.inf, -np.inf, -0.0, 1e-40]
+
+    def skewed(a):
+        buf = torch.zeros(a.size + skew, dtype=torch.float32, device="cuda")
+        buf[skew:] = torch.from_numpy(a.reshape(-1))
+        return buf[skew:].view(seq, H, dh)
+
+    def cache():
+        n = P * bs * H * dh
+        return torch.full((n + skew,), -7, dtype=torch.int16 if bf16 else torch.int32, device="cuda")[skew:].view(
+            P, bs, H, dh)
+
+    kc, vc = cache(), cache()
+    ie.kv_cache_write(skewed(K), skewed(V), kc, vc, _dev(table), start, bs, kv_dtype=ie.KV_BF16 if bf16 else ie.KV_F32)
+    for src, c in ((K, kc), (V, vc)):
+        bits = bf16_bits(src).view(np.int16) if bf16 else src.view(np.int32)
+        want = np.full((P, bs, H, dh), -7, bits.dtype)
+        pos = start + np.arange(seq)
+        want[table[pos // bs], pos % bs] = bits
+        assert np.array_equal(c.cpu().numpy(), want)
