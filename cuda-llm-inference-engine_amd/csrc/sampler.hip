@@ -10,13 +10,26 @@
 // One 1024-thread workgroup per row.  Rows of up to 65533 logits (GPT-2's
 // 50257 among them) are read once, as 16-byte chunks, into registers (64 keys
 // per thread):
-//   1. a lower bound M of the k-th largest key: the k-th largest of the 1024
-//      per-thread maxima (a radix select over one key per thread);
-//   2. the keys >= M (typically a few more than k) gathered into LDS;
+//   1. a lower bound M of the k-th largest key.  For k up to 64 (of 16 full
+//      waves): each wave finds, by a bit search with one ballot per bit, the
+//      first 20 bits of the r-th largest of its 64 per-thread maxima, r =
+//      ceil(k / waves), and M is the least of those, so at least k keys reach
+//      it; one barrier.  For larger k the least of the waves' bounds lets ever
+//      more keys through (8 rows at k = 400 83.8 against 24.2 us): M is the
+//      k-th largest of the 1024 maxima (a radix select over one key per
+//      thread, sixteen barriers);
+//   2. the keys >= M (typically k to a few times k) gathered into LDS;
 //   3. each gathered key ranked by counting those before it (larger key, or
-//      equal key and lower index), and the first k written.
-// Longer rows, and rows where more than 2048 keys reach M (many equal
-// values, or k near 1024), are streamed from memory (L2 after the first
+//      equal key and lower index), several threads per key while there are
+//      fewer keys than threads, and the first k written.
+// Bound by its chain of barriers and by one CU's intake of the row.  Against
+// keys in place of floats, the radix select for every k and one thread per
+// ranked key: 8 rows of 50257 at k = 40 17.0 -> 9.4 us, 16 at 100 22.7 ->
+// 12.2, 4 at 600 83.6 -> 36.7, 1 at 1 12.2 -> 7.8; 3 rows of 1000 at 10 11.5 ->
+// 8.5.
+// Longer rows, rows that hold a NaN (whose order is its key's: the floats
+// above would drop it), and rows where more than 2048 keys reach M (many
+// equal values, or k near 1024), are streamed from memory (L2 after the first
 // pass) through an exact radix select of the k-th largest key, 8 bits per
 // pass (the histogram in LDS; each wave instruction adds its leading lane's
 // bin with one atomic, the other lanes' bins lane by lane), a gather of the
@@ -230,8 +243,8 @@ __device__ __forceinline__ void topk_stream_row(TopkShared& sh, const float* __r
 // Rows whose 16-byte chunks number at most 16 x 1024 (n + 3 <= 65536): the
 // row is read once as 16-byte chunks from its 16-byte-aligned base, thread t
 // holding chunks t + 1024 q (q < 16), i.e. indices 4 (t + 1024 q) + c - s
-// where s = the row start's float offset within its chunk.  Key 0 (the bit
-// pattern of a NaN, which rows do not hold) marks slots outside the row.
+// where s = the row start's float offset within its chunk; slots outside the
+// row hold -inf.
 __global__ __launch_bounds__(kTopkThreads) void topk_reg_kernel(const float* __restrict__ logits, int n, int k,
                                                                 float* __restrict__ out_vals,
                                                                 int* __restrict__ out_idx) {
@@ -243,53 +256,87 @@ __global__ __launch_bounds__(kTopkThreads) void topk_reg_kernel(const float* __r
     // chunks wholly inside the row: [cf, cl]; the (at most two) others that
     // touch it are read element by element by the one lane that holds each
     const int cf = s == 0 ? 0 : 1, cl = (n + s) / 4 - 1;
-    uint32_t key[kTopkRegPer];
+    // The row's values stay floats (compared as such: -0 equals +0, and the
+    // slots past its ends hold -inf); only maxima and candidates become keys.
+    constexpr int NC = kTopkRegPer / 4;
+    float4 val[NC];
 #pragma unroll
-    for (int q = 0; q < kTopkRegPer / 4; ++q) {
-        const int c = (int)threadIdx.x + q * kTopkThreads, e0 = 4 * c - s;
+    for (int q = 0; q < NC; ++q) {
+        const int c = (int)threadIdx.x + q * kTopkThreads;
         // branch-free for whole chunks, so all 16 loads are in flight together
-        float4 v = cf <= cl ? x4[min(max(c, cf), cl)] : make_float4(0.f, 0.f, 0.f, 0.f);
-        const bool whole = c >= cf && c <= cl;
-        if (!whole && e0 < n && e0 + 3 >= 0) {
-            v.x = e0 >= 0 && e0 < n ? x[e0] : 0.f;
-            v.y = e0 + 1 >= 0 && e0 + 1 < n ? x[e0 + 1] : 0.f;
-            v.z = e0 + 2 >= 0 && e0 + 2 < n ? x[e0 + 2] : 0.f;
-            v.w = e0 + 3 < n ? x[e0 + 3] : 0.f;
-        }
-        const float e[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int u = 0; u < 4; ++u) key[4 * q + u] = e0 + u >= 0 && e0 + u < n ? order_key(e[u]) : 0u;
+        val[q] = cf <= cl ? x4[min(max(c, cf), cl)] : make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    // index of key[j]: one base per thread plus a constant per slot (written
-    // this way the compiler does not keep 64 precomputed indices live)
-    const int ibase = 4 * (int)threadIdx.x - s;
-    auto index = [&](int j) { return ibase + (j >> 2) * (4 * kTopkThreads) + (j & 3); };
-
-    // Lower bound M: the k-th largest of the 1024 per-thread maxima (k <=
-    // 1024).  Those k maxima are k keys >= M, so every key of the top k is
-    // >= M.  The keys >= M (typically a few more than k) are gathered into
-    // LDS and ranked there; only when more than kTopkCand keys reach M (many
-    // ties, or k near 1024) is the row streamed through the radix select.
-    // (every loop over key[] is fully unrolled: an early exit would leave the
-    // array indexed at run time, i.e. in scratch memory)
-    uint32_t tmax = 0;
+    float fmx = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < kTopkRegPer; ++j) tmax = max(tmax, key[j]);
-    uint32_t remaining, eqcount;
-    const uint32_t M = radix_kth(
-        sh, (uint32_t)k,
-        [&](uint32_t hmask, uint32_t prefix, int shift) {
-            hist_add(sh.hist, (tmax & hmask) == prefix, (tmax >> shift) & 255u, lane);
-        },
-        lane, wid, remaining, eqcount);
-    if (threadIdx.x == 0) sh.gt = 0;
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < kTopkRegPer; ++j)
-        if (key[j] != 0u && key[j] >= M) {
-            const uint32_t slot = atomicAdd(&sh.gt, 1u);
-            if (slot < (uint32_t)kTopkCand) put(sh, slot, key[j], index(j));
+    for (int q = 0; q < NC; ++q) {
+        const int c = (int)threadIdx.x + q * kTopkThreads, e0 = 4 * c - s;
+        if (c < cf || c > cl) {
+            auto at = [&](int e) { return e >= 0 && e < n ? x[e] : -INFINITY; };
+            val[q] = make_float4(at(e0), at(e0 + 1), at(e0 + 2), at(e0 + 3));
         }
+        // (a NaN stays in this maximum)
+        fmx = __builtin_elementwise_maximum(fmx, __builtin_elementwise_maximum(val[q].x, val[q].y));
+        fmx = __builtin_elementwise_maximum(fmx, __builtin_elementwise_maximum(val[q].z, val[q].w));
+    }
+    const bool nan = __ballot(fmx != fmx) != 0;  // in this wave's part
+    // index of a chunk's first element: one base per thread plus a constant
+    const int ibase = 4 * (int)threadIdx.x - s;
+
+    // Lower bound M of the k-th largest (see the top).  (Every loop over val[]
+    // is fully unrolled: an early exit would leave the array indexed at run
+    // time, i.e. in scratch memory.)
+    const uint32_t tmax = order_key(fmx);
+    // Full waves: every lane holds at least one whole chunk of the row.
+    const int full = min(kTopkWaves, (n - 4) / 256);
+    uint32_t M;
+    if (full > 0 && k <= 4 * full) {  // uniform
+        const int r = (k + full - 1) / full;
+        uint32_t m = 0;
+#pragma unroll
+        for (int bit = 31; bit >= 12; --bit) {
+            const uint32_t c = m | (1u << bit);
+            if (__popcll(__ballot(tmax >= c)) >= r) m = c;
+        }
+        if (lane == 0) sh.wave_tot[wid] = nan ? 0u : wid < full ? m : 0xffffffffu;  // (no real m is 0)
+        if (threadIdx.x == 0) sh.gt = 0;
+        __syncthreads();
+        M = sh.wave_tot[0];
+#pragma unroll
+        for (int w = 1; w < kTopkWaves; ++w) M = min(M, sh.wave_tot[w]);
+    } else {
+        uint32_t remaining, eqcount;
+        M = radix_kth(
+            sh, (uint32_t)k,
+            [&](uint32_t hmask, uint32_t prefix, int shift) {
+                hist_add(sh.hist, (tmax & hmask) == prefix, (tmax >> shift) & 255u, lane);
+            },
+            lane, wid, remaining, eqcount);
+        if (lane == 0) sh.wave_tot[wid] = nan ? 0u : M;
+        if (threadIdx.x == 0) sh.gt = 0;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < kTopkWaves; ++w) M = min(M, sh.wave_tot[w]);
+    }
+    if (M == 0) {  // uniform: a NaN in the row
+        __syncthreads();
+        topk_stream_row(sh, x, n, k, out_vals, out_idx, lane, wid);
+        return;
+    }
+    const float Mf = M <= order_key(-INFINITY) ? -INFINITY : key_value(M);
+#pragma unroll
+    for (int q = 0; q < NC; ++q) {
+        const float e[4] = {val[q].x, val[q].y, val[q].z, val[q].w};
+        if (__ballot(fmaxf(fmaxf(e[0], e[1]), fmaxf(e[2], e[3])) >= Mf)) {  // (uniform: few chunks have any)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int i = ibase + q * (4 * kTopkThreads) + u;
+                if (e[u] >= Mf && i >= 0 && i < n) {
+                    const uint32_t slot = atomicAdd(&sh.gt, 1u);
+                    if (slot < (uint32_t)kTopkCand) put(sh, slot, order_key(e[u]), i);
+                }
+            }
+        }
+    }
     __syncthreads();
     const uint32_t cnt = sh.gt;
     if (cnt > (uint32_t)kTopkCand) {  // uniform
@@ -298,18 +345,28 @@ __global__ __launch_bounds__(kTopkThreads) void topk_reg_kernel(const float* __r
         return;
     }
     // rank sort: a candidate's place is the number of candidates before it
-    // (larger key, or equal key and lower index); places are distinct
-    for (int t = threadIdx.x; t < (int)cnt; t += kTopkThreads) {
-        const uint32_t kt = sh.ckey[t];
-        const int it = sh.cidx[t];
+    // (larger key, or equal key and lower index: the larger of the words
+    // packed here); places are distinct.  2^per threads share a candidate,
+    // reading two others at a time.
+    __shared__ __attribute__((aligned(16))) uint64_t pk[kTopkCand + 2];
+    for (int t = threadIdx.x; t < (int)cnt + 2; t += kTopkThreads)
+        pk[t] = t < (int)cnt ? ((uint64_t)sh.ckey[t] << 32) | (0xffffffffu - (uint32_t)sh.cidx[t]) : 0;
+    __syncthreads();
+    int per = 0;
+    while (per < 5 && ((int)cnt << (per + 1)) <= kTopkThreads) ++per;
+    const int sub = threadIdx.x & ((1 << per) - 1);
+    for (int t = threadIdx.x >> per; t < (int)cnt; t += kTopkThreads >> per) {
+        const uint64_t mine = pk[t];
         int rank = 0;
-        for (int u = 0; u < (int)cnt; ++u) {
-            const uint32_t ku = sh.ckey[u];
-            rank += ku > kt || (ku == kt && sh.cidx[u] < it);
+#pragma unroll 4
+        for (int u = 2 * sub; u < (int)cnt; u += 2 << per) {
+            const ulonglong2 o = *reinterpret_cast<const ulonglong2*>(pk + u);
+            rank += (int)(o.x > mine) + (int)(o.y > mine);
         }
-        if (rank < k) {
-            out_vals[(size_t)blockIdx.x * k + rank] = key_value(kt);
-            out_idx[(size_t)blockIdx.x * k + rank] = it;
+        for (int o = 1; o < 1 << per; o <<= 1) rank += __shfl_xor(rank, o, 64);
+        if (sub == 0 && rank < k) {
+            out_vals[(size_t)blockIdx.x * k + rank] = key_value(sh.ckey[t]);
+            out_idx[(size_t)blockIdx.x * k + rank] = sh.cidx[t];
         }
     }
 }

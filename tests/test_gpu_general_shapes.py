@@ -133,3 +133,35 @@ def test_kv_write_rows(ie, seq, start, H, dh, bs, skew, bf16):
         pos = start + np.arange(seq)
         want[table[pos // bs], pos % bs] = bits
         assert np.array_equal(c.cpu().numpy(), want)
+
+
+def _key_order(row):
+    """Indices by the float's order key (a NaN past the infinity of its sign), descending, lower index first."""
+    b = row.view(np.uint32).copy()
+    b[b == 0x80000000] = 0
+    key = np.where(b & 0x80000000, ~b, b | 0x80000000).astype(np.uint32)
+    return np.argsort(-key.astype(np.int64), kind="stable")
+
+
+# Top-k.  n: fewer than 256 + 4 logits (no wave whose lanes all hold a chunk), one such wave, 15 and 16; k on both sides
+# of four per full wave, and where the gathered keys pass the 2048 that are ranked; the maxima in one thread's or one
+# wave's chunks (the bound lets every key through); rows mostly -inf; rows that hold NaNs.
+@pytest.mark.parametrize("n,k", [(4, 4), (259, 3), (260, 4), (260, 5), (3844, 60), (3844, 61), (4100, 64), (4099, 65),
+                                 (4101, 512), (50257, 64), (50257, 65), (50257, 700), (65533, 1024), (8000, 16)])
+def test_topk_bounds(ie, n, k):
+    import torch
+
+    r = rng(n + k)
+    x = r.standard_normal((7, n)).astype(np.float32)
+    x[1, :min(n, 64)] += 50  # the first chunks
+    x[2, ::max(1, min(4096, n // 2))] += 50  # one thread's
+    x[3, r.random(n) < 0.995] = -np.inf
+    x[4] = np.round(x[4] * 2)
+    x[5, r.integers(0, n, 3)] = np.nan
+    x[6] = np.nan
+    v, i = ie.topk(torch.from_numpy(x).cuda(), k)
+    v, i = v.cpu().numpy(), i.cpu().numpy()
+    for b in range(7):
+        want = _key_order(x[b])[:k]
+        assert np.array_equal(i[b], want), b
+        assert np.array_equal(v[b], x[b][want], equal_nan=True), b
