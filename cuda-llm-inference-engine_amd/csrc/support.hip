@@ -4,6 +4,7 @@
 // are written for low latency, not as roofline kernels.
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 
 #include "device_util.h"
 #include "ie_internal.h"
@@ -163,6 +164,88 @@ __global__ __launch_bounds__(256) void vocab_proj_kernel(int rows, const float* 
         if (li == r) mine = t;
     }
     if (ok && li < rows && li < RT) logits[(size_t)li * V + j] = mine;
+}
+
+// The same sums (each lane's products and their order, then row16_sum) for 2
+// to MB hidden rows.  vocab_proj_kernel re-reads every hidden row from the
+// caches for each vocabulary row, which bounds it for more than one; here they
+// are staged in LDS once per workgroup of 16 waves (one per CU), a wave takes
+// 4 R vocabulary rows per tile, so each LDS read serves R of them, and P
+// chunks of 64 k of their weights are in flight.  1600 x 50257 (322 MB): 1 row
+// 52.5 us by that kernel; 2 / 8 / 16 rows 246 / 248 / 249 by it -> 54.5 / 60.2 /
+// 68.7 us, bound by the weights' stream at few rows and by fp32 FMAs (one
+// hidden row's per LDS read) at 16; 900 x 1000, 4 / 16 rows 21.0 / 26.4 -> 4.4 /
+// 9.3 us.
+constexpr int kProjLds = 128 << 10;
+template <int MB, int R, int P>
+__global__ __launch_bounds__(1024) void vocab_proj_rows_kernel(int rows, const float* __restrict__ h,
+                                                               const float* __restrict__ wte,
+                                                               float* __restrict__ logits, int d, int V) {
+    __shared__ float4 hs[kProjLds / 16];
+    const int lane = threadIdx.x & 63, li = lane & 15, g = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ntiles = (V + 4 * R - 1) / (4 * R), nch = (d + 63) / 64, d4 = d >> 2;
+    // tiles go round the workgroups first
+    int t = w * (int)gridDim.x + (int)blockIdx.x;
+    const float* wrow[R];
+    float4 wv[P][R];
+    auto load = [&](float4 (&dst)[R], int c) {
+        const int k = min(4 * li + 64 * c, d - 4);
+#pragma unroll
+        for (int rr = 0; rr < R; ++rr)
+            dst[rr] = *reinterpret_cast<const float4*>(wrow[rr] + k);
+    };
+    auto begin = [&](int t) {
+#pragma unroll
+        for (int rr = 0; rr < R; ++rr) wrow[rr] = wte + (size_t)min(t * 4 * R + 4 * rr + g, V - 1) * d;
+#pragma unroll
+        for (int u = 0; u < P; ++u) load(wv[u], u);
+    };
+    if (t < ntiles) begin(t);
+    for (int e = threadIdx.x; e < rows * d4; e += 1024) hs[e] = reinterpret_cast<const float4*>(h)[e];
+    __syncthreads();
+    for (; t < ntiles; t += 16 * (int)gridDim.x) {
+        float acc[R][MB];
+#pragma unroll
+        for (int rr = 0; rr < R; ++rr)
+#pragma unroll
+            for (int r = 0; r < MB; ++r) acc[rr][r] = 0.0f;
+        for (int c0 = 0; c0 < nch; c0 += P) {
+#pragma unroll
+            for (int u = 0; u < P; ++u) {
+                const int c = c0 + u;
+                if (4 * li + 64 * c < d) {
+                    const float4* hc = hs + 16 * c + li;
+#pragma unroll
+                    for (int r = 0; r < MB; ++r) {
+                        const float4 hv = hc[min(r, rows - 1) * d4];
+#pragma unroll
+                        for (int rr = 0; rr < R; ++rr) {
+                            float a = acc[rr][r];
+                            a = fmaf(wv[u][rr].x, hv.x, a);
+                            a = fmaf(wv[u][rr].y, hv.y, a);
+                            a = fmaf(wv[u][rr].z, hv.z, a);
+                            a = fmaf(wv[u][rr].w, hv.w, a);
+                            acc[rr][r] = a;
+                        }
+                    }
+                }
+                load(wv[u], c + P);
+            }
+        }
+        const int v0 = t * 4 * R + g;
+        if (t + 16 * (int)gridDim.x < ntiles) begin(t + 16 * (int)gridDim.x);
+#pragma unroll
+        for (int rr = 0; rr < R; ++rr) {
+            float mine = 0.0f;
+#pragma unroll
+            for (int r = 0; r < MB; ++r) {
+                const float s = row16_sum(acc[rr][r]);
+                if (li == r) mine = s;
+            }
+            if (li < rows && v0 + 4 * rr < V) logits[(size_t)li * V + v0 + 4 * rr] = mine;
+        }
+    }
 }
 
 // The same projection on v_mfma_f32_16x16x4_f32 for any row count 1..16
@@ -585,9 +668,29 @@ void launch_vocab_proj(int rows, const float* h, const float* wte, float* logits
         return;
     }
     const unsigned blocks = (unsigned)((V + 15) / 16);
+    // One row has nothing to share; rows past the LDS stage (16 of more than
+    // 2048) read the caches.  All give the same bits per row.
     if (rows == 1)
         vocab_proj_kernel<1><<<blocks, 256, 0, s>>>(rows, h, wte, logits, d, V);
-    else
+    else if ((size_t)rows * d * sizeof(float) <= (size_t)kProjLds) {
+        auto go = [&](auto mb, auto r) {
+            constexpr int MB = decltype(mb)::value, R = decltype(r)::value;
+            const unsigned grid = (unsigned)std::min<long long>((V + 4LL * R - 1) / (4 * R), num_cus());
+            vocab_proj_rows_kernel<MB, R, 8 / R><<<grid, 1024, 0, s>>>(rows, h, wte, logits, d, V);
+        };
+        std::integral_constant<int, 1> r1;
+        std::integral_constant<int, 2> r2;
+        // Above four rows the LDS reads count, and R = 2 halves them where it
+        // still leaves half of the chip's waves a tile: 8 / 16 rows of 900 x
+        // 30000 25.9 / 34.2 -> 24.6 / 30.0 us (2044 x 9000 18.8 / 25.2 against
+        // 18.5 / 25.9, 900 x 1000 6.2 / 9.3 against 7.1 / 10.9; 2 / 4 rows of
+        // 516 x 50257 23.8 / 24.0 against 24.0 / 25.2).
+        const bool pairs = (V + 7LL) / 8 >= 8LL * num_cus();
+        if (rows <= 2) go(std::integral_constant<int, 2>{}, r1);
+        else if (rows <= 4) go(std::integral_constant<int, 4>{}, r1);
+        else if (rows <= 8) pairs ? go(std::integral_constant<int, 8>{}, r2) : go(std::integral_constant<int, 8>{}, r1);
+        else pairs ? go(std::integral_constant<int, 16>{}, r2) : go(std::integral_constant<int, 16>{}, r1);
+    } else
         vocab_proj_kernel<16><<<blocks, 256, 0, s>>>(rows, h, wte, logits, d, V);
 }
 

@@ -165,3 +165,27 @@ def test_topk_bounds(ie, n, k):
         want = _key_order(x[b])[:k]
         assert np.array_equal(i[b], want), b
         assert np.array_equal(v[b], x[b][want], equal_nan=True), b
+
+
+# The language-model head at widths that are no multiple of 256 (or past 1280).  d: one float4, a partial chunk of 64, a
+# whole one, either side of the chunks in flight (8 x 64, 4 x 64); rows at each padded count and either side; V: part of
+# a tile, one and two vocabulary rows per wave (16384 on is the rule's line on 256 units), several tiles per wave; the
+# last rows x d that is staged whole (16 x 2048) and the first that is not.
+@pytest.mark.parametrize("d,V", [(4, 33), (60, 5), (64, 1027), (260, 2050), (516, 17001), (300, 50257), (1328, 999),
+                                 (2044, 16383), (2048, 16385), (2052, 300), (4096, 77)])
+def test_vocab_proj_any_width(ie, d, V):
+    import torch
+
+    r = rng(d + V)
+    h = torch.from_numpy(r.standard_normal((16, d)).astype(np.float32)).cuda()
+    w = torch.from_numpy((0.02 * r.standard_normal((V, d))).astype(np.float32)).cuda()
+    one = torch.cat([ie.vocab_proj(h[i:i + 1].contiguous(), w) for i in range(16)])
+    # chains of 4 ceil(d / 64) fused multiply-adds, then four additions: n roundings of at most 2^-24 each
+    n = 4 * ((d + 63) // 64) + 4
+    bound = n * 2.0 ** -24 * (h.double().abs() @ w.double().abs().t().contiguous())
+    assert ((one.double() - h.double() @ w.double().t().contiguous()).abs() <= bound).all()
+    for rows in (2, 3, 4, 5, 8, 9, 15, 16):
+        out = torch.full((rows * V + 8,), 7.0, device="cuda")
+        ie.vocab_proj(h[:rows].contiguous(), w, out[:rows * V].view(rows, V))
+        assert torch.equal(out[:rows * V].view(rows, V), one[:rows]), rows
+        assert (out[rows * V:] == 7.0).all()
