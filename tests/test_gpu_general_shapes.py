@@ -189,3 +189,22 @@ def test_vocab_proj_any_width(ie, d, V):
         ie.vocab_proj(h[:rows].contiguous(), w, out[:rows * V].view(rows, V))
         assert torch.equal(out[:rows * V].view(rows, V), one[:rows]), rows
         assert (out[rows * V:] == 7.0).all()
+
+
+# The GELU epilogue against 64 bits, v given as the bias of a zero product, over every size of v: 0.5 v (1 + tanh u) =
+# v s with s = 1 / (1 + exp(-2u)).  Five roundings of the exponent (three operations, two constants) move v s by at most
+# 5 |2u| s (1 - s) <= 1.12 units of 2^-24 |v|, the exponential's last place by 2 s (1 - s) <= 0.5, the result's by 1.
+@pytest.mark.parametrize("M", [1, 16, 40, 600])
+def test_gelu_epilogue_range(ie, M):
+    r = rng(M)
+    mag = np.concatenate([2.0 ** r.uniform(-140, 127, 2000), r.uniform(0, 12, 4000), [0.0, 1e-45, 5.5, 5.6, 3e38]])
+    v = np.concatenate([mag, -mag]).astype(np.float32)
+    N = v.size
+    A, W = np.zeros((M, 64), np.int8), np.ones((N, 64), np.int8)
+    got = ie.int8_gemm(_dev(pack_i8(A)), _dev(pack_i8(W)), _dev(np.ones(M, np.float32)), _dev(np.ones(N, np.float32)),
+                       ie.EPI_BIAS_GELU, _dev(v)).cpu().numpy().astype(np.float64)
+    d = v.astype(np.float64)
+    u = 0.7978845608 * (d + 0.044715 * d ** 3)
+    with np.errstate(over="ignore"):
+        want = d / (1.0 + np.exp(-2.0 * u))
+    assert (np.abs(got - want) <= 2.7 * 2.0 ** -24 * np.abs(d) + 2.0 ** -149).all()
