@@ -27,7 +27,9 @@
 // bytes, and the A chunks of it that the stage before already counted are
 // copied from a block of zeros instead, so every copy stays inside its row
 // and the loop is the same (M = 300, K = 1600, N = 4801 30.2 us on a
-// 128 x 128 register-staged kernel with one step in flight, 12.0 here).
+// 128 x 128 register-staged kernel with one step in flight, 10.9 here).
+
+#include <type_traits>
 
 #include "device_util.h"
 #include "epilogue.h"
@@ -77,7 +79,7 @@ __global__ __launch_bounds__(256) void gemm_i8_tile_kernel(int M, int N, int K, 
     constexpr int MI = BM / 64, NJ = BN / 64;  // 32x32 blocks per wave
     constexpr int LA = BM / 32, LB = BN / 32;  // wave-loads per operand per stage (8 rows each, 4 waves)
     constexpr int LPS = LA + LB;
-    static_assert(MI >= 1 && NJ >= 1 && (NSTAGE - 1) * LPS <= 63, "tile and ring fit");
+    static_assert(NSTAGE >= 2 && NSTAGE <= 4 && MI >= 1 && NJ >= 1 && (NSTAGE - 1) * LPS <= 63, "tile and ring fit");
     // (kEpiQKVRoute: BM row slots after the ring, in the same array: a
     // second LDS object would make the compiler drain the copies in flight
     // before every LDS read of the K loop)
@@ -108,9 +110,7 @@ __global__ __launch_bounds__(256) void gemm_i8_tile_kernel(int M, int N, int K, 
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0;
 
     const int nk = TAIL ? (K + BK - 1) / BK : K / BK;
-    // Copies stage kt_src into LDS slot `slot`.  Every iteration issues one
-    // stage, so the loop body is branch-free: past the last stage the copy
-    // re-reads stage nk-1 into the slot just freed, which is never read again.
+    // Copies stage kt_src into LDS slot `slot`.
     auto issue = [&](int kt_src, int slot) {
         int8_t* sa = lds + slot * STAGE;
         int8_t* sb = sa + OA;
@@ -121,10 +121,66 @@ __global__ __launch_bounds__(256) void gemm_i8_tile_kernel(int M, int N, int K, 
         for (int j = 0; j < LB; ++j) load_rows(BT, K, N, n0, k0, (wave * LB + j) * 8, sb);
     };
 
+    // Lane l of a 32x32 block holds rows 8q + 4(l/32) + r (q, r < 4) of
+    // column l % 32.  Every operand the stores need (scales, bias, residual;
+    // clamped indices) is requested before the first stage and has arrived with
+    // it.  Requested after the K loop, behind copies past the last stage, their
+    // latency was part of every launch (M = 512, K = 768, N = 3072 with the
+    // residual 7.32 -> 6.86 us; M = 300, K = 1600, N = 4800 with the bias 11.5 ->
+    // 10.9; M = 1000, K = 2000, N = 4000 24.4 -> 22.4).  In straight-line code:
+    // loaded in the branchy store loop, each would also wait for all earlier
+    // stores (vmcnt counts stores, and C may alias them).
+    const int h = lane >> 5;
+    const int rbase = m0 + wm * (BM / 2) + 4 * h;
+    const int cbase = n0 + wn * (BN / 2) + (lane & 31);
+    constexpr bool HAS_BIAS =
+        EPI == IE_EPI_BIAS || EPI == IE_EPI_BIAS_GELU || EPI == IE_EPI_BIAS_RESIDUAL || ROUTE;
+    constexpr bool HAS_RES = EPI == IE_EPI_BIAS_RESIDUAL;
+    auto row = [&](int i, int v) { return rbase + i * 32 + 8 * (v >> 2) + (v & 3); };
+    float sa[MI][16] = {}, sb[NJ] = {}, bv[NJ] = {}, rv[MI][16][NJ] = {};
+    int slot0 = 0;
+    if constexpr (ROUTE) slot0 = route.row_slot[min(m0 + (int)(threadIdx.x % BM), M - 1)];
+    if constexpr (EPI != IE_EPI_I32) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const int n = min(cbase + j * 32, N - 1);
+            sb[j] = sB[n];
+            if constexpr (HAS_BIAS) bv[j] = bias[n];
+        }
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int m = min(row(i, v), M - 1);
+                sa[i][v] = sA[m];
+                if constexpr (HAS_RES) {
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) rv[i][v][j] = residual[(size_t)m * N + min(cbase + j * 32, N - 1)];
+                }
+            }
+    }
+
     // Prologue: stages 0 .. NSTAGE-2 in flight, stage 0 landed.
 #pragma unroll
     for (int p = 0; p < NSTAGE - 1; ++p) issue(min(p, nk - 1), p);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NSTAGE - 2) * LPS) : "memory");
+    if constexpr (EPI != IE_EPI_I32) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                asm volatile("" ::"v"(sa[i][v]));
+                if constexpr (HAS_RES) {
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) asm volatile("" ::"v"(rv[i][v][j]));
+                }
+            }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            asm volatile("" ::"v"(sb[j]));
+            if constexpr (HAS_BIAS) asm volatile("" ::"v"(bv[j]));
+        }
+    }
     __builtin_amdgcn_s_barrier();
 
     const int frow = lane & 31;
@@ -147,7 +203,13 @@ __global__ __launch_bounds__(256) void gemm_i8_tile_kernel(int M, int N, int K, 
     frags(lds, lds + OA, 0, 0);
 
     constexpr int SUB = BK / 32;  // MFMA k-substeps per stage
-    for (int kt = 0; kt < nk; ++kt) {
+    // Stage kt: COPY also requests stage kt + NSTAGE - 1 into the slot freed by
+    // stage kt - 1 (every wave passed its last barrier); LEFT is the number of
+    // stages that may still be in flight once stage kt + 1 has landed, -1 if
+    // kt is the last.
+    auto stage = [&](int kt, auto copy, auto left) {
+        constexpr bool COPY = decltype(copy)::value;
+        constexpr int LEFT = decltype(left)::value;
         const int8_t* sa = lds + (kt % NSTAGE) * STAGE;
         const int8_t* sb = sa + OA;
 #pragma unroll
@@ -155,9 +217,7 @@ __global__ __launch_bounds__(256) void gemm_i8_tile_kernel(int M, int N, int K, 
             const int slot = ks & 1;
             __builtin_amdgcn_sched_barrier(0);
             if (ks + 1 < SUB) {
-                // the copies of stage kt + NSTAGE - 1 go into the slot freed
-                // by iteration kt - 1 (every wave passed its last barrier)
-                if (ks == 0) issue(min(kt + NSTAGE - 1, nk - 1), (kt + NSTAGE - 1) % NSTAGE);
+                if (COPY && ks == 0) issue(kt + NSTAGE - 1, (kt + NSTAGE - 1) % NSTAGE);
                 frags(sa, sb, ks + 1, slot ^ 1);
                 mfmas(slot);
             } else {
@@ -166,71 +226,36 @@ __global__ __launch_bounds__(256) void gemm_i8_tile_kernel(int M, int N, int K, 
                 // s_barrier, since __syncthreads()' fence drains vmcnt to 0),
                 // then the next stage's first fragments
                 mfmas(slot);
-                __builtin_amdgcn_sched_barrier(0);
-                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NSTAGE - 2) * LPS) : "memory");
-                __builtin_amdgcn_s_barrier();
-                __builtin_amdgcn_sched_barrier(0);
-                const int8_t* na = lds + ((kt + 1) % NSTAGE) * STAGE;
-                frags(na, na + OA, 0, 0);
+                if constexpr (LEFT >= 0) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LEFT * LPS) : "memory");
+                    __builtin_amdgcn_s_barrier();
+                    __builtin_amdgcn_sched_barrier(0);
+                    const int8_t* na = lds + ((kt + 1) % NSTAGE) * STAGE;
+                    frags(na, na + OA, 0, 0);
+                }
             }
         }
         __builtin_amdgcn_sched_barrier(0);
-    }
+    };
+    // The last NSTAGE - 1 stages copy nothing, so nothing is in flight after
+    // them (copies of the last stage into freed slots, which kept one loop
+    // body, cost their traffic and a wait before the epilogue).
+    int kt = 0;
+    for (; kt < nk - (NSTAGE - 1); ++kt) stage(kt, std::true_type{}, std::integral_constant<int, NSTAGE - 2>{});
+    if constexpr (NSTAGE >= 4)
+        if (kt < nk - 2) stage(kt++, std::false_type{}, std::integral_constant<int, 1>{});
+    if constexpr (NSTAGE >= 3)
+        if (kt < nk - 1) stage(kt++, std::false_type{}, std::integral_constant<int, 0>{});
+    stage(kt, std::false_type{}, std::integral_constant<int, -1>{});
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
 
-    // Epilogue.  Lane l of a 32x32 block holds rows 8q + 4(l/32) + r (q, r < 4)
-    // of column l % 32.  Every operand the stores need (scales, bias,
-    // residual; clamped indices) is gathered first and consumed once in
-    // straight-line code: loaded inside the branchy store loop, each would
-    // wait for all earlier stores (vmcnt counts stores, and C may alias them).
-    const int h = lane >> 5;
-    const int rbase = m0 + wm * (BM / 2) + 4 * h;
-    const int cbase = n0 + wn * (BN / 2) + (lane & 31);
-    constexpr bool HAS_BIAS =
-        EPI == IE_EPI_BIAS || EPI == IE_EPI_BIAS_GELU || EPI == IE_EPI_BIAS_RESIDUAL || ROUTE;
-    constexpr bool HAS_RES = EPI == IE_EPI_BIAS_RESIDUAL;
-    auto row = [&](int i, int v) { return rbase + i * 32 + 8 * (v >> 2) + (v & 3); };
-    float sa[MI][16] = {}, sb[NJ] = {}, bv[NJ] = {}, rv[MI][16][NJ] = {};
-    // kEpiQKVRoute: the tile's row slots go to LDS (32 of them per lane in
-    // registers cost a wave per SIMD), read back beside each store
+    // (the row slots go to LDS: 32 of them per lane in registers cost a wave
+    // per SIMD)
     int* lslot = reinterpret_cast<int*>(lds + NSTAGE * STAGE);
     if constexpr (ROUTE) {
-        if (threadIdx.x < BM) lslot[threadIdx.x] = route.row_slot[min(m0 + (int)threadIdx.x, M - 1)];
+        if (threadIdx.x < BM) lslot[threadIdx.x] = slot0;
         __syncthreads();
-    }
-    if constexpr (EPI != IE_EPI_I32) {
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const int n = min(cbase + j * 32, N - 1);
-            sb[j] = sB[n];
-            if constexpr (HAS_BIAS) bv[j] = bias[n];
-        }
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int m = min(row(i, v), M - 1);
-                sa[i][v] = sA[m];
-                if constexpr (HAS_RES) {
-#pragma unroll
-                    for (int j = 0; j < NJ; ++j) rv[i][v][j] = residual[(size_t)m * N + min(cbase + j * 32, N - 1)];
-                }
-            }
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                asm volatile("" ::"v"(sa[i][v]));
-                if constexpr (HAS_RES) {
-#pragma unroll
-                    for (int j = 0; j < NJ; ++j) asm volatile("" ::"v"(rv[i][v][j]));
-                }
-            }
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            asm volatile("" ::"v"(sb[j]));
-            if constexpr (HAS_BIAS) asm volatile("" ::"v"(bv[j]));
-        }
     }
 #pragma unroll
     for (int i = 0; i < MI; ++i) {

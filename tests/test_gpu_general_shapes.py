@@ -208,3 +208,15 @@ def test_gelu_epilogue_range(ie, M):
     with np.errstate(over="ignore"):
         want = d / (1.0 + np.exp(-2.0 * u))
     assert (np.abs(got - want) <= 2.7 * 2.0 ** -24 * np.abs(d) + 2.0 ** -149).all()
+
+
+# The 64 x 64 and 128 x 64 LDS tiles: fewer stages than the ring (one to three of 128), as many, more, and a tail; one
+# workgroup per CU, two, up to three, and past each (256 units; partial tiles both ways).
+@pytest.mark.parametrize("K", [128, 256, 272, 384, 512, 1296, 2064])
+@pytest.mark.parametrize("M,N", [(640, 1600), (641, 1601), (512, 4096), (1150, 1800), (768, 4096), (833, 3840),
+                                 (1000, 4160)])
+def test_gemm_tile_rounds(ie, orc, M, N, K):
+    _gemm_case(ie, orc, M, N, K, ie.EPI_I32, 0, M + N + K)
+    if K in (256, 1296):
+        for epi in (ie.EPI_BIAS_GELU, 3):
+            _gemm_case(ie, orc, M, N, K, epi, 0, M + N + K)
