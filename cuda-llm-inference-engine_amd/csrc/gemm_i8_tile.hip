@@ -10,7 +10,7 @@
 // small workgroups per CU cover it better than one large one.  The tile is
 // BM x BN (64 x 64 or 128 x 64) on four waves (2 x 2, each (BM/2) x (BN/2)
 // as 32x32 blocks of v_mfma_i32_32x32x32_i8), and K advances through a ring
-// of NSTAGE 128-byte stages in LDS (2-3; 4 for long K or a one-round grid),
+// of NSTAGE 128-byte stages in LDS (two to four, see TileLaunch),
 // NSTAGE - 1 of them in flight while one is read:
 //   * global -> LDS copies are global_load_lds_dwordx4 (16 B per lane straight
 //     into LDS); a wave-load fills 8 rows x 128 B; the lane -> global address
@@ -298,41 +298,41 @@ struct TileLaunch {
                                  reinterpret_cast<const int8_t*>(a.BT), a.sA, a.sB, a.bias, a.residual, a.C, tm, tn,
                                  a.route);
     }
-    // Measured on the GPT-2 prefill shapes (M = 128-2048, K = 768 / 3072,
-    // N = 768-3072, bias epilogue; same box, bit-identical C): 128 x 64 tiles
-    // beat 64 x 64 once there are two per CU (M = 2048, N = 2304: 12.1
-    // against 13.7 us) and keep two stages (three: 11.1 -> 13.7 us, fewer
-    // workgroups per CU); 64 x 64 tiles take three stages at K = 768, two in
-    // flight, which pays when the weights come from the MALL or HBM rather
-    // than L2 (GPT-2 prefill TTFT at batch 1: 0.705 -> 0.684 ms; weights
-    // rotated through 1 GiB, M = 512, N = 768: 7.55 -> 5.95 us; the same
-    // weights every launch, L2-resident: 5.09 -> 5.20 us), and four over long
-    // K (K = 3072) or when the grid is one round of workgroups, one per CU
-    // (rotated weights, K = 768: M = 512, N = 768 5.88 -> 5.37 us; M = 128,
-    // N = 2304 6.01 -> 5.41 us, N = 3072 6.05 -> 5.49 us; with 288-384 tiles
-    // four stages measured 3% slower); six or eight stages measured slower
-    // still, in one round too (K = 3072: 10.4 -> 10.9-11.1 us); 128 x 128
-    // tiles lost everywhere.
+    // 64 x 64 tiles take as many stages as leave the grid in one round of
+    // workgroups (32 KiB of LDS each for two stages, 48 for three, 64 for
+    // four; bias epilogue, weights rotated through 600 MB):
+    //   * past two per CU two stages: a third costs a second round (M = 640, N =
+    //     4096, K = 1280 / 3072 11.7 / 21.6 -> 11.0 / 18.8 us; M = 768, N = 4096,
+    //     K = 2000 19.8 -> 18.7; M = 768, N = 3072, K = 768 8.75 -> 8.6);
+    //   * up to two per CU three at short K (M = 512, N = 3072, K = 768: 6.84 /
+    //     6.55 / 6.48 us for two / three / four; M = 512, N = 4096, K = 2000 13.0 /
+    //     14.1 / 14.0), four from K = 2048 on or in a round of one per CU (M =
+    //     512, N = 4096, K = 4096 27.1 / 21.2 / 20.7; M = 128, N = 8192, K = 4096
+    //     27.3 / 17.6 / 14.3); six or eight measured slower.
+    // 128 x 64 tiles take two (three or four leave two or one workgroup per CU:
+    // M = 1024, N = 5120, K = 3072 30.8 / 34.3 / 36.3 us; M = 2048, N = 2304, K = 768
+    // 10.5 / 12.6 / 16.5).  128 x 128 tiles won only at some long K past one
+    // round (M = 1000, N = 4000, K = 2000 / 4096 19.3 / 29.0 against 20.6 / 32.6 us)
+    // and lost by up to 30% elsewhere.
     static void run(const GemmArgs& a, hipStream_t s) {
-        const bool long_k = a.K >= 2048;
-        if (gemm_i8_tile_shape(a) == 128064) {
-            if (long_k) go<128, 64, 4>(a, s);
-            else go<128, 64, 2>(a, s);
-        } else {
-            const long long tiles = (long long)((a.M + 63) / 64) * ((a.N + 63) / 64);
-            if (long_k || tiles <= num_cus()) go<64, 64, 4>(a, s);
-            else go<64, 64, 3>(a, s);
-        }
+        const long long tiles = (long long)((a.M + 63) / 64) * ((a.N + 63) / 64), cus = num_cus();
+        if (gemm_i8_tile_shape(a) == 128064) go<128, 64, 2>(a, s);
+        else if (tiles > 2 * cus) go<64, 64, 2>(a, s);
+        else if (a.K >= 2048 || tiles <= cus) go<64, 64, 4>(a, s);
+        else go<64, 64, 3>(a, s);
     }
 };
 
 }  // namespace
 
-// Tile shape BM * 1000 + BN for a problem: 128 x 64 once that gives two
-// tiles per CU, else 64 x 64.
+// Tile shape BM * 1000 + BN for a problem: 128 x 64 once that gives two tiles
+// per CU, or once 64 x 64 tiles pass one round of three workgroups per CU
+// (M = 1000, N = 4000, 504 tiles against 1008: K = 1280 / 2000 / 4096 15.2 / 24.4 /
+// 37.9 -> 13.6 / 20.6 / 32.6 us; M = 768, N = 4096, 768 of 64 x 64: 11.6 / 18.7 /
+// 29.8 against 12.0 / 18.2 / 30.5); else 64 x 64.
 int gemm_i8_tile_shape(const GemmArgs& a) {
-    const long long t = (long long)((a.M + 127) / 128) * ((a.N + 63) / 64);
-    return t >= 2LL * num_cus() ? 128064 : 64064;
+    const long long tn = (a.N + 63) / 64, t64 = (a.M + 63) / 64 * tn, t128 = (a.M + 127) / 128 * tn;
+    return t128 >= 2LL * num_cus() || t64 > 3LL * num_cus() ? 128064 : 64064;
 }
 
 // Grids small enough for one round of 32 x 32 blocks take the K-split
