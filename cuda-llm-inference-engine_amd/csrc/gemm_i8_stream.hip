@@ -34,6 +34,8 @@
 // 16-byte aligned A and BT.  Rows past M or N read the last valid row (results
 // discarded).  K % 128 != 0 (TAIL): the last group covers the row's last 128
 // bytes, the A chunks already counted copied from a block of zeros.
+#include <type_traits>
+
 #include "device_util.h"
 #include "epilogue.h"
 #include "ie_internal.h"
@@ -101,17 +103,55 @@ __global__ __launch_bounds__(64 * KS) void gemm_i8_stream_kernel(
 #pragma unroll
         for (int j = 0; j < 4; ++j) copy_rows(BT, K, N, n0, k0, 8 * j, dst + 32 * KG);
     };
+    // Accumulator v of lane l is C[rbase + 8 (v / 4) + v % 4][n0 + l % 32].
+    // Every operand the stores need (scales, bias, residual; clamped
+    // indices) is requested by the wave that stores, before its first group,
+    // and has arrived with it: after the K loop their latency was part of
+    // every launch (with the residual M = 512, K = 768, N = 768 4.54 -> 4.12 us,
+    // M = 128, K = 768, N = 3072 4.83 -> 4.32; K = 3072, N = 768 6.20 -> 5.90; the
+    // copies past the last group went too).  In straight-line code: loaded in the branchy
+    // store loop, each would also wait for all earlier stores (vmcnt counts
+    // stores, and C may alias them).
+    const int cbase = n0 + (lane & 31);
+    const int rbase = m0 + 4 * (lane >> 5);
+    constexpr bool ROUTE = EPI == kEpiQKVRoute;
+    constexpr bool HAS_BIAS =
+        EPI == IE_EPI_BIAS || EPI == IE_EPI_BIAS_GELU || EPI == IE_EPI_BIAS_RESIDUAL || ROUTE;
+    constexpr bool HAS_RES = EPI == IE_EPI_BIAS_RESIDUAL;
+    float sa[16] = {}, sb = 0.0f, bv = 0.0f, rv[16] = {};
+    int slot[ROUTE ? 16 : 1] = {};
+    if (EPI != IE_EPI_I32 && wave == 0) {
+        const int n = min(cbase, N - 1);
+        sb = sB[n];
+        if constexpr (HAS_BIAS) bv = bias[n];
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const int m = min(rbase + 8 * (v >> 2) + (v & 3), M - 1);
+            sa[v] = sA[m];
+            if constexpr (HAS_RES) rv[v] = residual[(size_t)m * N + n];
+            if constexpr (ROUTE) slot[v] = route.row_slot[m];
+        }
+    }
     if (nk > 0) {
-        // Groups past the range re-read its last group (into slots that are
-        // never read), so every step issues exactly COPIES loads and each wait
-        // below leaves the LR - 2 younger groups in flight.
 #pragma unroll
         for (int p = 0; p < LR - 1; ++p) issue(g0 + min(p, nk - 1), p);
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"((LR - 2) * COPIES) : "memory");
+        if (EPI != IE_EPI_I32 && wave == 0) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                asm volatile("" ::"v"(sa[v]));
+                if constexpr (HAS_RES) asm volatile("" ::"v"(rv[v]));
+                if constexpr (ROUTE) asm volatile("" ::"v"(slot[v]));
+            }
+            asm volatile("" ::"v"(sb));
+            if constexpr (HAS_BIAS) asm volatile("" ::"v"(bv));
+        }
         const int fr = lane & 31, h = lane >> 5;
-        for (int u = 0; u < nk; ++u) {
-            // slot (u - 1) % LR: its reads fed the previous step's MFMAs
-            issue(g0 + min(u + LR - 1, nk - 1), (u + LR - 1) % LR);
+        // Group u.  COPY also requests group u + LR - 1 into the slot of u - 1,
+        // whose reads fed the previous step's MFMAs; LEFT is the number of
+        // groups that may still be in flight once u + 1 has landed.
+        auto step = [&](int u, auto copy, auto left) {
+            if constexpr (decltype(copy)::value) issue(g0 + u + LR - 1, (u + LR - 1) % LR);
             const int8_t* src = ring + (u % LR) * LSLOT;
             // MFMA step q takes chunk 2q + h of each lane's row, for A and B alike
             i32x4 af[4], bf[4];
@@ -123,9 +163,15 @@ __global__ __launch_bounds__(64 * KS) void gemm_i8_stream_kernel(
 #pragma unroll
             for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(af[q], bf[q], acc, 0, 0, 0);
             // group u + 1 has landed
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((LR - 2) * COPIES) : "memory");
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(left)::value * COPIES) : "memory");
+        };
+        // The last LR - 1 groups copy nothing (see the tile kernel's loop).
+        static_assert(LR == 4, "the steps after the loop");
+        int u = 0;
+        for (; u < nk - (LR - 1); ++u) step(u, std::true_type{}, std::integral_constant<int, LR - 2>{});
+        if (u < nk - 2) step(u++, std::false_type{}, std::integral_constant<int, 1>{});
+        if (u < nk - 1) step(u++, std::false_type{}, std::integral_constant<int, 0>{});
+        step(u, std::false_type{}, std::integral_constant<int, 0>{});
     }
     if constexpr (KS > 1) {
         // the rings are drained: once every wave is past its K loop their
@@ -139,38 +185,6 @@ __global__ __launch_bounds__(64 * KS) void gemm_i8_stream_kernel(
         for (int w = 0; w < KS - 1; ++w) acc += red[w * 64 + lane];
     }
 
-    // Accumulator v of lane l is C[rbase + 8 (v / 4) + v % 4][n0 + l % 32].
-    // Every operand the stores need (scales, bias, residual; clamped
-    // indices) is gathered first and consumed once in straight-line code:
-    // loaded inside the branchy store loop, each would wait for all earlier
-    // stores (vmcnt counts stores, and C may alias them).
-    const int cbase = n0 + (lane & 31);
-    const int rbase = m0 + 4 * (lane >> 5);
-    constexpr bool ROUTE = EPI == kEpiQKVRoute;
-    constexpr bool HAS_BIAS =
-        EPI == IE_EPI_BIAS || EPI == IE_EPI_BIAS_GELU || EPI == IE_EPI_BIAS_RESIDUAL || ROUTE;
-    constexpr bool HAS_RES = EPI == IE_EPI_BIAS_RESIDUAL;
-    float sa[16] = {}, sb = 0.0f, bv = 0.0f, rv[16] = {};
-    int slot[ROUTE ? 16 : 1] = {};
-    if constexpr (EPI != IE_EPI_I32) {
-        const int n = min(cbase, N - 1);
-        sb = sB[n];
-        if constexpr (HAS_BIAS) bv = bias[n];
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int m = min(rbase + 8 * (v >> 2) + (v & 3), M - 1);
-            sa[v] = sA[m];
-            if constexpr (HAS_RES) rv[v] = residual[(size_t)m * N + n];
-            if constexpr (ROUTE) slot[v] = route.row_slot[m];
-        }
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            asm volatile("" ::"v"(sa[v]));
-            if constexpr (HAS_RES) asm volatile("" ::"v"(rv[v]));
-        }
-        asm volatile("" ::"v"(sb));
-        if constexpr (HAS_BIAS) asm volatile("" ::"v"(bv));
-    }
     if (cbase < N) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
