@@ -33,13 +33,15 @@ namespace ie {
 // scale; 4.0e-8 -> 2.9e-8 and 1.3e-8 -> 1.0e-8 at 0.25 and 8), largest error 1.2e-7
 // -> 7.3e-8 of |v|.  From 2^60 on the step is skipped (infinity times its
 // reciprocal 0 is a NaN): v past the exponential's range gives -0, as before.
+// So it is where the quotient is infinite (infinity less infinity is one too):
+// +infinity gives itself and -infinity a NaN, as -infinity (1 + tanh u) does.
 __device__ __forceinline__ float gelu_tanh(float v) {
     // -2 log2(e) 0.7978845608 = -2.302208198
     const float e = __builtin_amdgcn_exp2f(-2.302208198f * fmaf(0.044715f, v * v * v, v));
     const float d = 1.0f + e, lo = fminf(1.0f, e) - (d - fmaxf(1.0f, e));  // 1 + e = d + lo exactly
     const float r = __builtin_amdgcn_rcpf(d), q = v * r;
     const float q2 = fmaf(fmaf(-lo, q, fmaf(-d, q, v)), r, q);
-    return d < 0x1p60f ? q2 : q;
+    return d < 0x1p60f && fabsf(q) < INFINITY ? q2 : q;
 }
 
 // The epilogue value for a float output, from the bias and residual values.

@@ -210,6 +210,23 @@ def test_gelu_epilogue_range(ie, M):
     assert (np.abs(got - want) <= 2.7 * 2.0 ** -24 * np.abs(d) + 2.0 ** -149).all()
 
 
+# Infinities and NaNs through the GELU of every GEMM family (decode, small-grid, LDS tiles, register-staged): from the
+# bias, and from a product whose scale overflows.  As the oracle's tanh form: +inf stays, -inf and NaN give NaN.
+@pytest.mark.parametrize("M,K", [(1, 768), (3, 256), (16, 768), (16, 4096), (40, 768), (40, 60), (600, 768), (600, 100)])
+def test_gelu_epilogue_infinities(ie, orc, M, K):
+    N = 900
+    A, W = np.ones((M, K), np.int8), np.ones((N, K), np.int8)
+    W[5] = -1
+    sA, sB, bias = np.ones(M, np.float32), np.full(N, 1e-3, np.float32), np.zeros(N, np.float32)
+    bias[[0, 1, 2, 3, 4]] = [np.inf, -np.inf, np.nan, 3.4e38, -3.4e38]
+    sB[[5, 6]] = np.inf  # -inf and inf out of the product itself
+    got = ie.int8_gemm(_dev(pack_i8(A)), _dev(pack_i8(W)), _dev(sA), _dev(sB), ie.EPI_BIAS_GELU,
+                       _dev(bias)).cpu().numpy()
+    want = orc.gemm(pack_i8(A), pack_i8(W), sA, sB, ie.EPI_BIAS_GELU, bias, None)
+    assert np.isposinf(want[:, [0, 6]]).all() and np.isnan(want[:, [1, 2, 5]]).all()
+    assert np.allclose(got, want, rtol=2e-6, atol=1e-7, equal_nan=True)
+
+
 # The 64 x 64 and 128 x 64 LDS tiles: fewer stages than the ring (one to three of 128), as many, more, and a tail; one
 # workgroup per CU, two, up to three, and past each (256 units; partial tiles both ways).
 @pytest.mark.parametrize("K", [128, 256, 272, 384, 512, 1296, 2064])
