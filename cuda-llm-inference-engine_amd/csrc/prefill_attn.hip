@@ -28,7 +28,8 @@
 // sixteenth of the bf16 one, so here the two products run on
 // v_mfma_f32_16x16x32_bf16 with every fp32 operand written as the sum of three
 // bf16 (each rounded to nearest even, 8 bits apiece, so the sum is the fp32
-// value): six of the nine partial products (those down to 2^-16 of the
+// value; V and the weights are scaled for it, keys below 2^-110 lose less
+// than 2^-133, see load_query): six of the nine partial products (those down to 2^-16 of the
 // largest; the rest are below 2^-24 of it) accumulate in fp32.  A bf16 cache is
 // exact in one part and takes three.  Error against 64 bits: about half the
 // fp32 kernel's over d, keys and caches (flash 2048 x 128 1.9e-7 against
@@ -41,10 +42,11 @@
 //     a block or group without keys changes nothing;
 //   * scores are pre-multiplied by log2(e)/sqrt(d) (folded into q, as in the
 //     fp32 kernel), so the softmax uses the hardware exp2.
-// An operand that is infinite, NaN or rounds to an infinite bf16 has no
-// three-part form and makes NaN: a tile whose outputs are not all finite is
-// computed again with fp32 MFMAs (exact_tile), which gives what the operands'
-// own arithmetic gives.
+// An operand that is infinite, NaN or too large for its (scaled) parts makes
+// NaN, and a query may be too small or too large for its own (load_query): a
+// tile with such a query or whose outputs are not all finite is computed again
+// with fp32 MFMAs (exact_tile), which gives what the operands' own arithmetic
+// gives.
 //
 // Which family: a paged launch by the cache type alone (bf16: the three-part
 // kernels), so a query's bits never depend on the batch or on how a prompt is
@@ -340,9 +342,12 @@ __device__ __forceinline__ uint32_t round_pair(float x0, float x1) {
     typedef float f32x2 __attribute__((ext_vector_type(2)));
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x0, x1}), bf16x2));
 }
-__device__ __forceinline__ void split_pair(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
-    h = round_pair(x0, x1);
-    const float r0 = x0 - __builtin_bit_cast(float, h << 16), r1 = x1 - __builtin_bit_cast(float, h & 0xffff0000u);
+// The parts of x0 s and x1 s, what the first leaves taken from the unrounded
+// product.
+__device__ __forceinline__ void split_pair(float x0, float x1, float s, uint32_t& h, uint32_t& m, uint32_t& l) {
+    h = round_pair(x0 * s, x1 * s);
+    const float r0 = fmaf(x0, s, -__builtin_bit_cast(float, h << 16));
+    const float r1 = fmaf(x1, s, -__builtin_bit_cast(float, h & 0xffff0000u));
     m = round_pair(r0, r1);
     l = round_pair(r0 - __builtin_bit_cast(float, m << 16), r1 - __builtin_bit_cast(float, m & 0xffff0000u));
 }
@@ -355,12 +360,21 @@ struct Parts {
 template <typename KV>
 constexpr int kParts = sizeof(KV) == 4 ? 3 : 1;
 
-__device__ __forceinline__ Parts<3> split8(const float (&x)[8]) {
+// The weights and the fp32 values of V are split times 2^24 (exact), so that no
+// part of a normal weight or of any value is below bf16's range; the output
+// is divided by both.  (Unscaled, values below 1e-34 lost their third part and
+// those below 1e-36 more than 1e-5 of themselves; 1 x 16 x 2048 x 128 125.6 -> 128.7 us
+// for the multiplications, ordinary operands' bits unchanged.)
+constexpr float kUp = 0x1p24f;
+template <typename KV>
+constexpr float kDown = sizeof(KV) == 4 ? 0x1p-48f : 0x1p-24f;  // (a bf16 value is one part as it is)
+
+__device__ __forceinline__ Parts<3> split8(const float (&x)[8], float s = 1.0f) {
     Parts<3> r;
-    split_pair(x[0], x[1], r.p[0].x, r.p[1].x, r.p[2].x);
-    split_pair(x[2], x[3], r.p[0].y, r.p[1].y, r.p[2].y);
-    split_pair(x[4], x[5], r.p[0].z, r.p[1].z, r.p[2].z);
-    split_pair(x[6], x[7], r.p[0].w, r.p[1].w, r.p[2].w);
+    split_pair(x[0], x[1], s, r.p[0].x, r.p[1].x, r.p[2].x);
+    split_pair(x[2], x[3], s, r.p[0].y, r.p[1].y, r.p[2].y);
+    split_pair(x[4], x[5], s, r.p[0].z, r.p[1].z, r.p[2].z);
+    split_pair(x[6], x[7], s, r.p[0].w, r.p[1].w, r.p[2].w);
     return r;
 }
 
@@ -461,7 +475,7 @@ __device__ __forceinline__ void attend(GetV&& val, const float (&sc)[8], Group<D
 #pragma unroll
         for (int t = 0; t < D / 16; ++t) gr.o[t] *= alpha;
     }
-    const Parts<3> pp = split8(p);
+    const Parts<3> pp = split8(p, kUp);
     // four tiles side by side, so that an accumulator's MFMAs are not back to back
 #pragma unroll
     for (int t0 = 0; t0 < D / 16; t0 += 4) {
@@ -582,16 +596,24 @@ __device__ __forceinline__ void exact_tile(const Where<D, KV, LAYOUT, BS16>& w, 
     }
 }
 
+// The query's operand; whether one of the lane's elements has no three-part
+// form that serves: a non-zero one below 2^-98 (2^-102 with qscale, about 1/8),
+// whose parts bf16 may not hold (what they lose is below 2^-133 and counts
+// beside keys of 2^64 and more), or one from 2^64 on, beside which what tiny
+// keys lose counts.
 template <int D>
-__device__ __forceinline__ void load_query(const float* row, float qscale, int g, Parts<3> (&q)[D / 32]) {
+__device__ __forceinline__ bool load_query(const float* row, float qscale, int g, Parts<3> (&q)[D / 32]) {
+    bool bad = false;
 #pragma unroll
     for (int s = 0; s < D / 32; ++s) {
         const float4 a = *reinterpret_cast<const float4*>(row + 32 * s + 8 * g);
         const float4 b = *reinterpret_cast<const float4*>(row + 32 * s + 8 * g + 4);
-        const float x[8] = {a.x * qscale, a.y * qscale, a.z * qscale, a.w * qscale,
-                            b.x * qscale, b.y * qscale, b.z * qscale, b.w * qscale};
-        q[s] = split8(x);
+        const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) bad |= x[e] != 0.0f && !(fabsf(x[e]) >= 0x1p-98f && fabsf(x[e]) < 0x1p64f);
+        q[s] = split8(x, qscale);
     }
+    return bad;
 }
 
 // Rows of a block's keys for a lane.  With 16-token pages and contiguous rows
@@ -697,8 +719,8 @@ __global__ __launch_bounds__(256 * GW, D == 64 && GW == 1 ? 3 : 2) void prefill_
         for (int d = 0; d < VE; ++d) {
             uint2 s[NP];
             if constexpr (NP == 3) {
-                split_pair(elem<KV>(vr[0], d), elem<KV>(vr[1], d), s[0].x, s[1].x, s[2].x);
-                split_pair(elem<KV>(vr[2], d), elem<KV>(vr[3], d), s[0].y, s[1].y, s[2].y);
+                split_pair(elem<KV>(vr[0], d), elem<KV>(vr[1], d), kUp, s[0].x, s[1].x, s[2].x);
+                split_pair(elem<KV>(vr[2], d), elem<KV>(vr[3], d), kUp, s[0].y, s[1].y, s[2].y);
             } else {
                 s[0] = make_uint2(pair_bf16(vr[0][d / 2], vr[1][d / 2], d & 1), pair_bf16(vr[2][d / 2], vr[3][d / 2], d & 1));
             }
@@ -716,7 +738,7 @@ __global__ __launch_bounds__(256 * GW, D == 64 && GW == 1 ? 3 : 2) void prefill_
 #pragma unroll
     for (int k = 0; k < PER; ++k) iters += steps(k);
     Parts<3> q[D / 32];
-    load_query<D>(Q + w.qrow(qi), qscale, g, q);
+    const bool qbad = load_query<D>(Q + w.qrow(qi), qscale, g, q);
     Group<D> gr, tot;
     gr.clear();
     tot.clear();
@@ -797,8 +819,8 @@ __global__ __launch_bounds__(256 * GW, D == 64 && GW == 1 ? 3 : 2) void prefill_
     }
     }
 
-    const float inv = tot.l > 0.0f ? 1.0f / tot.l : 0.0f;
-    float bad = 0.0f;
+    const float inv = tot.l > 0.0f ? 1.0f / tot.l * kDown<KV> : 0.0f;
+    float bad = qbad ? 1.0f : 0.0f;
 #pragma unroll
     for (int t = 0; t < TT; ++t)
 #pragma unroll
@@ -806,7 +828,7 @@ __global__ __launch_bounds__(256 * GW, D == 64 && GW == 1 ? 3 : 2) void prefill_
             tot.o[t][v] *= inv;
             bad = fmaf(tot.o[t][v], 0.0f, bad);
         }
-    if (__ballot(!(bad == 0.0f))) {  // uniform: not all finite
+    if (__ballot(!(bad == 0.0f))) {  // uniform: not all finite, or a query without parts
         exact_tile(w, qw, qscale);
     } else if (qw + i < P) {
         float* out = O + w.qrow(qi) + 4 * g;
@@ -862,7 +884,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void prefill_split_kernel(
         load_v(c0);
     }
     Parts<3> q[D / 32];
-    load_query<D>(Q + w.qrow(qi), qscale, g, q);
+    const bool qbad = load_query<D>(Q + w.qrow(qi), qscale, g, q);
     while (c0 < kend) {
         const int cn = c0 + kGroups * kKB;
         float sc[8];
@@ -873,7 +895,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void prefill_split_kernel(
                 if constexpr (NP == 3) {
                     const float x[8] = {elem<KV>(vr[0], t), elem<KV>(vr[1], t), elem<KV>(vr[2], t), elem<KV>(vr[3], t),
                                         elem<KV>(vr[4], t), elem<KV>(vr[5], t), elem<KV>(vr[6], t), elem<KV>(vr[7], t)};
-                    return split8(x);
+                    return split8(x, kUp);
                 } else {
                     auto pair = [&](int e) { return pair_bf16(vr[e][t / 2], vr[e + 1][t / 2], t & 1); };
                     return Parts<1>{{make_uint4(pair(0), pair(2), pair(4), pair(6))}};
@@ -907,8 +929,8 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void prefill_split_kernel(
 #pragma unroll
         for (int e = 0; e < PER; ++e) x[e] = merge_value(x[e], sm_o[k][qq][col + e], a, b);
     }
-    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-    float bad = 0.0f;
+    const float inv = L > 0.0f ? 1.0f / L * kDown<KV> : 0.0f;
+    float bad = qbad ? 1.0f : 0.0f;
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
         x[e] *= inv;

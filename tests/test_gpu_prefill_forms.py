@@ -112,3 +112,75 @@ def test_paged_bf16_infinite_value(ie):
     assert np.isfinite(got[:48]).all() and np.isfinite(got[64:, 1]).all()
     kept = np.delete(got[53:, 0], 8, axis=1)
     assert np.isfinite(kept).all()
+
+
+FORM_SHAPES = {"split": (1, 1, 800), "tile1": (2, 64, 250), "tile2": (1, 24, 780)}
+
+
+def attention64(q, k, v, causal):
+    """softmax(q k^T / sqrt(d)) v per (b, h) on the CPU in 64 bits."""
+    import torch
+
+    q, k, v = (x.double() for x in (q, k, v))
+    s = q @ k.transpose(-1, -2) / q.shape[-1] ** 0.5
+    if causal:
+        s = s.masked_fill(~torch.ones(s.shape[-2:], dtype=torch.bool).tril(), -float("inf"))
+    return torch.softmax(s, dim=-1) @ v
+
+
+# Operands far from 1, whose bf16 parts could fall below bf16's range (2^-133) or pass it: V at the smallest normal
+# numbers and among the subnormals, at both ends of the range, Q and K of sizes that offset each other.  The bar is
+# the other tests'; subnormal results have 2^-149 of their own.
+@pytest.mark.parametrize("shape", sorted(FORM_SHAPES))
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("qs,ks,vs", [(1, 1, 1e-33), (1, 1, 1e-36), (1, 1, 2.0 ** -126), (1, 1, 2.0 ** -135),
+                                      (1, 1, 1e25), (1, 1, 1e37), (1e37, 1e-37, 1), (1e-37, 1e37, 1e-20),
+                                      (1e36, 1e-36, 1e-36)])
+def test_flash_operand_sizes(ie, d, shape, qs, ks, vs):
+    import torch
+
+    B, H, N = FORM_SHAPES[shape]
+    g = torch.Generator().manual_seed(d + N)
+    Q, K, V = (torch.randn(B, H, N, d, generator=g) * s for s in (qs, ks, vs))
+    got = ie.flash_attn(Q.cuda(), K.cuda(), V.cuda(), causal=True).cpu().double()
+    for h in {0, H - 1}:
+        want = attention64(Q[0, h], K[0, h], V[0, h], True)
+        assert ((got[0, h] - want).abs() <= REL * want.abs().max() + 2.0 ** -149).all()
+
+
+# Weights near the smallest normal number on values as much larger than the others': the small weights' own bits
+# count.  The score of about -125 (in powers of two) has three roundings, each moving its weight by up to 125 x 2^-24 ln 2.
+@pytest.mark.parametrize("shape", sorted(FORM_SHAPES))
+@pytest.mark.parametrize("d", [64, 128])
+def test_flash_tiny_weights(ie, d, shape):
+    import torch
+
+    B, H, N = FORM_SHAPES[shape]
+    g = torch.Generator().manual_seed(d + N)
+    Q, K = torch.zeros(B, H, N, d), torch.zeros(B, H, N, d)
+    Q[..., 0] = 1.0
+    K[..., 3, 0] = -125 * d ** 0.5 * 0.6931471805599453
+    V = (1.0 + torch.rand(B, H, N, d, generator=g)) * 2.0 ** -64
+    V[:, :, 3] = (1.0 + torch.rand(B, H, d, generator=g)) * 2.0 ** 75
+    got = ie.flash_attn(Q.cuda(), K.cuda(), V.cuda(), causal=False).cpu().double()
+    want = attention64(Q[0, 0], K[0, 0], V[0, 0], False)
+    assert (want > 4 * 2.0 ** -64).all()  # the one key's share is the larger part
+    assert ((got[0, 0] - want).abs() <= (3 * 125 * 2.0 ** -24 + REL) * want).all()
+
+
+@pytest.mark.parametrize("qs,ks,vs", [(1e-37, 1e37, 1), (1e36, 1e-36, 1), (1, 1, 2.0 ** -130), (1, 1, 1e37)])
+@pytest.mark.parametrize("P,H", [(70, 2), (100, 170)])  # the split kernel, the tile kernel
+def test_paged_bf16_operand_sizes(ie, P, H, qs, ks, vs):
+    import torch
+
+    d, bs = 64, 16
+    nb = (P + bs - 1) // bs
+    g = torch.Generator().manual_seed(P)
+    Q = torch.randn(1, P, H, d, generator=g) * qs
+    K, V = ((torch.randn(nb, bs, H, d, generator=g) * s).to(torch.bfloat16) for s in (ks, vs))
+    table = torch.arange(nb, dtype=torch.int32).view(1, nb)
+    got = ie.prefill_attn(Q.cuda(), K.cuda(), V.cuda(), table.cuda(), 0, bs, H, kv_dtype=ie.KV_BF16).cpu().double()
+    for h in {0, H - 1}:
+        k, v = (x.view(-1, H, d)[:P, h].float() for x in (K, V))
+        want = attention64(Q[0, :, h], k, v, True)
+        assert ((got[0, :, h] - want).abs() <= REL * want.abs().max() + 2.0 ** -149).all()
