@@ -603,15 +603,27 @@ __device__ __forceinline__ void exact_tile(const Where<D, KV, LAYOUT, BS16>& w, 
 // keys lose counts.
 template <int D>
 __device__ __forceinline__ bool load_query(const float* row, float qscale, int g, Parts<3> (&q)[D / 32]) {
-    bool bad = false;
+    float x[D / 32][8], lo = INFINITY, hi = 0.0f;
 #pragma unroll
     for (int s = 0; s < D / 32; ++s) {
         const float4 a = *reinterpret_cast<const float4*>(row + 32 * s + 8 * g);
         const float4 b = *reinterpret_cast<const float4*>(row + 32 * s + 8 * g + 4);
-        const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        const float y[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
-        for (int e = 0; e < 8; ++e) bad |= x[e] != 0.0f && !(fabsf(x[e]) >= 0x1p-98f && fabsf(x[e]) < 0x1p64f);
-        q[s] = split8(x, qscale);
+        for (int e = 0; e < 8; ++e) {
+            x[s][e] = y[e];
+            lo = fminf(lo, fabsf(y[e]));
+            hi = fmaxf(hi, fabsf(y[e]));
+        }
+        q[s] = split8(x[s], qscale);
+    }
+    bool bad = false;
+    if (__ballot(lo < 0x1p-98f || hi >= 0x1p64f)) {  // (uniform; seldom, zeros among them)
+#pragma unroll
+        for (int s = 0; s < D / 32; ++s)
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                bad |= x[s][e] != 0.0f && !(fabsf(x[s][e]) >= 0x1p-98f && fabsf(x[s][e]) < 0x1p64f);
     }
     return bad;
 }
