@@ -43,14 +43,17 @@
 //   * scores are pre-multiplied by log2(e)/sqrt(d) (folded into q, as in the
 //     fp32 kernel), so the softmax uses the hardware exp2.
 // An operand that is infinite, NaN or too large for its (scaled) parts makes
-// NaN, and a query may be too small or too large for its own (load_query): a
-// tile with such a query or whose outputs are not all finite is computed again
-// with fp32 MFMAs (exact_tile), which gives what the operands' own arithmetic
-// gives.
+// NaN, and a query may be too small or too large for its own (load_query): the
+// queries of a tile whose outputs are not all finite, and such queries, are
+// computed again with fp32 MFMAs (exact_tile), which gives what the operands'
+// own arithmetic gives; the tile's others keep their bits.
 //
 // Which family: a paged launch by the cache type alone (bf16: the three-part
-// kernels), so a query's bits never depend on the batch or on how a prompt is
-// chunked; a contiguous one by its shape (prefill_form).
+// kernels), so the bits of a finite result never depend on the batch or on how
+// a prompt is chunked; a contiguous one by its shape (prefill_form).  (An infinite or
+// NaN value of V at a key that a query does not see can still reach it, 0 times it
+// being a NaN: in the fp32 MFMAs from the keys of its own 16 queries.  Such a
+// query is computed again, or is itself a NaN, as its tile lies.)
 //
 // In the three-part kernels a wave owns 16 queries of one (b, h).  Operands
 // (lane l: i = l % 16, g = l / 16): S^T = K Q^T, 16 keys x 16 queries per MFMA, leaves lane l with query i and
@@ -560,9 +563,11 @@ __device__ __forceinline__ Where<D, KV, LAYOUT, BS16> locate(const float* Q, con
 }
 
 // 16 queries from q0 on with fp32 MFMAs, one wave over all their keys: the
-// form for operands that have no three-part one.
+// form for operands that have no three-part one.  Writes those of `rows` (bit
+// i: query q0 + i).
 template <int D, typename KV, int LAYOUT, bool BS16>
-__device__ __forceinline__ void exact_tile(const Where<D, KV, LAYOUT, BS16>& w, int q0, float qscale) {
+__device__ __forceinline__ void exact_tile(const Where<D, KV, LAYOUT, BS16>& w, int q0, float qscale,
+                                           uint32_t rows) {
     if (q0 >= w.P) return;
     const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
     const int qi = min(q0 + i, w.P - 1);
@@ -587,13 +592,19 @@ __device__ __forceinline__ void exact_tile(const Where<D, KV, LAYOUT, BS16>& w, 
         consume(c, c0, g, q, klim, m, l, o);
     }
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-    if (q0 + i < w.P) {
+    if (q0 + i < w.P && (rows >> i & 1)) {
         float* out = w.O + w.qrow(qi);
 #pragma unroll
         for (int t = 0; t < D / 16; ++t)
 #pragma unroll
             for (int v = 0; v < 4; ++v) out[(D / 16) * (4 * g + v) + t] = o[t][v] * inv;
     }
+}
+
+// The queries (bit i) that have a lane (i, g) among `lanes`.
+__device__ __forceinline__ uint32_t query_rows(uint64_t lanes) {
+    const uint32_t x = (uint32_t)lanes | (uint32_t)(lanes >> 32);
+    return (x | x >> 16) & 0xffffu;
 }
 
 // The query's operand; whether one of the lane's elements has no three-part
@@ -840,14 +851,14 @@ __global__ __launch_bounds__(256 * GW, D == 64 && GW == 1 ? 3 : 2) void prefill_
             tot.o[t][v] *= inv;
             bad = fmaf(tot.o[t][v], 0.0f, bad);
         }
-    if (__ballot(!(bad == 0.0f))) {  // uniform: not all finite, or a query without parts
-        exact_tile(w, qw, qscale);
-    } else if (qw + i < P) {
+    const uint32_t rows = query_rows(__ballot(!(bad == 0.0f)));  // not all finite, or without parts
+    if (qw + i < P && !(rows >> i & 1)) {
         float* out = O + w.qrow(qi) + 4 * g;
 #pragma unroll
         for (int t = 0; t < TT; ++t)
             *reinterpret_cast<float4*>(out + 16 * t) = make_float4(tot.o[t][0], tot.o[t][1], tot.o[t][2], tot.o[t][3]);
     }
+    if (rows) exact_tile(w, qw, qscale, rows);
 }
 
 template <int D, typename KV, int LAYOUT, bool BS16>
@@ -942,21 +953,24 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void prefill_split_kernel(
         for (int e = 0; e < PER; ++e) x[e] = merge_value(x[e], sm_o[k][qq][col + e], a, b);
     }
     const float inv = L > 0.0f ? 1.0f / L * kDown<KV> : 0.0f;
-    float bad = qbad ? 1.0f : 0.0f;
+    float bad = 0.0f;
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
         x[e] *= inv;
         bad = fmaf(x[e], 0.0f, bad);
     }
-    if (__syncthreads_or(!(bad == 0.0f))) {
-        if (wave == 0) exact_tile(w, q0, qscale);
-        return;
-    }
-    if (q0 + qq < P) {
+    // of this wave's four queries (16 lanes each): not all finite, or without parts
+    const uint64_t lanes = __ballot(!(bad == 0.0f));
+    uint32_t rows = query_rows(__ballot(qbad)) & (0xfu << (4 * wave));
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        if (lanes >> (16 * k) & 0xffff) rows |= 1u << (4 * wave + k);
+    if (q0 + qq < P && !(rows >> qq & 1)) {
         float* out = O + w.qrow(q0 + qq) + col;
 #pragma unroll
         for (int e = 0; e < PER; e += 4) *reinterpret_cast<float4*>(out + e) = make_float4(x[e], x[e + 1], x[e + 2], x[e + 3]);
     }
+    if (rows) exact_tile(w, q0, qscale, rows);
 }
 
 enum PrefillForm { kFp32, kSplit, kTile1, kTile2 };

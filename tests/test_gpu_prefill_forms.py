@@ -184,3 +184,36 @@ def test_paged_bf16_operand_sizes(ie, P, H, qs, ks, vs):
         k, v = (x.view(-1, H, d)[:P, h].float() for x in (K, V))
         want = attention64(Q[0, :, h], k, v, True)
         assert ((got[0, :, h] - want).abs() <= REL * want.abs().max() + 2.0 ** -149).all()
+
+
+# Queries that are computed again (they see an infinite key, or are themselves too small for three parts) and the others
+# of their tiles: those keep the bits that they have in any other chunk of the prompt.
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("H", [2, 170])  # the split kernel, the tile kernel for the whole prompt
+def test_paged_bf16_queries_beside_one_computed_again(ie, d, H):
+    import torch
+
+    P, bs = 100, 16
+    Q, kc, vc, table = case(3 * H + d, 1, P, 0, H, 1, d, bs, 1)
+    plain = host(ie.prefill_attn(dev(Q), dev(kc), dev(vc), dev(table), 0, bs, H, kv_dtype=ie.KV_BF16))[0]
+    kc = kc.copy()
+    kc[int(table[0, 40 // bs]), 40 % bs, 0, 4] = 0x7F80  # position 40, head 0: inf
+    Q = Q.copy()
+    Q[0, 70, 1] *= 1e-33
+    Q[0, 5, 1, 3] = 1e-38
+    kd, vd, td = dev(kc), dev(vc), dev(table)
+    for chunks in ((0, P), (0, 33, P), (0, 41, 71, P), (0, 7, 35, 60, P)):
+        got = np.concatenate([host(ie.prefill_attn(dev(Q[:, a:b]), kd, vd, td, a, bs, H, kv_dtype=ie.KV_BF16))[0]
+                              for a, b in zip(chunks, chunks[1:])])
+        assert np.array_equal(got[:40, 0], plain[:40, 0]), chunks
+        assert not np.isfinite(got[40:, 0]).all()
+        same = np.delete(np.arange(P), [5, 70])
+        assert np.array_equal(got[same, 1], plain[same, 1]), chunks
+        # the small queries: (almost) equal weights
+        k, v = (torch.from_numpy(x.astype(np.int32) << 16).view(torch.float32)[table[0]].reshape(-1, H, d)[:, 1].double()
+                for x in (kc, vc))
+        for t in (5, 70):
+            w = torch.softmax(k[:t + 1] @ torch.from_numpy(Q[0, t, 1]).double() / d ** 0.5, 0)
+            want = (w @ v[:t + 1]).numpy()
+            assert np.abs(got[t, 1] - want).max() <= REL * np.abs(want).max()
+        assert np.array_equal(got[:, 2:], plain[:, 2:])
