@@ -29,7 +29,7 @@
 // v_mfma_f32_16x16x32_bf16 with every fp32 operand written as the sum of three
 // bf16 (each rounded to nearest even, 8 bits apiece, so the sum is the fp32
 // value; V and the weights are scaled for it, keys below 2^-110 lose less
-// than 2^-133, see load_query): six of the nine partial products (those down to 2^-16 of the
+// than 2^-133, see split_query): six of the nine partial products (those down to 2^-16 of the
 // largest; the rest are below 2^-24 of it) accumulate in fp32.  A bf16 cache is
 // exact in one part and takes three.  Error against 64 bits: about half the
 // fp32 kernel's over d, keys and caches (flash 2048 x 128 1.9e-7 against
@@ -43,7 +43,7 @@
 //   * scores are pre-multiplied by log2(e)/sqrt(d) (folded into q, as in the
 //     fp32 kernel), so the softmax uses the hardware exp2.
 // An operand that is infinite, NaN or too large for its (scaled) parts makes
-// NaN, and a query may be too small or too large for its own (load_query): the
+// NaN, and a query may be too small or too large for its own (split_query): the
 // queries of a tile whose outputs are not all finite, and such queries, are
 // computed again with fp32 MFMAs (exact_tile), which gives what the operands'
 // own arithmetic gives; the tile's others keep their bits.
@@ -607,24 +607,33 @@ __device__ __forceinline__ uint32_t query_rows(uint64_t lanes) {
     return (x | x >> 16) & 0xffffu;
 }
 
-// The query's operand; whether one of the lane's elements has no three-part
-// form that serves: a non-zero one below 2^-98 (2^-102 with qscale, about 1/8),
-// whose parts bf16 may not hold (what they lose is below 2^-133 and counts
-// beside keys of 2^64 and more), or one from 2^64 on, beside which what tiny
-// keys lose counts.
+// A lane's share of its query's row: elements 32 s + 8 g on.
 template <int D>
-__device__ __forceinline__ bool load_query(const float* row, float qscale, int g, Parts<3> (&q)[D / 32]) {
-    float x[D / 32][8], lo = INFINITY, hi = 0.0f;
+__device__ __forceinline__ void load_query(const float* row, int g, float (&x)[D / 32][8]) {
 #pragma unroll
     for (int s = 0; s < D / 32; ++s) {
         const float4 a = *reinterpret_cast<const float4*>(row + 32 * s + 8 * g);
         const float4 b = *reinterpret_cast<const float4*>(row + 32 * s + 8 * g + 4);
         const float y[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
+        for (int e = 0; e < 8; ++e) x[s][e] = y[e];
+    }
+}
+
+// The query's operand; whether one of the lane's elements has no three-part
+// form that serves: a non-zero one below 2^-98 (2^-102 with qscale, about 1/8),
+// whose parts bf16 may not hold (what they lose is below 2^-133 and counts
+// beside keys of 2^64 and more), or one from 2^64 on, beside which what tiny
+// keys lose counts.
+template <int D>
+__device__ __forceinline__ bool split_query(const float (&x)[D / 32][8], float qscale, Parts<3> (&q)[D / 32]) {
+    float lo = INFINITY, hi = 0.0f;
+#pragma unroll
+    for (int s = 0; s < D / 32; ++s) {
+#pragma unroll
         for (int e = 0; e < 8; ++e) {
-            x[s][e] = y[e];
-            lo = fminf(lo, fabsf(y[e]));
-            hi = fmaxf(hi, fabsf(y[e]));
+            lo = fminf(lo, fabsf(x[s][e]));
+            hi = fmaxf(hi, fabsf(x[s][e]));
         }
         q[s] = split8(x[s], qscale);
     }
@@ -755,13 +764,15 @@ __global__ __launch_bounds__(256 * GW, D == 64 && GW == 1 ? 3 : 2) void prefill_
     // These four waves' steps: groups PER hf .. PER hf + PER - 1, a block at a time.
     int grp = PER * hf, blk = grp;
     bool act = blk < nblk;
+    float qx[D / 32][8];
+    load_query<D>(Q + w.qrow(qi), g, qx);
     if (act) load(blk);
     auto steps = [&](int k) { return k < nblk ? (nblk - k + kGroups - 1) / kGroups : 0; };
     int iters = 0;  // (the second half has no more than the first)
 #pragma unroll
     for (int k = 0; k < PER; ++k) iters += steps(k);
     Parts<3> q[D / 32];
-    const bool qbad = load_query<D>(Q + w.qrow(qi), qscale, g, q);
+    const bool qbad = split_query<D>(qx, qscale, q);
     Group<D> gr, tot;
     gr.clear();
     tot.clear();
@@ -871,6 +882,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void prefill_split_kernel(
     constexpr int VW = D / 16 * (int)sizeof(KV) / 4;  // of d / 16
     __shared__ float sm_o[kGroups][kQW][D + 4];
     __shared__ float sm_m[kGroups][kQW], sm_l[kGroups][kQW];
+    __shared__ uint32_t sm_bad;  // queries without parts
     const int lane = threadIdx.x & 63, g = lane >> 4, i = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // its group
     const int ntiles = (P + kQW - 1) / kQW;
@@ -899,43 +911,47 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void prefill_split_kernel(
         for (int e = 0; e < 8; ++e) load_words(vb.at(e >> 2, 4 * g + (e & 3), D / 16 * i), vr[e]);
     };
 
-    Group<D> gr;
-    gr.clear();
-    int c0 = wave * kKB;
-    if (c0 < kend) {
+    // (a wave without blocks has nothing to do here; in one branch, so that no
+    // wait is for more than the path has issued)
+    if (int c0 = wave * kKB; c0 < kend) {
+        // the query first: it waits for no block table, and is split while the keys arrive
+        float qx[D / 32][8];
+        load_query<D>(Q + w.qrow(qi), g, qx);
         load_k(c0);
         load_v(c0);
-    }
-    Parts<3> q[D / 32];
-    const bool qbad = load_query<D>(Q + w.qrow(qi), qscale, g, q);
-    while (c0 < kend) {
-        const int cn = c0 + kGroups * kKB;
-        float sc[8];
-        scores<D, NP>([&](int j, int s) { return parts8<KV>(kr[j][s]); }, q, c0, klim, c0 + kKB > wlo, g, sc);
-        if (cn < kend) load_k(cn);
-        attend<D, NP>(
-            [&](int t) {
-                if constexpr (NP == 3) {
-                    const float x[8] = {elem<KV>(vr[0], t), elem<KV>(vr[1], t), elem<KV>(vr[2], t), elem<KV>(vr[3], t),
-                                        elem<KV>(vr[4], t), elem<KV>(vr[5], t), elem<KV>(vr[6], t), elem<KV>(vr[7], t)};
-                    return split8(x, kUp);
-                } else {
-                    auto pair = [&](int e) { return pair_bf16(vr[e][t / 2], vr[e + 1][t / 2], t & 1); };
-                    return Parts<1>{{make_uint4(pair(0), pair(2), pair(4), pair(6))}};
-                }
-            },
-            sc, gr);
-        if (cn < kend) load_v(cn);
-        c0 = cn;
-    }
-
+        Parts<3> q[D / 32];
+        const bool qbad = split_query<D>(qx, qscale, q);
+        if (wave == 0) sm_bad = query_rows(__ballot(qbad));  // (wave 0 has a block)
+        Group<D> gr;
+        gr.clear();
+        while (c0 < kend) {
+            const int cn = c0 + kGroups * kKB;
+            float sc[8];
+            scores<D, NP>([&](int j, int s) { return parts8<KV>(kr[j][s]); }, q, c0, klim, c0 + kKB > wlo, g, sc);
+            if (cn < kend) load_k(cn);
+            attend<D, NP>(
+                [&](int t) {
+                    if constexpr (NP == 3) {
+                        const float x[8] = {elem<KV>(vr[0], t), elem<KV>(vr[1], t), elem<KV>(vr[2], t), elem<KV>(vr[3], t),
+                                            elem<KV>(vr[4], t), elem<KV>(vr[5], t), elem<KV>(vr[6], t), elem<KV>(vr[7], t)};
+                        return split8(x, kUp);
+                    } else {
+                        auto pair = [&](int e) { return pair_bf16(vr[e][t / 2], vr[e + 1][t / 2], t & 1); };
+                        return Parts<1>{{make_uint4(pair(0), pair(2), pair(4), pair(6))}};
+                    }
+                },
+                sc, gr);
+            if (cn < kend) load_v(cn);
+            c0 = cn;
+        }
 #pragma unroll
-    for (int t = 0; t < D / 16; ++t)
+        for (int t = 0; t < D / 16; ++t)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) sm_o[wave][i][(D / 16) * (4 * g + v) + t] = gr.o[t][v];
-    if (g == 0) {
-        sm_m[wave][i] = gr.m;
-        sm_l[wave][i] = gr.l;
+            for (int v = 0; v < 4; ++v) sm_o[wave][i][(D / 16) * (4 * g + v) + t] = gr.o[t][v];
+        if (g == 0) {
+            sm_m[wave][i] = gr.m;
+            sm_l[wave][i] = gr.l;
+        }
     }
     __syncthreads();
 
@@ -946,6 +962,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void prefill_split_kernel(
     for (int e = 0; e < PER; ++e) x[e] = 0.0f;
 #pragma unroll
     for (int k = 0; k < kGroups; ++k) {
+        if (k * kKB >= kend) break;  // uniform: a group without blocks changes nothing
         float a, b;
         M = merge_weights(M, sm_m[k][qq], a, b);
         L = merge_value(L, sm_l[k][qq], a, b);
@@ -961,7 +978,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void prefill_split_kernel(
     }
     // of this wave's four queries (16 lanes each): not all finite, or without parts
     const uint64_t lanes = __ballot(!(bad == 0.0f));
-    uint32_t rows = query_rows(__ballot(qbad)) & (0xfu << (4 * wave));
+    uint32_t rows = __builtin_amdgcn_readfirstlane(sm_bad) & (0xfu << (4 * wave));
 #pragma unroll
     for (int k = 0; k < 4; ++k)
         if (lanes >> (16 * k) & 0xffff) rows |= 1u << (4 * wave + k);
