@@ -675,7 +675,7 @@ struct BlockRows {
             return base + map.off(min(c0 + 16 * j + r, kend - 1), 0) + elem;
         } else {
             const int pos = min(c0 + 16 * j, (kend - 1) & ~15);
-            // (16 rows of at most 65535 heads: below 2^32 bytes)
+            // (16 rows are at most 2^32 bytes: launch_d)
             const uint32_t ofs = ((uint32_t)min(r, kend - 1 - pos) * (uint32_t)map.stride + elem) * (uint32_t)sizeof(KV);
             return reinterpret_cast<const KV*>(reinterpret_cast<const char*>(j ? half1 : half0) + ofs);
         }
@@ -1048,8 +1048,10 @@ void launch_d(const PrefillArgs& a, hipStream_t s) {
         fp32 ? launch_fp32<D, 1, false>(a, s) : launch_t<D, float, 1, false>(a, s);
     else if (fp32)
         bs16 ? launch_fp32<D, 0, true>(a, s) : launch_fp32<D, 0, false>(a, s);
+    else if (bs16 && 16ull * a.H_kv * D * sizeof(uint16_t) <= 1ull << 32)  // BlockRows' 32-bit offsets
+        launch_t<D, uint16_t, 0, true>(a, s);
     else
-        bs16 ? launch_t<D, uint16_t, 0, true>(a, s) : launch_t<D, uint16_t, 0, false>(a, s);
+        launch_t<D, uint16_t, 0, false>(a, s);
 }
 
 }  // namespace

@@ -217,3 +217,29 @@ def test_paged_bf16_queries_beside_one_computed_again(ie, d, H):
             want = (w @ v[:t + 1]).numpy()
             assert np.abs(got[t, 1] - want).max() <= REL * np.abs(want).max()
         assert np.array_equal(got[:, 2:], plain[:, 2:])
+
+
+# 16 rows of a page past 4 GiB (2.24 million heads): 32-bit row offsets would wrap from the last row on.  A few heads
+# hold values, the others zeros; the split kernel (P = 16) and the tile kernel (17, a second page).
+@pytest.mark.parametrize("P", [16, 17])
+def test_paged_bf16_rows_past_4_gib(ie, P):
+    import torch
+
+    H, d, bs = 2_240_000, 64, 16
+    nb = (P + bs - 1) // bs
+    heads = torch.tensor([0, 1, H // 2 + 1, H - 1])
+    g = torch.Generator().manual_seed(P)
+    q = torch.randn(P, 4, d, generator=g)
+    k, v = (torch.randn(nb, bs, 4, d, generator=g).to(torch.bfloat16) for _ in range(2))
+    Q = torch.zeros(1, P, H, d, device="cuda")
+    K, V = (torch.zeros(nb, bs, H, d, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    Q[0][:, heads.cuda()] = q.cuda()
+    for big, small in ((K, k), (V, v)):
+        big[:, :, heads.cuda()] = small.cuda()
+    table = torch.arange(nb, dtype=torch.int32, device="cuda").view(1, nb)
+    got = ie.prefill_attn(Q, K, V, table, 0, bs, H, kv_dtype=ie.KV_BF16)[0][:, heads.cuda()].cpu().double()
+    del Q, K, V
+    torch.cuda.empty_cache()
+    for i in range(4):
+        want = attention64(q[:, i], *(x.reshape(-1, 4, d)[:P, i].float() for x in (k, v)), True)
+        assert (got[:, i] - want).abs().max() <= REL * want.abs().max()
