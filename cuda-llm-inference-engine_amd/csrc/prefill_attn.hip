@@ -140,13 +140,14 @@ struct Chunk {
 
 // Where token `pos` of the current (b, kv head) lives, in elements from the
 // head's base pointer.
-//   LAYOUT 0, BS16: paged with block size 16; `phys` is the chunk's block.
+//   LAYOUT 0, BS16: paged, blocks of `runs` whole runs of 16 tokens (the fp32
+//                   kernel: 1); `phys` is the chunk's run in the cache.
 //   LAYOUT 0:       paged, any block size (per-lane table lookup).
 //   LAYOUT 1:       contiguous rows.
 template <int LAYOUT, bool BS16>
 struct TokenMap {
     const int* bt;
-    int block_size;
+    int block_size, runs;
     size_t stride;  // elements between consecutive token rows of one head
     __device__ __forceinline__ size_t off(int pos, int phys) const {
         if constexpr (LAYOUT == 1) {
@@ -157,6 +158,14 @@ struct TokenMap {
             const int blk = pos / block_size;
             return ((size_t)bt[blk] * block_size + (pos - blk * block_size)) * stride;
         }
+    }
+    // the run that holds token pos (BS16; wave-uniform)
+    __device__ __forceinline__ int run_of(int pos) const {
+        const uint32_t r = (uint32_t)pos >> 4;
+        if (runs == 1) return bt[r];
+        // (a first block, in which a short prompt lies, without the division)
+        const uint32_t blk = r < (uint32_t)runs ? 0 : r / (uint32_t)runs;
+        return bt[blk] * runs + (int)(r - blk * (uint32_t)runs);
     }
 };
 
@@ -527,7 +536,7 @@ struct Where {
     // keys that queries up to qi need
     __device__ __forceinline__ int limit(int qi) const { return causal ? min(start + qi + 1, nkeys) : nkeys; }
     __device__ __forceinline__ int phys(int pos, int kend) const {
-        if constexpr (LAYOUT == 0 && BS16) return map.bt[min(pos, kend - 1) >> 4];
+        if constexpr (LAYOUT == 0 && BS16) return map.run_of(min(pos, kend - 1));
         else return 0;
     }
 };
@@ -542,6 +551,7 @@ __device__ __forceinline__ Where<D, KV, LAYOUT, BS16> locate(const float* Q, con
     if constexpr (LAYOUT == 0) {
         w.map.bt = block_table + (size_t)b * nbps;
         w.map.block_size = block_size;
+        w.map.runs = block_size >> 4;
         w.map.stride = (size_t)H_kv * D;
         w.kbase = kcache + (size_t)kvh * D;
         w.vbase = vcache + (size_t)kvh * D;
@@ -648,10 +658,10 @@ __device__ __forceinline__ bool split_query(const float (&x)[D / 32][8], float q
     return bad;
 }
 
-// Rows of a block's keys for a lane.  With 16-token pages and contiguous rows
-// key r of half j of a block at c0 lies at a uniform base (of the page, or of
-// the half) plus r rows, so an address is a scalar base plus a 32-bit lane
-// offset; other block sizes look each key up.  Keys at or past kend read the
+// Rows of a block's keys for a lane.  With pages of whole 16-token runs and
+// contiguous rows key r of half j of a block at c0 lies at a uniform base (of
+// the run, or of the half) plus r rows, so an address is a scalar base plus a
+// 32-bit lane offset; other block sizes look each key up.  Keys at or past kend read the
 // last one.
 template <typename KV, int LAYOUT, bool BS16>
 struct BlockRows {
@@ -666,7 +676,7 @@ struct BlockRows {
     }
     __device__ __forceinline__ const KV* start_of(int pos) const {
         if constexpr (LAYOUT == 1) return base + (size_t)pos * map.stride;
-        else if constexpr (BS16) return base + (size_t)map.bt[pos >> 4] * 16 * map.stride;
+        else if constexpr (BS16) return base + (size_t)map.run_of(pos) * 16 * map.stride;
         else return base;
     }
     // elements `elem` on of key 16 j + r (r < 16); j uniform
@@ -1044,14 +1054,14 @@ void launch_fp32(const PrefillArgs& a, hipStream_t s) {
 template <int D>
 void launch_d(const PrefillArgs& a, hipStream_t s) {
     const bool fp32 = prefill_form(a) == kFp32, bs16 = a.block_size == 16;
+    // BlockRows: whole 16-token runs, and 32-bit offsets inside one
+    const bool runs = a.block_size % 16 == 0 && 16ull * a.H_kv * D * sizeof(uint16_t) <= 1ull << 32;
     if (!a.paged)
         fp32 ? launch_fp32<D, 1, false>(a, s) : launch_t<D, float, 1, false>(a, s);
     else if (fp32)
         bs16 ? launch_fp32<D, 0, true>(a, s) : launch_fp32<D, 0, false>(a, s);
-    else if (bs16 && 16ull * a.H_kv * D * sizeof(uint16_t) <= 1ull << 32)  // BlockRows' 32-bit offsets
-        launch_t<D, uint16_t, 0, true>(a, s);
     else
-        launch_t<D, uint16_t, 0, false>(a, s);
+        runs ? launch_t<D, uint16_t, 0, true>(a, s) : launch_t<D, uint16_t, 0, false>(a, s);
 }
 
 }  // namespace
