@@ -1002,30 +1002,48 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void prefill_split_kernel(
 
 enum PrefillForm { kFp32, kSplit, kTile1, kTile2 };
 
-// Measured on one box (us, graph-timed; W = 64-query tiles of the launch).
-// Paged bf16: few tiles take the split kernel (d 64: 1 x 256 x 8 heads 7.35 on
-// the fp32 MFMAs, 5.75 here; 1 x 1024 x 8 23.5 -> 13.6; d 128: 41.2 -> 20.9), from
-// 320 on the tile kernel, one workgroup of waves over short contexts (d 128, 16 x
-// 128 x 12: split 20.4, GW = 1 13.9, GW = 2 21.5; fp32 MFMAs 24.7) and two over
-// longer ones until there are tiles for several workgroups per CU (d 64, 4 x 512 x
-// 12: 18.7 / 20.5 / 17.5).
-// Contiguous fp32: the tile kernels where they have the tiles (d 128: 4 x 512 x 32
-// heads 146 -> 76 on GW = 1, 1 x 2048 x 16 210 -> 126 on GW = 2, 161 on GW = 1; d
-// 64: 4 x 256 x 32 23.9 -> 19.1, 1 x 2048 x 16 97 -> 78), the split kernel for a
-// few long ones (d 128, 1 x 1024 x 4 33.2 -> 29.7), the fp32 kernel for the rest,
-// whose launches are over before the splitting pays (d 64, 2 x 512 x 12: 17.8
-// against 19.5 split, 22.3 GW = 2).
+// Measured on one box (us, graph-timed), split / GW = 1 / GW = 2 (/ fp32 MFMAs);
+// tiles: of 64 queries.
+// Paged bf16.  Few tiles take the split kernel (d 64: 1 x 512 x 8 heads 13.7 /
+// 19.7 / 16.4 / 20.3 for 256 of them), and so do up to 16 queries, of which a tile
+// would fill one wave in four (d 64, 1 query of 400 pairs after 800 tokens 20.2 /
+// 30.4 / 41.9 / 28.6).  From 320 tiles on GW = 1, whose workgroups share a CU (d
+// 64, 640 tiles of 64 queries after 1000 tokens 102.6 / 58.5 / 82.3 / 132.5), but for
+// long prompts where most tiles are short and the first ones set the time: in
+// up to 400 tiles at d = 64 the split kernel (384 tiles of 512 / 1024 queries 17.6 /
+// 20.6 / 19.1 and 23.1 / 34.9 / 27.1), in up to 512 at d = 128 GW = 2 (384 tiles of 1024
+// 45.9 / 47.2 / 39.5).
+// Contiguous fp32.  The tile kernels where they have the tiles (d 128: 4 x 512 x 32
+// heads 146 -> 76 on GW = 1; 1 x 2048 x 16 heads 210 -> 127 on GW = 2, 161 on GW = 1).
+// GW = 2 takes a CU per workgroup, so its second round must be worth it: causal
+// d 128 from 256 tiles on (288 tiles of N = 1000 88.0 / 80.1 / 61.6 / 73.0; 192: 60.9 /
+// 78.3 / 59.6 / 48.2), non-causal, twice the work, from 144 (168 of 1500 120 / 115 / 87 /
+// 119; 130 of 800 55.0 / 64.2 / 49.8 / 47.5), d 64 from 384 (408 of 1500 62.3 / 76.2 / 53.5 /
+// 63.0; 264 of 2100 55.1 / 102.4 / 72.7 / 61.5; non-causal 286 of 800 50.8 / 53.9 / 60.0 / 51.0),
+// causal N < 1500 from 300 (403 of 800 44.8 / 42.5 / 33.4 / 41.2).  Below, the split
+// kernel for a few long problems (d 128: 96 tiles of 1000 35.4 / 78.0 / 58.9 / 40.1,
+// non-causal 59.5 / 80.2 / 60.3 / 54.6; 40 of 600 22.8 / 48.2 / 38.6 / 23.7, 28 of 420 19.4 /
+// 37.5 / 31.1 / 17.9) and at d 64 for any number of long ones (188 of 3000
+// 60.4 / 142.7 / 100.3 / 69.9), the fp32 kernel for the rest, whose launches are over
+// before the splitting pays.
 PrefillForm prefill_form(const PrefillArgs& a) {
     const long long tiles = (long long)((a.P + kWaves * kQW - 1) / (kWaves * kQW)) * a.H_q * a.B;
     const int keys = a.start_pos + a.P;
     if (a.paged) {
         if (a.kv_dtype != IE_KV_BF16) return kFp32;
-        if (tiles < 320) return kSplit;
-        return tiles >= 1024 || keys <= 256 ? kTile1 : kTile2;
+        if (a.P <= kQW || tiles < 320) return kSplit;
+        if (a.d == 64 && a.P >= 200 && tiles < 400) return kSplit;
+        if (a.d == 128 && a.P >= 512 && a.start_pos <= a.P / 4 && tiles <= 512) return kTile2;
+        return kTile1;
     }
     if (tiles >= (keys <= 768 ? 512 : 1024)) return kTile1;
-    if (keys >= 768) return tiles >= 256 ? kTile2 : tiles <= 128 ? kSplit : kFp32;
-    return a.d == 128 && keys >= 384 && tiles <= 64 ? kSplit : kFp32;
+    if (keys < 768) return a.d == 128 && keys >= 576 && tiles <= 64 ? kSplit : kFp32;
+    if (a.d == 64) {
+        if (tiles >= (a.causal && keys < 1500 ? 300 : 384)) return kTile2;
+        return tiles <= 128 || keys >= 1500 ? kSplit : kFp32;
+    }
+    if (tiles >= (a.causal ? 256 : 144)) return kTile2;
+    return tiles <= (a.causal ? 128 : 64) ? kSplit : kFp32;
 }
 
 template <int D, typename KV, int LAYOUT, bool BS16>

@@ -243,3 +243,32 @@ def test_paged_bf16_rows_past_4_gib(ie, P):
     for i in range(4):
         want = attention64(q[:, i], *(x.reshape(-1, 4, d)[:P, i].float() for x in (k, v)), True)
         assert (got[:, i] - want).abs().max() <= REL * want.abs().max()
+
+
+# The launch rule's other lines for bf16 pages: at most 16 queries of many pairs (the split kernel), a long prompt from
+# the start at d = 128 (two sets of waves) and at d = 64 (the split kernel), blocks of two and three 16-token runs and
+# of none.  Each against the prompt in one-query chunks of one sequence at the same positions.
+@pytest.mark.parametrize("B,P,start,H,d,bs", [(8, 16, 100, 48, 128, 16), (8, 17, 100, 48, 64, 16), (1, 520, 0, 36, 128, 16),
+                                              (2, 520, 130, 18, 128, 32), (2, 210, 60, 45, 64, 48), (6, 70, 90, 30, 64, 32),
+                                              (6, 70, 90, 30, 128, 20)])
+def test_paged_bf16_launch_rule(ie, B, P, start, H, d, bs):
+    Q, kc, vc, table = case(P + start + H + bs, B, P, start, H, 1, d, bs, 1)
+    kd, vd = dev(kc), dev(vc)
+    whole = host(ie.prefill_attn(dev(Q), kd, vd, dev(table), start, bs, H, kv_dtype=ie.KV_BF16))
+    for b in {0, B - 1}:
+        for t in sorted({0, 1, 15, P // 2, P - 1}):
+            one = host(ie.prefill_attn(dev(Q[b:b + 1, t:t + 1]), kd, vd, dev(table[b:b + 1]), start + t, bs, H,
+                                       kv_dtype=ie.KV_BF16))
+            assert np.array_equal(one[0, 0], whole[b, t]), (b, t)
+    k, v = (from_bf16(x)[table[0]].reshape(-1, H, d)[:start + P] for x in (kc, vc))
+    for h in {0, H - 1}:
+        s = Q[0, :, h].astype(np.float64) @ k[:, h].T / d ** 0.5
+        s[np.arange(start + P)[None] > start + np.arange(P)[:, None]] = -np.inf
+        w = np.exp(s - s.max(1, keepdims=True))
+        want = w @ v[:, h] / w.sum(1, keepdims=True)
+        assert np.abs(whole[0, :, h] - want).max() <= REL * np.abs(want).max()
+
+
+def from_bf16(bits):
+    """bf16 bit patterns as 64-bit floats."""
+    return (bits.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
