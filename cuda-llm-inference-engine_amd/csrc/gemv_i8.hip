@@ -33,6 +33,7 @@
 #include "device_util.h"
 #include "epilogue.h"
 #include "gemv_common.h"
+#include "gemv_plan.h"
 #include "ie_internal.h"
 
 namespace ie {
@@ -921,7 +922,6 @@ constexpr size_t kStreamWeightBytes = 64ull << 20;
 // weights up to this size: each row block re-reads the weights, which for
 // these stay in the caches.
 constexpr size_t kRowSplitWeightBytes = 8ull << 20;
-constexpr size_t kLdsBytes = 160ull << 10;  // per workgroup on gfx950
 
 template <int MT, int EPI, int K16, int SRC = kSrcInt8, int GF = 0, int NW = 4>
 void launch_fixed(const GemmArgs& a, hipStream_t s, const GemvFusion& f = GemvFusion{}) {
@@ -1035,38 +1035,12 @@ void launch_burst(const GemmArgs& a, hipStream_t s) {
     else go(std::integral_constant<int, 4>{});
 }
 
-// Slicing of the any-K kernel: the KS (1, 2, 4 or 8 waves per item) whose
-// rounds x (steps per slice + 1) is least, the 1 for an item's reduction and
-// store; one workgroup per CU.
-struct AnyPlan {
-    int ks_log, spk;
-    long long batches;  // of a wave's stream
-    unsigned blocks;
-    size_t lds;
-};
 constexpr int kAnyRing = 4;
-AnyPlan any_plan(const GemmArgs& a) {
-    const long long items = (a.N + 3) / 4, cus = num_cus();
-    const int steps = (a.K + 255) / 256;
-    AnyPlan best{};
-    long long cost = -1;
-    for (int l = 0; l <= 3; ++l) {
-        const int slots = 8 >> l, spk = ((steps + (1 << l) - 1) / (1 << l) + 1) / 2 * 2;
-        const long long blocks = std::min((items + slots - 1) / slots, cus);
-        const long long rounds = (items + blocks * slots - 1) / (blocks * slots), c = rounds * (spk + 1);
-        if (cost < 0 || c < cost) {
-            cost = c;
-            best = {l, spk, rounds * (spk / 2), (unsigned)blocks, 2 * 8 * 64 * 4 + (size_t)a.M * ((spk << l) * 256 + 64)};
-        }
-    }
-    return best;
-}
-bool any_applies(const GemmArgs& a) { return a.K >= 16 && any_plan(a).lds <= kLdsBytes; }
+AnyPlan plan_any(const GemmArgs& a) { return a.K >= 16 ? any_plan(a.M, a.N, a.K, num_cus()) : AnyPlan{}; }
 
 template <int EPI>
 struct AnyLaunch {
-    static void run(const GemmArgs& a, hipStream_t s) {
-        const AnyPlan p = any_plan(a);
+    static void run(const GemmArgs& a, const AnyPlan& p, hipStream_t s) {
         const bool nt = (size_t)a.N * a.K >= kStreamWeightBytes;
         const unsigned cpr = (unsigned)(p.spk << p.ks_log) * 16;
         auto go = [&](auto mb) {
@@ -1165,7 +1139,10 @@ void launch_mt(const GemmArgs& a, hipStream_t s) {
     // 35.9 -> 10.3 / 13.0.
     const bool edge = a.N <= (a.K <= 640 ? 2048 : 1024) || a.N >= 8192;
     const bool short_k = MT <= 8 && (a.K <= 512 || (edge && a.K <= (a.M <= 2 ? 1280 : 640)));
-    if (!short_k && any_applies(a)) return AnyLaunch<EPI>::run(a, s);
+    if (!short_k) {
+        const AnyPlan p = plan_any(a);
+        if (p.lds) return AnyLaunch<EPI>::run(a, p, s);
+    }
     const dim3 grid((a.N + kRowsPerWG - 1) / kRowsPerWG);
     gemv_i8_kernel<MT, EPI><<<grid, 256, 0, s>>>(a.M, a.N, a.K, a.A, a.BT, a.sA, a.sB, a.bias,
                                                   a.residual, a.C);
@@ -1212,10 +1189,10 @@ int num_cus() {
 
 void launch_gemv_i8(const GemmArgs& a, hipStream_t s) {
     if (a.M == 0 || a.N == 0) return;
-    if (vec_ok(a))
-        dispatch_epilogue<GemvLaunch>(a.epi, a, s);
-    else if (any_applies(a))
-        dispatch_epilogue<AnyLaunch>(a.epi, a, s);
+    if (vec_ok(a)) return dispatch_epilogue<GemvLaunch>(a.epi, a, s);
+    const AnyPlan p = plan_any(a);
+    if (p.lds)
+        dispatch_epilogue<AnyLaunch>(a.epi, a, p, s);
     else
         dispatch_epilogue<GenericLaunch>(a.epi, a, s);
 }

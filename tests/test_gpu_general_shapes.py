@@ -210,6 +210,13 @@ def test_gelu_epilogue_range(ie, M):
     assert (np.abs(got - want) <= 2.7 * 2.0 ** -24 * np.abs(d) + 2.0 ** -149).all()
 
 
+# Decode rows whose cheapest slicing does not fit LDS although another one does (K % 16 == 0 and not).
+@pytest.mark.parametrize("M,K,N,words", [(14, 8708, 1024, 0), (16, 8704, 1027, 0), (16, 9700, 500, 1), (4, 36900, 5, 0),
+                                         (1, 131068, 9, 0)])
+def test_gemv_any_width_second_slicing(ie, orc, M, K, N, words):
+    _gemm_case(ie, orc, M, N, K, ie.EPI_I32, words, M + K + N)
+
+
 # Infinities and NaNs through the GELU of every GEMM family (decode, small-grid, LDS tiles, register-staged): from the
 # bias, and from a product whose scale overflows.  As the oracle's tanh form: +inf stays, -inf and NaN give NaN.
 @pytest.mark.parametrize("M,K", [(1, 768), (3, 256), (16, 768), (16, 4096), (40, 768), (40, 60), (600, 768), (600, 100)])
