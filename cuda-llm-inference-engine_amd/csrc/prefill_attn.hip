@@ -140,38 +140,39 @@ struct Chunk {
 
 // Where token `pos` of the current (b, kv head) lives, in elements from the
 // head's base pointer.
-//   LAYOUT 0, BS16: paged, blocks of `runs` whole runs of 16 tokens (the fp32
-//                   kernel: 1); `phys` is the chunk's run in the cache.
-//   LAYOUT 0:       paged, any block size (per-lane table lookup).
-//   LAYOUT 1:       contiguous rows.
-template <int LAYOUT, bool BS16>
+//   LAYOUT 0, PAGE 1: paged, blocks of 16 tokens; `phys` is the chunk's block.
+//   LAYOUT 0, PAGE 2: blocks of 2^run_log runs of 16 tokens; `phys` is the
+//                     chunk's run in the cache.
+//   LAYOUT 0, PAGE 0: any block size (per-lane table lookup).
+//   LAYOUT 1:         contiguous rows.
+template <int LAYOUT, int PAGE>
 struct TokenMap {
     const int* bt;
-    int block_size, runs;
+    int block_size, run_log;
     size_t stride;  // elements between consecutive token rows of one head
     __device__ __forceinline__ size_t off(int pos, int phys) const {
         if constexpr (LAYOUT == 1) {
             return (size_t)pos * stride;
-        } else if constexpr (BS16) {
+        } else if constexpr (PAGE) {
             return ((size_t)phys * 16 + (pos & 15)) * stride;
         } else {
             const int blk = pos / block_size;
             return ((size_t)bt[blk] * block_size + (pos - blk * block_size)) * stride;
         }
     }
-    // the run that holds token pos (BS16; wave-uniform)
+    // the run that holds token pos (PAGE 1 and 2; wave-uniform).  A form of its own
+    // for blocks of 16: shifts cost a long prompt 1-2% here, a branch 5% (each
+    // lookup then waits for the one before).
     __device__ __forceinline__ int run_of(int pos) const {
-        const uint32_t r = (uint32_t)pos >> 4;
-        if (runs == 1) return bt[r];
-        // (a first block, in which a short prompt lies, without the division)
-        const uint32_t blk = r < (uint32_t)runs ? 0 : r / (uint32_t)runs;
-        return bt[blk] * runs + (int)(r - blk * (uint32_t)runs);
+        const int r = pos >> 4;
+        if constexpr (PAGE == 1) return bt[r];
+        return (bt[r >> run_log] << run_log) + (r & ((1 << run_log) - 1));
     }
 };
 
-template <int D, typename KV, int LAYOUT, bool BS16>
+template <int D, typename KV, int LAYOUT, int PAGE>
 __device__ __forceinline__ void load_chunk(Chunk<D, KV>& c, int c0, int kend, int i, int g, int phys,
-                                           const TokenMap<LAYOUT, BS16>& map, const KV* kbase,
+                                           const TokenMap<LAYOUT, PAGE>& map, const KV* kbase,
                                            const KV* vbase) {
     const int kp = min(c0 + i, kend - 1);
     load_words(kbase + map.off(kp, phys) + (D / 4) * g, c.k);
@@ -223,7 +224,7 @@ __device__ __forceinline__ void consume(const Chunk<D, KV>& c, int c0, int g, co
 // 16-token chunks round-robin, merged in LDS.
 // LAYOUT 0: Q/O [B, P, H_q, D], keys = start + P cached tokens.
 // LAYOUT 1: Q/K/V/O [B, H, P, D], keys = P, start = 0.
-template <int D, typename KV, int LAYOUT, bool BS16>
+template <int D, typename KV, int LAYOUT, int PAGE>
 __global__ __launch_bounds__(256) void prefill_fp32_kernel(
     const float* __restrict__ Q, const KV* __restrict__ kcache, const KV* __restrict__ vcache,
     const int* __restrict__ block_table, int nbps, int block_size, int P, int H_q, int H_kv,
@@ -246,7 +247,7 @@ __global__ __launch_bounds__(256) void prefill_fp32_kernel(
     const int qi = min(q0 + i, P - 1);
 
     size_t qrow;
-    TokenMap<LAYOUT, BS16> map{};
+    TokenMap<LAYOUT, PAGE> map{};
     const KV* kbase;
     const KV* vbase;
     if constexpr (LAYOUT == 0) {
@@ -280,7 +281,7 @@ __global__ __launch_bounds__(256) void prefill_fp32_kernel(
 
     constexpr int STEP = 16 * kWaves;
     auto phys = [&](int cs) {
-        if constexpr (LAYOUT == 0 && BS16) return map.bt[min(cs, kend - 1) >> 4];
+        if constexpr (LAYOUT == 0 && PAGE) return map.bt[min(cs, kend - 1) >> 4];
         else return 0;
     };
     Chunk<D, KV> ca, cb;
@@ -522,9 +523,9 @@ __device__ __forceinline__ float merge_weights(float M, float m, float& a, float
 __device__ __forceinline__ float merge_value(float X, float x, float a, float b) { return fmaf(X, a, x * b); }
 
 // Where a tile's queries, keys and outputs are.
-template <int D, typename KV, int LAYOUT, bool BS16>
+template <int D, typename KV, int LAYOUT, int PAGE>
 struct Where {
-    TokenMap<LAYOUT, BS16> map{};
+    TokenMap<LAYOUT, PAGE> map{};
     const KV *kbase, *vbase;
     const float* Q;
     float* O;
@@ -536,22 +537,22 @@ struct Where {
     // keys that queries up to qi need
     __device__ __forceinline__ int limit(int qi) const { return causal ? min(start + qi + 1, nkeys) : nkeys; }
     __device__ __forceinline__ int phys(int pos, int kend) const {
-        if constexpr (LAYOUT == 0 && BS16) return map.run_of(min(pos, kend - 1));
+        if constexpr (LAYOUT == 0 && PAGE) return map.run_of(min(pos, kend - 1));
         else return 0;
     }
 };
 
-template <int D, typename KV, int LAYOUT, bool BS16>
-__device__ __forceinline__ Where<D, KV, LAYOUT, BS16> locate(const float* Q, const KV* kcache, const KV* vcache,
+template <int D, typename KV, int LAYOUT, int PAGE>
+__device__ __forceinline__ Where<D, KV, LAYOUT, PAGE> locate(const float* Q, const KV* kcache, const KV* vcache,
                                                              const int* block_table, int nbps, int block_size, int P,
                                                              int H_q, int H_kv, int start, int causal, float* O, int h,
                                                              int b) {
-    Where<D, KV, LAYOUT, BS16> w;
+    Where<D, KV, LAYOUT, PAGE> w;
     const int kvh = h / (H_q / H_kv);
     if constexpr (LAYOUT == 0) {
         w.map.bt = block_table + (size_t)b * nbps;
         w.map.block_size = block_size;
-        w.map.runs = block_size >> 4;
+        w.map.run_log = 27 - __builtin_clz(block_size);
         w.map.stride = (size_t)H_kv * D;
         w.kbase = kcache + (size_t)kvh * D;
         w.vbase = vcache + (size_t)kvh * D;
@@ -575,8 +576,8 @@ __device__ __forceinline__ Where<D, KV, LAYOUT, BS16> locate(const float* Q, con
 // 16 queries from q0 on with fp32 MFMAs, one wave over all their keys: the
 // form for operands that have no three-part one.  Writes those of `rows` (bit
 // i: query q0 + i).
-template <int D, typename KV, int LAYOUT, bool BS16>
-__device__ __forceinline__ void exact_tile(const Where<D, KV, LAYOUT, BS16>& w, int q0, float qscale,
+template <int D, typename KV, int LAYOUT, int PAGE>
+__device__ __forceinline__ void exact_tile(const Where<D, KV, LAYOUT, PAGE>& w, int q0, float qscale,
                                            uint32_t rows) {
     if (q0 >= w.P) return;
     const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
@@ -658,30 +659,30 @@ __device__ __forceinline__ bool split_query(const float (&x)[D / 32][8], float q
     return bad;
 }
 
-// Rows of a block's keys for a lane.  With pages of whole 16-token runs and
+// Rows of a block's keys for a lane.  With pages of 2^n 16-token runs and
 // contiguous rows key r of half j of a block at c0 lies at a uniform base (of
 // the run, or of the half) plus r rows, so an address is a scalar base plus a
 // 32-bit lane offset; other block sizes look each key up.  Keys at or past kend read the
 // last one.
-template <typename KV, int LAYOUT, bool BS16>
+template <typename KV, int LAYOUT, int PAGE>
 struct BlockRows {
-    const TokenMap<LAYOUT, BS16>& map;
+    const TokenMap<LAYOUT, PAGE>& map;
     const KV* base;  // the head's rows
     const KV *half0, *half1;
     int c0, kend;
-    __device__ __forceinline__ BlockRows(const TokenMap<LAYOUT, BS16>& m, const KV* b, int c0_, int kend_)
+    __device__ __forceinline__ BlockRows(const TokenMap<LAYOUT, PAGE>& m, const KV* b, int c0_, int kend_)
         : map(m), base(b), c0(c0_), kend(kend_) {
         half0 = start_of(c0);
         half1 = start_of(min(c0 + 16, (kend - 1) & ~15));  // (past the end: its keys read the first half's last)
     }
     __device__ __forceinline__ const KV* start_of(int pos) const {
         if constexpr (LAYOUT == 1) return base + (size_t)pos * map.stride;
-        else if constexpr (BS16) return base + (size_t)map.run_of(pos) * 16 * map.stride;
+        else if constexpr (PAGE) return base + (size_t)map.run_of(pos) * 16 * map.stride;
         else return base;
     }
     // elements `elem` on of key 16 j + r (r < 16); j uniform
     __device__ __forceinline__ const KV* at(int j, int r, int elem) const {
-        if constexpr (LAYOUT == 0 && !BS16) {
+        if constexpr (LAYOUT == 0 && !PAGE) {
             return base + map.off(min(c0 + 16 * j + r, kend - 1), 0) + elem;
         } else {
             const int pos = min(c0 + 16 * j, (kend - 1) & ~15);
@@ -694,8 +695,8 @@ struct BlockRows {
 
 // LAYOUT 0: Q/O [B, P, H_q, D], keys = start + P cached tokens.
 // LAYOUT 1: Q/K/V/O [B, H, P, D], keys = P, start = 0.
-template <int D, typename KV, int LAYOUT, bool BS16, int GW>
-__global__ __launch_bounds__(256 * GW, D == 64 && GW == 1 ? 3 : 2) void prefill_tile_kernel(
+template <int D, typename KV, int LAYOUT, int PAGE, int GW>
+__global__ __launch_bounds__(256 * GW, D != 64 ? 2 : sizeof(KV) == 2 ? 4 : GW == 1 ? 3 : 2) void prefill_tile_kernel(
     const float* __restrict__ Q, const KV* __restrict__ kcache, const KV* __restrict__ vcache,
     const int* __restrict__ block_table, int nbps, int block_size, int P, int H_q, int H_kv,
     int start, int causal, float qscale, float* __restrict__ O) {
@@ -718,7 +719,7 @@ __global__ __launch_bounds__(256 * GW, D == 64 && GW == 1 ? 3 : 2) void prefill_
     const int pairs = (int)(gridDim.x / (unsigned)ntiles);  // H_q B
     const int r = (int)blockIdx.x / pairs, pr = (int)blockIdx.x - r * pairs;
     const int q0 = (ntiles - 1 - r) * QT;  // longest (last) tiles first
-    const auto w = locate<D, KV, LAYOUT, BS16>(Q, kcache, vcache, block_table, nbps, block_size, P, H_q, H_kv, start,
+    const auto w = locate<D, KV, LAYOUT, PAGE>(Q, kcache, vcache, block_table, nbps, block_size, P, H_q, H_kv, start,
                                                causal, O, pr % H_q, pr / H_q);
     const int kend = w.limit(min(q0 + QT - 1, P - 1));
     const int nblk = (kend + kKB - 1) / kKB;
@@ -733,7 +734,7 @@ __global__ __launch_bounds__(256 * GW, D == 64 && GW == 1 ? 3 : 2) void prefill_
     const int vj = wave & 1, vo = 2 * (wave >> 1) + (lane >> 5), ve = (lane & 31) * VE;
     auto load = [&](int blk) {
         const int c0 = blk * kKB;
-        const BlockRows<KV, LAYOUT, BS16> kb(w.map, w.kbase, c0, kend), vb(w.map, w.vbase, c0, kend);
+        const BlockRows<KV, LAYOUT, PAGE> kb(w.map, w.kbase, c0, kend), vb(w.map, w.vbase, c0, kend);
 #pragma unroll
         for (int j = 0; j < KT; ++j) {
             const int id = tid + T * j, key = id / CK, c = id % CK;
@@ -882,7 +883,7 @@ __global__ __launch_bounds__(256 * GW, D == 64 && GW == 1 ? 3 : 2) void prefill_
     if (rows) exact_tile(w, qw, qscale, rows);
 }
 
-template <int D, typename KV, int LAYOUT, bool BS16>
+template <int D, typename KV, int LAYOUT, int PAGE>
 __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void prefill_split_kernel(
     const float* __restrict__ Q, const KV* __restrict__ kcache, const KV* __restrict__ vcache,
     const int* __restrict__ block_table, int nbps, int block_size, int P, int H_q, int H_kv,
@@ -899,7 +900,7 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void prefill_split_kernel(
     const int pairs = (int)(gridDim.x / (unsigned)ntiles);  // H_q B
     const int r = (int)blockIdx.x / pairs, pr = (int)blockIdx.x - r * pairs;
     const int q0 = (ntiles - 1 - r) * kQW;  // longest (last) tiles first
-    const auto w = locate<D, KV, LAYOUT, BS16>(Q, kcache, vcache, block_table, nbps, block_size, P, H_q, H_kv, start,
+    const auto w = locate<D, KV, LAYOUT, PAGE>(Q, kcache, vcache, block_table, nbps, block_size, P, H_q, H_kv, start,
                                                causal, O, pr % H_q, pr / H_q);
     const int kend = w.limit(min(q0 + kQW - 1, P - 1));
     const int qi = min(q0 + i, P - 1);
@@ -909,14 +910,14 @@ __global__ __launch_bounds__(256, D == 64 ? 2 : 1) void prefill_split_kernel(
     // keys of octet g.
     uint32_t kr[2][D / 32][KW], vr[8][VW];
     auto load_k = [&](int c0) {
-        const BlockRows<KV, LAYOUT, BS16> kb(w.map, w.kbase, c0, kend);
+        const BlockRows<KV, LAYOUT, PAGE> kb(w.map, w.kbase, c0, kend);
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int s = 0; s < D / 32; ++s) load_words(kb.at(j, i, 32 * s + 8 * g), kr[j][s]);
     };
     auto load_v = [&](int c0) {
-        const BlockRows<KV, LAYOUT, BS16> vb(w.map, w.vbase, c0, kend);
+        const BlockRows<KV, LAYOUT, PAGE> vb(w.map, w.vbase, c0, kend);
 #pragma unroll
         for (int e = 0; e < 8; ++e) load_words(vb.at(e >> 2, 4 * g + (e & 3), D / 16 * i), vr[e]);
     };
@@ -1007,12 +1008,14 @@ enum PrefillForm { kFp32, kSplit, kTile1, kTile2 };
 // Paged bf16.  Few tiles take the split kernel (d 64: 1 x 512 x 8 heads 13.7 /
 // 19.7 / 16.4 / 20.3 for 256 of them), and so do up to 16 queries, of which a tile
 // would fill one wave in four (d 64, 1 query of 400 pairs after 800 tokens 20.2 /
-// 30.4 / 41.9 / 28.6).  From 320 tiles on GW = 1, whose workgroups share a CU (d
-// 64, 640 tiles of 64 queries after 1000 tokens 102.6 / 58.5 / 82.3 / 132.5), but for
-// long prompts where most tiles are short and the first ones set the time: in
-// up to 400 tiles at d = 64 the split kernel (384 tiles of 512 / 1024 queries 17.6 /
-// 20.6 / 19.1 and 23.1 / 34.9 / 27.1), in up to 512 at d = 128 GW = 2 (384 tiles of 1024
-// 45.9 / 47.2 / 39.5).
+// 27 / 31 / 28.6), and at d = 64, after more than 256 tokens, all that are one round
+// of it (400 tiles of 32 queries after 800 26.7 / 33.2 / 31.4 / 46.0).  From 320 tiles
+// on GW = 2 in one round of two per CU at d = 64 (384 of 40 queries after 2400 103 /
+// 89.8 / 77.8; 528 of 200 after 300 24.5 / 25.6 / 29.3, and a little past it in long
+// prompts, whose first tiles set the time: 528 of 700 25.6 / 27.0 / 22.8), at d = 128
+// (one per CU) for those alone (384 of 1024 48.1 / 47.6 / 39.9; 384 of 64 after 300
+// 51.0 / 30.2 / 38.8); else GW = 1, whose workgroups share a CU (d 64, 1024 tiles of 512
+// 40.3 / 25.8 / 30.3).
 // Contiguous fp32.  The tile kernels where they have the tiles (d 128: 4 x 512 x 32
 // heads 146 -> 76 on GW = 1; 1 x 2048 x 16 heads 210 -> 127 on GW = 2, 161 on GW = 1).
 // GW = 2 takes a CU per workgroup, so its second round must be worth it: causal
@@ -1032,9 +1035,10 @@ PrefillForm prefill_form(const PrefillArgs& a) {
     if (a.paged) {
         if (a.kv_dtype != IE_KV_BF16) return kFp32;
         if (a.P <= kQW || tiles < 320) return kSplit;
-        if (a.d == 64 && a.P >= 200 && tiles < 400) return kSplit;
-        if (a.d == 128 && a.P >= 512 && a.start_pos <= a.P / 4 && tiles <= 512) return kTile2;
-        return kTile1;
+        if (a.d == 128) return a.P >= 512 && a.start_pos <= a.P / 3 && tiles <= 512 ? kTile2 : kTile1;
+        if (keys <= 256) return kTile1;
+        if ((long long)((a.P + kQW - 1) / kQW) * a.H_q * a.B <= 960) return kSplit;
+        return tiles <= (a.P >= 512 ? 576 : 512) ? kTile2 : kTile1;
     }
     if (tiles >= (keys <= 768 ? 512 : 1024)) return kTile1;
     if (keys < 768) return a.d == 128 && keys >= 576 && tiles <= 64 ? kSplit : kFp32;
@@ -1046,40 +1050,42 @@ PrefillForm prefill_form(const PrefillArgs& a) {
     return tiles <= (a.causal ? 128 : 64) ? kSplit : kFp32;
 }
 
-template <int D, typename KV, int LAYOUT, bool BS16>
+template <int D, typename KV, int LAYOUT, int PAGE>
 void launch_t(const PrefillArgs& a, hipStream_t s) {
     const float qscale = 1.4426950408889634f / sqrtf((float)D);
     const PrefillForm form = prefill_form(a);
     const int per = form == kTile1 || form == kTile2 ? kWaves * kQW : kQW;  // queries per workgroup
     const unsigned grid = (unsigned)((long long)((a.P + per - 1) / per) * a.H_q * a.B);
-    auto* k = prefill_split_kernel<D, KV, LAYOUT, BS16>;
-    if (form == kTile1) k = prefill_tile_kernel<D, KV, LAYOUT, BS16, 1>;
-    if (form == kTile2) k = prefill_tile_kernel<D, KV, LAYOUT, BS16, 2>;
+    auto* k = prefill_split_kernel<D, KV, LAYOUT, PAGE>;
+    if (form == kTile1) k = prefill_tile_kernel<D, KV, LAYOUT, PAGE, 1>;
+    if (form == kTile2) k = prefill_tile_kernel<D, KV, LAYOUT, PAGE, 2>;
     k<<<grid, form == kTile2 ? 512 : 256, 0, s>>>(a.Q, static_cast<const KV*>(a.k), static_cast<const KV*>(a.v),
                                                  a.block_table, a.num_blocks_per_seq, a.block_size, a.P, a.H_q, a.H_kv,
                                                  a.start_pos, a.causal ? 1 : 0, qscale, a.O);
 }
 
-template <int D, int LAYOUT, bool BS16>
+template <int D, int LAYOUT, int PAGE>
 void launch_fp32(const PrefillArgs& a, hipStream_t s) {
     const float qscale = 1.4426950408889634f / sqrtf((float)D);
     const unsigned grid = (unsigned)((long long)((a.P + kQW - 1) / kQW) * a.H_q * a.B);
-    prefill_fp32_kernel<D, float, LAYOUT, BS16><<<grid, 256, 0, s>>>(
+    prefill_fp32_kernel<D, float, LAYOUT, PAGE><<<grid, 256, 0, s>>>(
         a.Q, static_cast<const float*>(a.k), static_cast<const float*>(a.v), a.block_table, a.num_blocks_per_seq,
         a.block_size, a.P, a.H_q, a.H_kv, a.start_pos, a.causal ? 1 : 0, qscale, a.O);
 }
 
 template <int D>
 void launch_d(const PrefillArgs& a, hipStream_t s) {
-    const bool fp32 = prefill_form(a) == kFp32, bs16 = a.block_size == 16;
-    // BlockRows: whole 16-token runs, and 32-bit offsets inside one
-    const bool runs = a.block_size % 16 == 0 && 16ull * a.H_kv * D * sizeof(uint16_t) <= 1ull << 32;
-    if (!a.paged)
-        fp32 ? launch_fp32<D, 1, false>(a, s) : launch_t<D, float, 1, false>(a, s);
-    else if (fp32)
-        bs16 ? launch_fp32<D, 0, true>(a, s) : launch_fp32<D, 0, false>(a, s);
+    const bool fp32 = prefill_form(a) == kFp32;
+    if (!a.paged) return fp32 ? launch_fp32<D, 1, 0>(a, s) : launch_t<D, float, 1, 0>(a, s);
+    if (fp32) return a.block_size == 16 ? launch_fp32<D, 0, 1>(a, s) : launch_fp32<D, 0, 0>(a, s);
+    // BlockRows: runs of 16 tokens, and 32-bit offsets inside one
+    const bool narrow = 16ull * a.H_kv * D * sizeof(uint16_t) <= 1ull << 32;
+    if (a.block_size == 16 && narrow)
+        launch_t<D, uint16_t, 0, 1>(a, s);
+    else if (a.block_size > 16 && (a.block_size & (a.block_size - 1)) == 0 && narrow)
+        launch_t<D, uint16_t, 0, 2>(a, s);
     else
-        runs ? launch_t<D, uint16_t, 0, true>(a, s) : launch_t<D, uint16_t, 0, false>(a, s);
+        launch_t<D, uint16_t, 0, 0>(a, s);
 }
 
 }  // namespace
