@@ -27,6 +27,9 @@
 //     K split) the compiler can no longer tell the LDS reads from the copies
 //     in flight and drains every copy before each read, so the partial tiles
 //     reuse the ring once it is empty;
+//   * KS = 1 takes the one or two groups of K < 256 without the ring's loop,
+//     whose code a launch that short waits for (K = 128, M = 95, N = 223 4.37 ->
+//     3.20 us);
 //   * KS = 2 (K split over two waves, their int32 tiles added in LDS, exact)
 //     measured best at K = 640-3072; one, three or four waves were slower
 //     (M = 128, K = 3072: 8.8 / 6.9 / 6.9 / 7.3 us for KS = 1 / 2 / 3 / 4).
@@ -132,10 +135,10 @@ __global__ __launch_bounds__(64 * KS) void gemm_i8_stream_kernel(
             if constexpr (ROUTE) slot[v] = route.row_slot[m];
         }
     }
-    if (nk > 0) {
-#pragma unroll
-        for (int p = 0; p < LR - 1; ++p) issue(g0 + min(p, nk - 1), p);
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((LR - 2) * COPIES) : "memory");
+    // Their arrival, on every path that reaches the stores: one that leaves them
+    // in flight would make every store wait for its operand and so for the store
+    // before it.
+    auto arrived = [&] {
         if (EPI != IE_EPI_I32 && wave == 0) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
@@ -146,6 +149,20 @@ __global__ __launch_bounds__(64 * KS) void gemm_i8_stream_kernel(
             asm volatile("" ::"v"(sb));
             if constexpr (HAS_BIAS) asm volatile("" ::"v"(bv));
         }
+    };
+    if (nk == 0) {
+        arrived();
+    } else {
+        if constexpr (KS == 1) {
+            issue(g0, 0);
+            if (nk > 1) issue(g0 + 1, 1);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        } else {
+#pragma unroll
+            for (int p = 0; p < LR - 1; ++p) issue(g0 + min(p, nk - 1), p);
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((LR - 2) * COPIES) : "memory");
+        }
+        arrived();
         const int fr = lane & 31, h = lane >> 5;
         // Group u.  COPY also requests group u + LR - 1 into the slot of u - 1,
         // whose reads fed the previous step's MFMAs; LEFT is the number of
@@ -168,9 +185,13 @@ __global__ __launch_bounds__(64 * KS) void gemm_i8_stream_kernel(
         // The last LR - 1 groups copy nothing (see the tile kernel's loop).
         static_assert(LR == 4, "the steps after the loop");
         int u = 0;
-        for (; u < nk - (LR - 1); ++u) step(u, std::true_type{}, std::integral_constant<int, LR - 2>{});
-        if (u < nk - 2) step(u++, std::false_type{}, std::integral_constant<int, 1>{});
-        if (u < nk - 1) step(u++, std::false_type{}, std::integral_constant<int, 0>{});
+        if constexpr (KS == 1) {
+            if (nk > 1) step(u++, std::false_type{}, std::integral_constant<int, 0>{});
+        } else {
+            for (; u < nk - (LR - 1); ++u) step(u, std::true_type{}, std::integral_constant<int, LR - 2>{});
+            if (u < nk - 2) step(u++, std::false_type{}, std::integral_constant<int, 1>{});
+            if (u < nk - 1) step(u++, std::false_type{}, std::integral_constant<int, 0>{});
+        }
         step(u, std::false_type{}, std::integral_constant<int, 0>{});
     }
     if constexpr (KS > 1) {
