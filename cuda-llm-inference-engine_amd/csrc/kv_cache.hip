@@ -5,6 +5,7 @@
 // sequence lives in physical block block_table[pos / block_size] at slot
 // pos % block_size.  bf16 caches store round-to-nearest-even bfloat16.
 #include <algorithm>
+#include <type_traits>
 
 #include "device_util.h"
 #include "ie_internal.h"
@@ -41,15 +42,19 @@ __global__ __launch_bounds__(256) void kv_write_kernel(const float* __restrict__
 // page is looked up once per workgroup and a thread moves 16 bytes of K and of
 // V.  Against one element per thread (two integer divisions each): 512 x 768
 // 3.16 -> 2.81 us (bf16 cache 3.15 -> 2.73), 1024 x 2048 bf16 7.27 -> 4.50 us.
-template <typename KV>
+// NARROW: rows of at most 64, 256 / blockDim.x tokens to a workgroup (with one
+// each most threads idled: 10660 tokens of 64 4.82 -> 3.48 us, 7070 of 4 4.04 -> 2.37).
+template <typename KV, bool NARROW>
 __global__ __launch_bounds__(256) void kv_write_vec_kernel(const float4* __restrict__ K, const float4* __restrict__ V,
                                                            KV* __restrict__ kc, KV* __restrict__ vc,
-                                                           const int* __restrict__ bt, int start_pos, int n4, int bs) {
-    const int j = blockIdx.y * 256 + threadIdx.x;
-    if (j >= n4) return;
-    const size_t src = (size_t)blockIdx.x * n4 + j;
+                                                           const int* __restrict__ bt, int seq_len, int start_pos,
+                                                           int n4, int bs) {
+    const int j = NARROW ? threadIdx.x : blockIdx.y * 256 + threadIdx.x;
+    const unsigned t = NARROW ? blockIdx.x * blockDim.y + threadIdx.y : blockIdx.x;
+    if (j >= n4 || (NARROW && t >= (unsigned)seq_len)) return;
+    const size_t src = (size_t)t * n4 + j;
     const float4 k = K[src], v = V[src];
-    const int pos = start_pos + (int)blockIdx.x, blk = pos / bs;
+    const int pos = start_pos + (int)t, blk = pos / bs;
     const size_t dst = ((size_t)bt[blk] * bs + (pos - blk * bs)) * n4 + j;
     if constexpr (sizeof(KV) == 4) {
         reinterpret_cast<float4*>(kc)[dst] = k;
@@ -90,15 +95,24 @@ void launch_kv_write(const float* K, const float* V, void* kc, void* vc, int kv_
     if (row % 4 == 0 && row / 4 <= 256LL * 65535 && (((uintptr_t)K | (uintptr_t)V) % 16) == 0 &&
         (((uintptr_t)kc | (uintptr_t)vc) % esz) == 0) {
         const int n4 = (int)(row / 4);
-        const dim3 grid((unsigned)seq_len, (unsigned)((n4 + 255) / 256));
-        const unsigned threads = (unsigned)std::min(256, (n4 + 63) / 64 * 64);
         const float4 *k4 = reinterpret_cast<const float4*>(K), *v4 = reinterpret_cast<const float4*>(V);
+        const bool narrow = n4 <= 64;
+        dim3 threads((unsigned)std::min(256, (n4 + 63) / 64 * 64)), grid((unsigned)seq_len, (unsigned)((n4 + 255) / 256));
+        if (narrow) {
+            unsigned tx = 1;
+            while ((int)tx < n4) tx *= 2;
+            threads = dim3(tx, 256 / tx);
+            grid = dim3((unsigned)(((long long)seq_len + threads.y - 1) / threads.y));
+        }
+        auto go = [&](auto* kcache, auto* vcache) {
+            using KV = std::remove_reference_t<decltype(*kcache)>;
+            auto* k = narrow ? kv_write_vec_kernel<KV, true> : kv_write_vec_kernel<KV, false>;
+            k<<<grid, threads, 0, s>>>(k4, v4, kcache, vcache, bt, seq_len, start_pos, n4, bs);
+        };
         if (kv_dtype == IE_KV_BF16)
-            kv_write_vec_kernel<uint16_t><<<grid, threads, 0, s>>>(k4, v4, static_cast<uint16_t*>(kc),
-                                                                   static_cast<uint16_t*>(vc), bt, start_pos, n4, bs);
+            go(static_cast<uint16_t*>(kc), static_cast<uint16_t*>(vc));
         else
-            kv_write_vec_kernel<float><<<grid, threads, 0, s>>>(k4, v4, static_cast<float*>(kc), static_cast<float*>(vc),
-                                                                bt, start_pos, n4, bs);
+            go(static_cast<float*>(kc), static_cast<float*>(vc));
         return;
     }
     const unsigned blocks = (unsigned)((total + 255) / 256);
