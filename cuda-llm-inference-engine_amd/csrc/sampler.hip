@@ -17,7 +17,10 @@
 //      it; one barrier.  For larger k the least of the waves' bounds lets ever
 //      more keys through (8 rows at k = 400 83.8 against 24.2 us): M is the
 //      k-th largest of the 1024 maxima (a radix select over one key per
-//      thread, sixteen barriers);
+//      thread, sixteen barriers).  Rows of fewer than 260 logits, and k past
+//      the number of maxima, have no bound: every key is a candidate (8 rows of
+//      6 at k = 3 13.0 -> 9.9 us), or the row is streamed at once if it has
+//      more than are ranked (1 of 3063 at k = 1024 39.6 -> 32.5);
 //   2. the keys >= M (typically k to a few times k) gathered into LDS;
 //   3. each gathered key ranked by counting those before it (larger key, or
 //      equal key and lower index), several threads per key while there are
@@ -288,8 +291,20 @@ __global__ __launch_bounds__(kTopkThreads) void topk_reg_kernel(const float* __r
     const uint32_t tmax = order_key(fmx);
     // Full waves: every lane holds at least one whole chunk of the row.
     const int full = min(kTopkWaves, (n - 4) / 256);
+    const int held = (n + s + 3) / 4;  // threads that hold any of it, if below 1024
+    if (k > held && n > kTopkCand) {   // uniform: no bound below the whole row, which is too much
+        topk_stream_row(sh, x, n, k, out_vals, out_idx, lane, wid);
+        return;
+    }
     uint32_t M;
-    if (full > 0 && k <= 4 * full) {  // uniform
+    if (k > held || full == 0) {  // uniform: every key is a candidate
+        if (lane == 0) sh.wave_tot[wid] = nan ? 0u : order_key(-INFINITY);
+        if (threadIdx.x == 0) sh.gt = 0;
+        __syncthreads();
+        M = sh.wave_tot[0];
+#pragma unroll
+        for (int w = 1; w < kTopkWaves; ++w) M = min(M, sh.wave_tot[w]);
+    } else if (k <= 4 * full) {  // uniform
         const int r = (k + full - 1) / full;
         uint32_t m = 0;
 #pragma unroll
