@@ -179,8 +179,9 @@ void launch_gemm_i8_mfma(const GemmArgs& a, hipStream_t s) {
     if (a.M == 0 || a.N == 0) return;
     const bool vec = (a.K % 16) == 0 && ((uintptr_t)a.A % 16) == 0 && ((uintptr_t)a.BT % 16) == 0;
     if (!vec || a.K < 128) {
-        // K < 16, or more 64-row tiles than a grid has in y: one thread per output
-        if (a.K >= 16 && (a.M + BM - 1) / BM <= 65535)
+        // K < 16, a few short rows, or more 64-row tiles than a grid has in y: one
+        // thread per output
+        if (a.K >= 16 && (vec || !short_ragged_rows(a)) && (a.M + BM - 1) / BM <= 65535)
             dispatch_epilogue<RaggedLaunch>(a.epi, a, s);
         else
             launch_gemm_i8_generic(a, s);

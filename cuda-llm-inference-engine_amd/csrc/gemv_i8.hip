@@ -1076,6 +1076,25 @@ void launch_fused(const GemmArgs& a, const GemvFusion& f, hipStream_t s) {
     else launch_mfma16<EPI, K / 64, SRC>(a, s, f);
 }
 
+// Rows short enough for the dot4 kernel, which starts 0.3-0.4 us sooner than the
+// any-K kernel (no plan, no reduction): K <= 512 (256 x 4096, M = 1 / 8 2.17 / 2.42
+// against 2.59 / 3.04 us), past 8 rows K <= 256 (11 rows of 256 x 218 3.11 against
+// 3.57; 9 of 320 x 298 3.88 against 3.52); longer for a few workgroups (1024 x 1024,
+// M = 1 2.40 against 2.65; 736 x 1753 2.70 / 2.99, 912 x 2445 3.79 / 3.08; 544 x 2644, M = 2
+// 2.74 / 2.95, 592 x 5560 3.48 / 3.23) and for very many, whose any-K rounds end with
+// one that is partly empty (736 x 8579, M = 7 4.92 / 5.64, 992 x 11539, M = 5 5.80 / 6.34,
+// 848 x 14085, M = 5 6.22 / 5.80; 1408 x 18404, M = 1 6.50 / 7.00, 1456 x 27712 9.48 / 8.93).
+bool dot4_ahead(const GemmArgs& a) {
+    if (a.M > 8) return a.K <= 256;
+    if (a.K <= 512) return true;
+    if (a.N <= 1024) return a.K <= (a.M <= 2 ? 1280 : 640);
+    if (a.N <= 2048) return a.K <= (a.M == 1 ? 864 : 640);
+    if (a.N <= 3200) return a.M <= 2 && a.K <= 640;
+    if (a.N < 8192) return false;
+    if (a.M <= 2) return a.K <= (a.N < 20000 ? 1600 : 1280);
+    return a.K <= (a.N < 12500 ? 1040 : 640);
+}
+
 template <int MT, int EPI>
 void launch_mt(const GemmArgs& a, hipStream_t s) {
     // Wide GPT-2-width GEMVs (the 768 x 50257 LM head): all of a wave's
@@ -1130,15 +1149,10 @@ void launch_mt(const GemmArgs& a, hipStream_t s) {
     }
     if constexpr (MT == 1)
         if (a.K == 3072 && a.N < 2048) return launch_fixed<MT, EPI, 192, kSrcInt8, 1, 1>(a, s);
-    // Any other K.  The dot4 kernel below starts 0.3-0.4 us sooner (no plan,
-    // no reduction) and keeps short rows: K <= 512 (256 x 4096, M = 1 / 8:
-    // 2.17 / 2.42 against 2.59 / 3.04 us) and, for a few workgroups or very
-    // many, K <= 640 (M <= 2: K <= 1280; 1024 x 1024, M = 1: 2.40 against
-    // 2.65).  Otherwise the any-K kernel: 1024 x 3000, M = 1 / 16 3.40 / 6.42 ->
-    // 3.11 / 4.03 us, 4096 x 4096 9.45 / 21.7 -> 5.0 / 6.4, 6144 x 8192 17.3 /
-    // 35.9 -> 10.3 / 13.0.
-    const bool edge = a.N <= (a.K <= 640 ? 2048 : 1024) || a.N >= 8192;
-    const bool short_k = MT <= 8 && (a.K <= 512 || (edge && a.K <= (a.M <= 2 ? 1280 : 640)));
+    // Any other K: the any-K kernel (1024 x 3000, M = 1 / 16 3.40 / 6.42 -> 3.11 / 4.03
+    // us, 4096 x 4096 9.45 / 21.7 -> 5.0 / 6.4, 6144 x 8192 17.3 / 35.9 -> 10.3 / 13.0) but
+    // for short rows (dot4_ahead).
+    const bool short_k = dot4_ahead(a);
     if (!short_k) {
         const AnyPlan p = plan_any(a);
         if (p.lds) return AnyLaunch<EPI>::run(a, p, s);
@@ -1187,10 +1201,27 @@ int num_cus() {
     return n;
 }
 
+// Rows that the kernels above cannot take (K % 16 != 0, or 4-byte alignment) and
+// that are so short that one thread per output, which starts at once, is ahead
+// of staging them: up to 28 bytes for a decode batch (M = 13, K = 20, N = 182
+// 2.59 against 3.70 us), a little longer by rows, features and products.  More
+// than 4 rows: K = 40, N = 28 2.61 / 2.71; more than 8: K = 48, N = 1366 3.05 / 3.67,
+// K = 56, N = 20300 7.51 / 5.73; one row of many features: K = 52, N = 42402 3.56 /
+// 5.33, K = 60, N = 14 2.95 / 2.46.  Prompt rows: K = 24, 763 x 289 3.46 / 3.82, 798 x
+// 464 4.04 / 3.78; K = 40, 756 x 55 2.91 / 3.52, 110 x 1880 4.44 / 3.65.
+bool short_ragged_rows(const GemmArgs& a) {
+    const double products = (double)a.M * a.N * a.K;
+    if (a.K > 60) return false;
+    if (a.M > kGemvMaxM) return products <= (a.K <= 28 ? 7e6 : a.K <= 44 ? 5e6 : 4e6);
+    if (a.K <= 28) return true;
+    if (a.M > 8) return products <= (a.K <= 44 ? 9e6 : 4.5e6);
+    return a.M > 4 ? a.K <= 40 : a.N >= 10000 && products <= 3e6;
+}
+
 void launch_gemv_i8(const GemmArgs& a, hipStream_t s) {
     if (a.M == 0 || a.N == 0) return;
     if (vec_ok(a)) return dispatch_epilogue<GemvLaunch>(a.epi, a, s);
-    const AnyPlan p = plan_any(a);
+    const AnyPlan p = short_ragged_rows(a) ? AnyPlan{} : plan_any(a);
     if (p.lds)
         dispatch_epilogue<AnyLaunch>(a.epi, a, p, s);
     else

@@ -123,6 +123,7 @@ bool gemm_i8_stream_applies(const GemmArgs& a);
 void launch_gemm_i8_stream(const GemmArgs& a, hipStream_t s);
 // One thread per output; any K % 4 == 0 and any alignment (gemv_i8.hip).
 void launch_gemm_i8_generic(const GemmArgs& a, hipStream_t s);
+bool short_ragged_rows(const GemmArgs& a);  // unaligned rows that it is ahead at
 constexpr int kGemvMaxM = 16;
 
 // ---- decode attention (decode_attn.hip) ----

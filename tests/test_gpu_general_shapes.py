@@ -135,6 +135,15 @@ def test_kv_write_rows(ie, seq, start, H, dh, bs, skew, bf16):
         assert np.array_equal(c.cpu().numpy(), want)
 
 
+# Rows of at most 64 float4s share a workgroup: a power of two of them, one short of and past one, tokens that fill a
+# workgroup and a last one that is partial.
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("seq,start,H,dh,bs", [(255, 3, 1, 4, 16), (257, 0, 1, 12, 16), (70, 15, 1, 64, 8), (33, 1, 2, 66, 16),
+                                               (5, 2, 2, 128, 16), (9, 2, 1, 260, 16), (129, 7, 2, 20, 5)])
+def test_kv_write_narrow_rows(ie, seq, start, H, dh, bs, bf16):
+    test_kv_write_rows(ie, seq, start, H, dh, bs, 0, bf16)
+
+
 def _key_order(row):
     """Indices by the float's order key (a NaN past the infinity of its sign), descending, lower index first."""
     b = row.view(np.uint32).copy()
@@ -165,6 +174,13 @@ def test_topk_bounds(ie, n, k):
         want = _key_order(x[b])[:k]
         assert np.array_equal(i[b], want), b
         assert np.array_equal(v[b], x[b][want], equal_nan=True), b
+
+
+# Rows without a bound: fewer than 260 logits, k past the threads that hold any (2048 logits are ranked, more streamed).
+@pytest.mark.parametrize("n,k", [(1, 1), (3, 3), (6, 2), (255, 64), (259, 1), (259, 259), (260, 65), (261, 66), (1000, 251),
+                                 (2047, 1000), (2048, 512), (2048, 513), (2049, 513), (2050, 514), (3063, 1024), (4090, 1024)])
+def test_topk_without_a_bound(ie, n, k):
+    test_topk_bounds(ie, n, k)
 
 
 # The language-model head at widths that are no multiple of 256 (or past 1280).  d: one float4, a partial chunk of 64, a
@@ -215,6 +231,21 @@ def test_gelu_epilogue_range(ie, M):
                                          (1, 131068, 9, 0)])
 def test_gemv_any_width_second_slicing(ie, orc, M, K, N, words):
     _gemm_case(ie, orc, M, N, K, ie.EPI_I32, words, M + K + N)
+
+
+# The lines between the kernels of short rows.  Unaligned rows of 16 to 64 bytes: one thread per output or staged, by rows
+# and products (decode and prompt rows); aligned decode rows: K and N on both sides of the dot4 kernel's.  K = 128 and 240
+# on a small grid: one and two groups without the ring's loop.
+@pytest.mark.parametrize("M,K,N,words", [(1, 28, 37, 0), (1, 32, 37, 1), (1, 60, 10001, 0), (7, 40, 33, 0), (7, 44, 33, 0),
+                                         (12, 44, 15000, 0), (12, 44, 17500, 0), (16, 60, 4700, 0), (16, 64, 77, 3),
+                                         (17, 16, 4000, 1), (300, 20, 1100, 0), (300, 28, 900, 0), (100, 44, 1100, 0),
+                                         (100, 44, 1200, 0), (60, 60, 1000, 0), (60, 60, 1200, 0), (9, 256, 70, 0),
+                                         (9, 272, 70, 0), (16, 16, 5, 0), (1, 864, 2048, 0), (1, 880, 2047, 0),
+                                         (2, 640, 3200, 0), (4, 1040, 12499, 0), (8, 1056, 8192, 0), (2, 1600, 9001, 0),
+                                         (33, 128, 65, 0), (200, 240, 70, 0), (17, 144, 33, 0)])
+def test_gemm_short_rows(ie, orc, M, K, N, words):
+    _gemm_case(ie, orc, M, N, K, ie.EPI_I32, words, M + K + N)
+    _gemm_case(ie, orc, M, N, K, ie.EPI_BIAS_GELU if K % 32 else 3, words, M + K + N)
 
 
 # Infinities and NaNs through the GELU of every GEMM family (decode, small-grid, LDS tiles, register-staged): from the
