@@ -391,8 +391,7 @@ __device__ __forceinline__ Parts<3> split8(const float (&x)[8], float s = 1.0f) 
     return r;
 }
 
-// Elements `odd` (0 or 1) of two words, as one word (one v_perm; of the mask and
-// shift form the compiler read a register it had overwritten).
+// Elements `odd` (0 or 1) of two words, as one word (one v_perm).
 __device__ __forceinline__ uint32_t pair_bf16(uint32_t lo, uint32_t hi, int odd) {
     return __builtin_amdgcn_perm(hi, lo, odd ? 0x07060302u : 0x05040100u);
 }

@@ -246,10 +246,10 @@ def test_paged_bf16_rows_past_4_gib(ie, P):
 
 
 # The launch rule's other lines for bf16 pages: at most 16 queries of many pairs (the split kernel), a long prompt from
-# the start at d = 128 (two sets of waves) and at d = 64 (the split kernel), blocks of two and three 16-token runs and
-# of none.  Each against the prompt in one-query chunks of one sequence at the same positions.
+# the start at d = 128 (two sets of waves), one round of the split kernel and of two sets of waves at d = 64, blocks of
+# two and three 16-token runs and of none.  Each against the prompt in one-query chunks of one sequence at the same positions.
 @pytest.mark.parametrize("B,P,start,H,d,bs", [(8, 16, 100, 48, 128, 16), (8, 17, 100, 48, 64, 16), (1, 520, 0, 36, 128, 16),
-                                              (2, 520, 130, 18, 128, 32), (2, 210, 60, 45, 64, 48), (6, 70, 90, 30, 64, 32),
+                                              (2, 520, 130, 18, 128, 32), (6, 32, 300, 56, 64, 16), (2, 210, 60, 45, 64, 48), (6, 70, 90, 30, 64, 32),
                                               (6, 70, 90, 30, 128, 20)])
 def test_paged_bf16_launch_rule(ie, B, P, start, H, d, bs):
     Q, kc, vc, table = case(P + start + H + bs, B, P, start, H, 1, d, bs, 1)
