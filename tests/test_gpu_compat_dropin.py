@@ -12,8 +12,8 @@ _bias_gelu / _bias_residual, run_layernorm, run_layernorm_residual (on
 tests/test_layernorm.cu's own cases), run_embedding,
 run_flash_attn_v2, sample_argmax and sample_top_k.  Here each output is
 checked against the oracle on the program's own inputs: quantizer, int32-exact
-GEMMs and embedding bit-exact, GELU 2e-6 relative plus the tanhf bound
-stated in the test, attention 1e-5 absolute (the reference's bar), LayerNorm
+GEMMs and embedding bit-exact, GELU 2e-6 relative plus the oracle's
+tanhf bound stated in the test, attention 1e-5 absolute (the reference's bar), LayerNorm
 1e-5 of scale, sampled ids equal.
 """
 import os
@@ -76,9 +76,9 @@ def test_int8_gemm_reference_cases(orc, run_dir):
         assert np.abs(C - ref).max() < 0.012 * np.sqrt(K), cs
         v = load(d, cs, "C_bias", np.float32, (M, N))
         assert np.array_equal(v, orc.gemm(Ap, Bp, sA, sB, 1, bias))
-        # GELU: the device's and glibc's tanhf may differ by an ulp or two,
-        # and 0.5 v (1 + tanh u) carries that absolute error (<= 1.2e-7 at
-        # |tanh| near 1) times |v| / 2 into the output, whose relative error
+        # GELU: the device computes v / (1 + exp(-2u)); the oracle's
+        # 0.5 v (1 + tanhf(u)) carries tanhf's absolute error (<= 1.2e-7 at
+        # |tanh| near 1) times |v| / 2 into its output, whose relative error
         # grows where 1 + tanh cancels (v well below 0).  Bar: 2e-6 relative
         # plus 1.2e-7 |v|, with v the (bit-exact) BiasOnly output.
         gelu = load(d, cs, "C_gelu", np.float32, (M, N))

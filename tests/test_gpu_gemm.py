@@ -2,8 +2,9 @@
 
 Bar: quantizer bit-exact; int32 accumulators bit-exact; Plain / BiasOnly /
 BiasResidual bit-exact (both sides evaluate the same roundings, fused
-multiply-adds written explicitly); BiasGELU within 2e-6 relative (the device
-and host tanhf differ in the last bits).  The reference's own acceptance bound
+multiply-adds written explicitly); BiasGELU within 2e-6 relative plus 1e-7 or
+1.2e-7 |v| (the oracle's 1 + tanhf cancels below 0; the device's quotient does
+not).  The reference's own acceptance bound
 (max |INT8 - FP32 GEMM| < 0.012*sqrt(K), tests/test_int8_gemm.cu:17) is checked
 on its own srand(42) inputs.  At 8192^3, where the oracle is too slow, sampled
 rows are compared exactly and the whole matrix through a column checksum.
@@ -539,8 +540,8 @@ def test_wide_kernel_shapes(ie, orc, epi, M, N):
     got = host(ie.int8_gemm(dev(Ap), dev(Wp), dev(sA), dev(sW), epi, dev(bias) if epi else None, out, out=out))
     want = orc.gemm(Ap[rows], Wp, sA[rows], sW, epi, bias if epi else None, res[rows] if epi == 3 else None)
     if epi == 2:
-        # device vs glibc tanhf: 2e-6 relative plus 1.2e-7 |v| (v = the
-        # BiasOnly value), the bound of the drop-in test's GELU check
+        # 2e-6 relative plus 1.2e-7 |v| (v = the BiasOnly value) for the
+        # oracle's cancelling 1 + tanhf: the drop-in test's GELU bound
         v = orc.gemm(Ap[rows], Wp, sA[rows], sW, 1, bias)
         err = np.abs(got[rows].astype(np.float64) - want)
         assert (err <= 2e-6 * np.abs(want) + 1.2e-7 * np.abs(v)).all(), err.max()

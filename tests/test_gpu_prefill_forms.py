@@ -13,8 +13,8 @@ pytestmark = pytest.mark.gpu
 
 
 # Paged bf16.  Fewer than 320 tiles of 64 queries: the split kernel (one key, one to five 32-key blocks, a context that
-# ends in a block's second page, other block sizes); 320 and more: the tile kernel, one set of waves up to 256 keys
-# and from 1024 tiles on, two between (a partial last tile, groups of unequal length).
+# ends in a block's second page, other block sizes); 320 and more: the tile kernel, one set of waves up to 256 keys, from
+# 1024 tiles on and at d = 128, two at d = 64 between (a partial last tile, groups of unequal length).
 @pytest.mark.parametrize("B,P,start,H_kv,G,d,bs", [
     (1, 1, 0, 1, 1, 64, 16), (2, 33, 0, 2, 1, 64, 16), (1, 17, 126, 2, 4, 128, 16), (2, 50, 300, 2, 2, 64, 16),
     (1, 40, 57, 2, 1, 128, 8), (1, 70, 13, 2, 2, 64, 48),
@@ -42,8 +42,8 @@ def test_paged_bf16_bits_do_not_depend_on_the_form(ie, d, P, B):
         assert np.array_equal(part[0], whole[1, t0:t1])
 
 
-# Contiguous fp32: few long problems on the split kernel, the tile kernel with two sets of waves (256 tiles of 768 keys
-# and more) and with one (512 tiles, 1024 of long ones).
+# Contiguous fp32: few long problems on the split kernel (385 keys: the fp32 one), the tile kernel with two sets of waves
+# (312 causal tiles at d = 64, 260 at d = 128, of 768 keys and more) and with one (512 tiles, 1024 of long ones).
 @pytest.mark.parametrize("B,H,N,d,causal", [(1, 2, 769, 64, True), (1, 2, 801, 128, False), (1, 4, 385, 128, True),
                                             (1, 24, 780, 64, True), (2, 10, 800, 128, False), (2, 64, 250, 64, True),
                                             (4, 32, 200, 128, False), (8, 32, 97, 64, False), (2, 40, 801, 64, True)])
@@ -267,6 +267,25 @@ def test_paged_bf16_launch_rule(ie, B, P, start, H, d, bs):
         w = np.exp(s - s.max(1, keepdims=True))
         want = w @ v[:, h] / w.sum(1, keepdims=True)
         assert np.abs(whole[0, :, h] - want).max() <= REL * np.abs(want).max()
+
+
+# The launch rule's lines for contiguous problems, a shape on each side: 64 tiles of 576 keys (d = 128), 128 / 64 and
+# 256 / 144 tiles of 768 (d = 128, causal or not), 128 / 300 / 384 and any number of 1500 keys (d = 64).
+@pytest.mark.parametrize("H,N,d,causal", [(6, 576, 128, True), (7, 600, 128, True), (6, 575, 128, False),
+                                          (9, 800, 128, True), (10, 800, 128, True), (20, 800, 128, True),
+                                          (4, 1000, 128, False), (5, 1000, 128, False), (11, 800, 128, False),
+                                          (12, 800, 128, False), (9, 800, 64, True), (10, 800, 64, True),
+                                          (23, 800, 64, True), (24, 800, 64, False), (12, 1500, 64, True),
+                                          (16, 1500, 64, True), (16, 1500, 64, False)])
+def test_flash_launch_rule(ie, H, N, d, causal):
+    import torch
+
+    g = torch.Generator().manual_seed(H + N + d)
+    Q, K, V = (torch.randn(1, H, N, d, generator=g) for _ in range(3))
+    got = ie.flash_attn(Q.cuda(), K.cuda(), V.cuda(), causal=causal).cpu().double()
+    for h in {0, H - 1}:
+        want = attention64(Q[0, h], K[0, h], V[0, h], causal)
+        assert ((got[0, h] - want).abs() <= REL * want.abs().max()).all()
 
 
 def from_bf16(bits):
