@@ -49,11 +49,12 @@
 // own arithmetic gives; the tile's others keep their bits.
 //
 // Which family: a paged launch by the cache type alone (bf16: the three-part
-// kernels), so the bits of a finite result never depend on the batch or on how
-// a prompt is chunked; a contiguous one by its shape (prefill_form).  (An infinite or
-// NaN value of V at a key that a query does not see can still reach it, 0 times it
-// being a NaN: in the fp32 MFMAs from the keys of its own 16 queries.  Such a
-// query is computed again, or is itself a NaN, as its tile lies.)
+// kernels), so over finite operands a query's bits never depend on the batch or on
+// how a prompt is chunked; a contiguous one by its shape (prefill_form).  (An
+// infinite or NaN value of V at a key that a query does not see can still reach it,
+// 0 times it being a NaN: from a later key of its block, and in the fp32 MFMAs from
+// the keys of its own 16 queries.  Such a query is computed again, or is itself a
+// NaN, as its tile lies.)
 //
 // In the three-part kernels a wave owns 16 queries of one (b, h).  Operands
 // (lane l: i = l % 16, g = l / 16): S^T = K Q^T, 16 keys x 16 queries per MFMA, leaves lane l with query i and
@@ -376,7 +377,7 @@ constexpr int kParts = sizeof(KV) == 4 ? 3 : 1;
 // The weights and the fp32 values of V are split times 2^24 (exact), so that no
 // part of a normal weight or of any value is below bf16's range; the output
 // is divided by both.  (Unscaled, values below 1e-34 lost their third part and
-// those below 1e-36 more than 1e-5 of themselves; 1 x 16 x 2048 x 128 125.6 -> 128.7 us
+// those below 1e-36 more than 1e-5 of themselves; 1 x 16 x 2048 x 128 125.8 -> 126.8 us
 // for the multiplications, ordinary operands' bits unchanged.)
 constexpr float kUp = 0x1p24f;
 template <typename KV>

@@ -151,7 +151,11 @@ int ie_decode_attn_noalloc(int B, int H_q, int H_kv, int d, const float* Q,
  * cached positions 0 .. start_pos + t.  Q and O are token-major
  * [B, P, H_q, d] fp32 (the QKV projection's layout); caches, block table and
  * kv_dtype as ie_decode_attn, with start_pos + P <= num_blocks_per_seq *
- * block_size.  d in {64,128}; H_q a multiple of H_kv. */
+ * block_size.  d in {64,128}; H_q a multiple of H_kv.  The kernels follow from
+ * the cache type alone, so with a finite cache a query's bits depend neither on
+ * B nor on how the prompt is cut into chunks.  (An infinite or NaN value within
+ * the 31 keys after a query may change its last bits or make them a NaN: which
+ * queries, the cut decides.) */
 int ie_prefill_attn(int B, int P, int H_q, int H_kv, int d, const float* Q,
                     const void* k_cache, const void* v_cache, int kv_dtype,
                     const int* block_table, int num_blocks_per_seq,
@@ -161,7 +165,10 @@ int ie_prefill_attn(int B, int P, int H_q, int H_kv, int d, const float* Q,
 /* FlashAttention forward over contiguous fp32 Q, K, V, O [B, H, N, d]
  * (run_flash_attn_v2, kernels/flash_attention/10_flash_attn_v2.cuh:7-9):
  * softmax(Q K^T / sqrt(d)) V per (b, h), keys j <= i when causal.  d in
- * {64,128}; O must not overlap Q, K or V. */
+ * {64,128}; O must not overlap Q, K or V.  The kernel is chosen by B, H, N and
+ * causal, so the last bits of a (b, h) may differ between launches of different
+ * shapes (all within the same error of the exact result); a repeated launch
+ * repeats its bits. */
 int ie_flash_attn(int B, int H, int N, int d, const float* Q, const float* K,
                   const float* V, float* O, int causal, ie_stream_t stream);
 
