@@ -1083,7 +1083,10 @@ void launch_fused(const GemmArgs& a, const GemvFusion& f, hipStream_t s) {
 // M = 1 2.40 against 2.65; 736 x 1753 2.70 / 2.99, 912 x 2445 3.79 / 3.08; 544 x 2644, M = 2
 // 2.74 / 2.95, 592 x 5560 3.48 / 3.23) and for very many, whose any-K rounds end with
 // one that is partly empty (736 x 8579, M = 7 4.92 / 5.64, 992 x 11539, M = 5 5.80 / 6.34,
-// 848 x 14085, M = 5 6.22 / 5.80; 1408 x 18404, M = 1 6.50 / 7.00, 1456 x 27712 9.48 / 8.93).
+// 848 x 14085, M = 5 6.22 / 5.80; past two rounds, 16384, by up to half a
+// one, 720 x 16400, M = 4 4.89 / 5.18, 720 x 20100 5.34 / 5.61, but 784 x 19900 5.77 /
+// 5.71, 720 x 22000, M = 8 6.74 / 6.59; 1408 x 18404, M = 1 6.50 / 7.00, 1456 x 27712
+// 9.48 / 8.93).
 bool dot4_ahead(const GemmArgs& a) {
     if (a.M > 8) return a.K <= 256;
     if (a.K <= 512) return true;
@@ -1092,6 +1095,7 @@ bool dot4_ahead(const GemmArgs& a) {
     if (a.N <= 3200) return a.M <= 2 && a.K <= 640;
     if (a.N < 8192) return false;
     if (a.M <= 2) return a.K <= (a.N < 20000 ? 1600 : 1280);
+    if (a.N > 16384 && a.N <= 20480) return a.K < 768;
     return a.K <= (a.N < 12500 ? 1040 : 640);
 }
 

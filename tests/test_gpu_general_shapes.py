@@ -242,6 +242,7 @@ def test_gemv_any_width_second_slicing(ie, orc, M, K, N, words):
                                          (100, 44, 1200, 0), (60, 60, 1000, 0), (60, 60, 1200, 0), (9, 256, 70, 0),
                                          (9, 272, 70, 0), (16, 16, 5, 0), (1, 864, 2048, 0), (1, 880, 2047, 0),
                                          (2, 640, 3200, 0), (4, 1040, 12499, 0), (8, 1056, 8192, 0), (2, 1600, 9001, 0),
+                                         (3, 752, 16385, 0), (8, 752, 16384, 0), (5, 656, 20481, 0),
                                          (33, 128, 65, 0), (200, 240, 70, 0), (17, 144, 33, 0)])
 def test_gemm_short_rows(ie, orc, M, K, N, words):
     _gemm_case(ie, orc, M, N, K, ie.EPI_I32, words, M + K + N)
